@@ -1845,22 +1845,26 @@ __global__ void k_fill_u64(unsigned long long *p, size_t n, unsigned long long v
         p[i] = v;
 }
 
-// Interpolation<Contact<Real>>::interact (interpolation_dynamics.hpp:46-60)
+// Interpolation<Contact<Real>>::interact (interpolation_dynamics.hpp:46-60).
+// One wave per observer, its neighbours over the lanes: a program has a few
+// probes, so the time is the latency of one observer's list.  One thread walking
+// an observer's 80 neighbours took 44 us for the two probes of a 90k-particle 3D
+// tank; with a wave, five advection steps and their probes take 6.33 ms instead
+// of 6.55.
 template <int D, class T>
-__global__ void k_interpolate(const Rec4<T> *obs, uint32_t n_obs, const Rec4<T> *tar, const T *data,
-                              uint32_t stride, const uint32_t *chunk, const uint32_t *count, const uint32_t *slice,
-                              const KernelPoly<T> *poly, T *out)
+__global__ void __launch_bounds__(64) k_interpolate(const Rec4<T> *obs, const Rec4<T> *tar, const T *data,
+                                                    uint32_t stride, const uint32_t *chunk, const uint32_t *count,
+                                                    const uint32_t *slice, const KernelPoly<T> *poly, T *out)
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_obs)
-        return;
+    const uint32_t i = blockIdx.x;
     const PV<T, D> pi = load_pv<T, D>(obs, i);
     T q = 0, w = 0;
     const uint32_t nb = chunk[i >> 6] + (i & 63u), nc = count[i];
-    for (uint32_t k = 0; k < nc; ++k)
+    for (uint32_t k = threadIdx.x; k < nc; k += 64u)
     {
         const uint32_t j = slice[nb + (k << 6)];
         const PV<T, D> pj = load_pv<T, D>(tar, j);
+        const T value = data[(size_t)j * stride];
         const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
         const T r2 = D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy;
         const T x = sqrt(r2) * poly->x_per_r;
@@ -1869,10 +1873,13 @@ __global__ void k_interpolate(const Rec4<T> *obs, uint32_t n_obs, const Rec4<T> 
         const T *c = poly->w[loc];
         const T W = ((c[3] * f + c[2]) * f + c[1]) * f + c[0];
         const T weight = W * pj.vol;
-        q += weight * data[(size_t)j * stride];
+        q += weight * value;
         w += weight;
     }
-    out[i] = q / (w + T(2.71051e-20));
+    q = lane_sum(q);
+    w = lane_sum(w);
+    if (threadIdx.x == 0)
+        out[i] = q / (w + T(2.71051e-20));
 }
 
 //---------------------------------------------------------------------------
@@ -2755,8 +2762,8 @@ struct InterpL
                         : field == SPHX_FIELD_VELOCITY ? (const T *)t->vel + component
                                                        : (const T *)t->C;
         const uint32_t stride = field == SPHX_FIELD_VELOCITY ? 4u : 1u;
-        hipLaunchKernelGGL((k_interpolate<D, T>), dim3(grid_for(o->n, 64)), dim3(64), 0, o->ctx->stream,
-                           (const Rec4<T> *)o->posvol, o->n, (const Rec4<T> *)t->posvol, data, stride,
+        hipLaunchKernelGGL((k_interpolate<D, T>), dim3(o->n), dim3(64), 0, o->ctx->stream,
+                           (const Rec4<T> *)o->posvol, (const Rec4<T> *)t->posvol, data, stride,
                            rel->chunk_offset, rel->neighbor_size, rel->slice, (const KernelPoly<T> *)rel->poly,
                            (T *)o->interp);
         LAUNCH_CHECK();

@@ -178,5 +178,14 @@ __device__ __forceinline__ double wave_sum(double v)
         v += __shfl_xor(v, off, 64);
     return v;
 }
+// sum over the L lanes of a group (consecutive lanes, L a power of 2), in every lane
+template <int L = 64, class T>
+__device__ __forceinline__ T lane_sum(T v)
+{
+#pragma unroll
+    for (int off = L / 2; off > 0; off >>= 1)
+        v += __shfl_xor(v, off, 64);
+    return v;
+}
 
 } // namespace sphx
