@@ -155,21 +155,19 @@ sphx_status refresh_staging(sphx_batch *b)
     for (auto &sc : b->scenes)
         if (sc.staged && sc.inner->stage_stale)
         {
-            sphx_status s = relation_stage(sc.inner);
+            sphx_status s = ensure_staged(sc.inner);
             if (s)
                 return s;
             SPHX_HIP(hipStreamSynchronize(sc.inner->source->ctx->stream));
-            sc.inner->stage_stale = false;
         }
     return SPHX_OK;
 }
 
 sphx_status upload_records(sphx_batch *b)
 {
-    if (!b->tables_dirty)
-        return SPHX_OK;
+    // also lists that the caller rebuilt between two steps
     sphx_status s = refresh_staging(b);
-    if (s)
+    if (s || !b->tables_dirty)
         return s;
     SPHX_HIP(hipMemcpyAsync(b->scene_tab, b->scene_tab_h.data(), b->scene_tab_h.size(), hipMemcpyHostToDevice,
                             b->stream));

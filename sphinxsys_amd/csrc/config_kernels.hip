@@ -1740,6 +1740,16 @@ sphx_status relation_stage(sphx_relation *rel)
     return SPHX_OK;
 }
 
+sphx_status ensure_staged(sphx_relation *rel)
+{
+    if (!rel->staged || !rel->stage_stale)
+        return SPHX_OK;
+    sphx_status s = relation_stage(rel);
+    if (!s)
+        rel->stage_stale = false;
+    return s;
+}
+
 // ParticleSortCK::prepareSequence + sort (particle_sort_ck.hpp:61-90): on
 // return b->sequence holds the sorted Morton keys and b->perm the permutation
 sphx_status morton_sequence(sphx_body *b, sphx_cell_linked_list *cll)

@@ -39,10 +39,17 @@ __device__ __forceinline__ float inv_sqrt<float>(float r2)
 {
     return rsqrtf(fmaxf(r2, 1e-30f));
 }
+// Halley's third-order iteration on the hardware's estimate y: with e = 1 - r2 y^2,
+// y (1 + e / 2 + 3 e^2 / 8) is off by 5 e^3 / 16, far below its rounding.  Seven
+// instructions instead of the thirty of a correctly rounded square root and
+// division.
 template <>
 __device__ __forceinline__ double inv_sqrt<double>(double r2)
 {
-    return 1.0 / sqrt(fmax(r2, 1e-300));
+    const double x = fmax(r2, 1e-300);
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
 __device__ __forceinline__ float frac_part(float x) { return __builtin_amdgcn_fractf(x); }
@@ -192,6 +199,46 @@ __device__ __forceinline__ T eval_poly(const PolyLDS<T> &lds, T r, T x_per_r)
     return ((c[3] * f + c[2]) * f + c[1]) * f + c[0];
 }
 
+// The tabulated kernel gradient over grad_scale at distance r, without the
+// table: the kernel is 0.625 dq^4 x (x - 20)^3 in the table coordinate x, a
+// quartic with leading coefficient 1 (times the scale), so the Lagrange cubic
+// through the nodes loc - 1 .. loc + 2 is the quartic less the product of the
+// distances to them, (f + 1) f (f - 1)(f - 2) = u (u - 2) with f = x - loc and
+// u = f^2 - f.  The FP64 passes use it: a table interval is a 32-byte LDS read
+// at random among the lanes and 8 registers for each pair in flight (pass 1 takes
+// 140 registers instead of 220, pass 2 174 instead of 256).  FP32-mixed keeps
+// the table: there the closed form made pass 1 slower (8M particles: 826 -> 873
+// us) and pass 2 faster (1125 -> 1070 us) by as much.
+__device__ __forceinline__ double kernel_gradient(double r, double x_per_r)
+{
+    const double f = frac_part(r * x_per_r), t = fma(r, x_per_r, -20.0);
+    const double u = fma(f, f, -f);
+    return fma(r * x_per_r, t * t * t, -(u * (u - 2.0)));
+}
+template <class T>
+constexpr bool kClosedGradient = std::is_same<T, double>::value;
+
+// the gradient tables of a pass in LDS, where it reads them
+template <class T>
+__device__ __forceinline__ void stage_gradients(const FluidArgs<T> &a, PolyLDS<T> &poly_in, PolyLDS<T> *poly_w)
+{
+    if constexpr (!kClosedGradient<T>)
+    {
+        stage_poly(poly_in, a.poly, true);
+        for (int k = 0; k < a.n_wall; ++k)
+            stage_poly(poly_w[k], a.wall[k].poly, true);
+    }
+}
+// kernel gradient of a wall pair
+template <class T>
+__device__ __forceinline__ T wall_gradient(const PolyLDS<T> &lds, const KernelPoly<T> *poly, T r)
+{
+    if constexpr (kClosedGradient<T>)
+        return poly->grad_scale * kernel_gradient(r, poly->x_per_r);
+    else
+        return eval_poly(lds, r, poly->x_per_r);
+}
+
 // walk the neighbour entries of one particle (slice layout: entry k at
 // base + 64 k); the indices of a batch are loaded before any of them is used
 // so that their latency overlaps
@@ -264,15 +311,15 @@ __device__ __forceinline__ T pair_kernel(const Coef4<T> &c, T f)
 // the positions are no longer needed (so the batch's records and geometry do
 // not hold registers at the same time); pair(record, geo) finishes a pair.
 // Pairs are finished in list order with the arithmetic of eval_poly, so the
-// sums are those of the plain walk.
+// sums are those of the plain walk.  In double the kernel gradient is the closed
+// form over grad_scale, which the caller's sums are multiplied by at the end.
 template <int D, uint32_t KB = 8, class T, class I, class Fetch, class Late, class Pair>
 __device__ __forceinline__ void walk_pipelined(const I *entries, uint32_t base, uint32_t count,
                                                const PV<T, D> &pi, const PolyLDS<T> &lds, T x_per_r,
                                                Fetch &&fetch, Late &&late, Pair &&pair)
 {
-    // pairs per batch: 8; 4 measured slower in double (4 waves per SIMD instead
-    // of 2); 6 is faster for the FP32-mixed passes: pass 2 spills at 8 under its
-    // register cap, pass 1 at 6 fits five waves per SIMD
+    // pairs per batch: 8 in double; 6 is faster for the FP32-mixed passes: pass 2
+    // spills at 8 under its register cap, pass 1 at 6 fits five waves per SIMD
     constexpr uint32_t kBatch = KB;
     const uint32_t nbatch = (count + kBatch - 1) / kBatch;
     uint32_t next[kBatch];
@@ -296,6 +343,26 @@ __device__ __forceinline__ void walk_pipelined(const I *entries, uint32_t base, 
 #pragma unroll
         for (uint32_t q = 0; q < kBatch; ++q)
             rec[q] = fetch(idx[q]);
+        if constexpr (kClosedGradient<T>)
+        {
+            // the batch's reads issued together, then each pair from start to end
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (uint32_t q = 0; q < kBatch; ++q)
+                if (FULL || q < rem)
+                {
+                    PairGeo<T> g;
+                    const PV<T, D> &pj = rec[q].pv;
+                    g.dx = pi.x - pj.x;
+                    g.dy = pi.y - pj.y;
+                    g.dz = D == 3 ? pi.z - pj.z : T(0);
+                    const T r2 = D == 3 ? dot3(g.dx, g.dx, g.dy, g.dy, g.dz, g.dz) : mad2(g.dx, g.dx, g.dy, g.dy);
+                    g.ir = inv_sqrt(r2);
+                    g.w = kernel_gradient(r2 * g.ir, x_per_r);
+                    pair(rec[q], g);
+                }
+            return;
+        }
         PairGeo<T> g[kBatch];
         int loc[kBatch];
         T f[kBatch];
@@ -403,25 +470,137 @@ struct Mat3
 };
 
 //---------------------------------------------------------------------------
+// Staged neighbour records in LDS.  A lane reads its neighbours' records at
+// random, so each array holds elements of at most 16 bytes one after another:
+// (x, y, z|Vol, Vol|0) in float, (x, y) and (z, Vol) or Vol in double (a 32-byte
+// record would use half of the banks in each of its two reads).
+//---------------------------------------------------------------------------
+template <class T, int D>
+struct StagedPV
+{
+    static constexpr size_t kBytes = sizeof(Rec4<T>);
+    Rec4<T> *rec;
+    __device__ __forceinline__ StagedPV(unsigned char *lds, uint32_t) : rec((Rec4<T> *)lds) {}
+    __device__ __forceinline__ void put(uint32_t r, const Rec4<T> &v) { rec[r] = v; }
+    __device__ __forceinline__ PV<T, D> get(uint32_t r) const { return load_pv<T, D>(rec, r); }
+};
+template <int D>
+struct StagedPV<double, D>
+{
+    static constexpr size_t kBytes = D == 3 ? 32 : 24;
+    double2 *xy;
+    double *zv;
+    __device__ __forceinline__ StagedPV(unsigned char *lds, uint32_t cap) : xy((double2 *)lds), zv((double *)(xy + cap))
+    {
+    }
+    __device__ __forceinline__ void put(uint32_t r, const Rec4<double> &v)
+    {
+        xy[r] = double2{v.x, v.y};
+        if (D == 3)
+            *(double2 *)(zv + 2u * r) = double2{v.z, v.w};
+        else
+            zv[r] = v.z;
+    }
+    __device__ __forceinline__ PV<double, D> get(uint32_t r) const
+    {
+        const double2 a = xy[r];
+        if (D == 2)
+            return PV<double, D>{a.x, a.y, 0.0, zv[r]};
+        const double2 b = *(const double2 *)(zv + 2u * r);
+        return PV<double, D>{a.x, a.y, b.x, b.y};
+    }
+};
+// staged velocities: one array per component in float, (x, y) and z in double
+template <class T, int D>
+struct StagedVec
+{
+    static constexpr size_t kBytes = 3 * sizeof(T);
+    T *x, *y, *z;
+    __device__ __forceinline__ StagedVec(unsigned char *lds, uint32_t cap) : x((T *)lds), y(x + cap), z(y + cap) {}
+    __device__ __forceinline__ void put(uint32_t r, const Rec4<T> &v)
+    {
+        x[r] = v.x;
+        y[r] = v.y;
+        if (D == 3)
+            z[r] = v.z;
+    }
+    __device__ __forceinline__ Rec4<T> get(uint32_t r) const { return Rec4<T>{x[r], y[r], D == 3 ? z[r] : T(0), T(0)}; }
+};
+template <int D>
+struct StagedVec<double, D>
+{
+    static constexpr size_t kBytes = D == 3 ? 24 : 16;
+    double2 *xy;
+    double *z;
+    __device__ __forceinline__ StagedVec(unsigned char *lds, uint32_t cap) : xy((double2 *)lds), z((double *)(xy + cap))
+    {
+    }
+    __device__ __forceinline__ void put(uint32_t r, const Rec4<double> &v)
+    {
+        xy[r] = double2{v.x, v.y};
+        if (D == 3)
+            z[r] = v.z;
+    }
+    __device__ __forceinline__ Rec4<double> get(uint32_t r) const
+    {
+        const double2 a = xy[r];
+        return Rec4<double>{a.x, a.y, D == 3 ? z[r] : 0.0, 0.0};
+    }
+};
+
+// Records staged at most, by what lets several 256-thread blocks share the
+// 160 KB of a CU; a block with a larger set reads its neighbours from global
+// memory in that kernel.  FP32-mixed: pass 1 20 B a record, five blocks; pass 2
+// 28 B, four blocks; the sums 16 B, six.  FP64 in 3D: pass 1 40 B, three blocks;
+// pass 2 56 B, two; the sums 32 B, three; in 2D a block has about 450 distinct
+// neighbours and 768 records leave four blocks or more.
+template <int D, int P>
+__host__ __device__ constexpr uint32_t pass1_cap()
+{
+    return P == P_MIXED ? 1400 : D == 3 ? 1344 : 768;
+}
+template <int D, int P>
+__host__ __device__ constexpr uint32_t pass2_cap()
+{
+    return P == P_MIXED ? 1400 : D == 3 ? 1440 : 768;
+}
+template <int D, int P>
+__host__ __device__ constexpr uint32_t sum_cap()
+{
+    return P == P_MIXED || D == 3 ? kStageCap : 768;
+}
+template <int D, int P>
+constexpr size_t pass1_lds()
+{
+    using T = typename Prec<P>::T;
+    return pass1_cap<D, P>() * (StagedPV<T, D>::kBytes + sizeof(T));
+}
+template <int D, int P>
+constexpr size_t pass2_lds()
+{
+    using T = typename Prec<P>::T;
+    return pass2_cap<D, P>() * (StagedPV<T, D>::kBytes + StagedVec<T, D>::kBytes);
+}
+template <int D, int P>
+constexpr size_t sum_lds()
+{
+    return sum_cap<D, P>() * StagedPV<typename Prec<P>::T, D>::kBytes;
+}
+static_assert(pass1_cap<3, P_MIXED>() <= kStageCap && pass2_cap<3, P_FP64>() <= kStageCap, "a prefix of the staging capacity");
+
+//---------------------------------------------------------------------------
 // pass 1: inner + wall interact of AcousticStep1stHalf, then its update
 // (v += (F_prior + F) / m dt); optionally the 2nd half's initialize.
 // CORR (LinearCorrectionCK): the inner pair term 2 AverageP(B_j p_i, B_i p_j) e_ij
 // = k (p_i B_j + p_j B_i) e_ij is summed as p_i grad_sum_i + B_i sum_j p_j dW V_j e_ij
 // (grad_sum_i = sum_j B_j e_ij dW V_j is fixed while positions and volumes are),
 // the wall term as B_i sum_w (p_i + p_w) dW V_w e.
-// The FP32-mixed pass stages at most kPass1Cap records (20 B each: 28 KB and
-// the static tables, five blocks a CU) and walks six pairs per batch (94
-// VGPRs: five waves per SIMD, no spills); a block with a larger staged set
-// reads its neighbours from global memory in this pass.
+// The FP32-mixed pass walks six pairs per batch (94 VGPRs: five waves per SIMD,
+// no spills).  The FP64 passes are bound by their neighbour reads: 989k particles
+// in 3D took 425 us (pass 1) and 572 us (pass 2) a launch with 32-byte records
+// gathered through the vector cache at two waves per SIMD, 248 and 325 us with
+// the block's records staged in LDS.
 //---------------------------------------------------------------------------
-constexpr uint32_t kPass1Cap = 1400;
-static_assert(kPass1Cap <= kStageCap, "pass 1 stages a prefix of the staging capacity");
-
-template <int P>
-__host__ __device__ constexpr uint32_t pass1_cap()
-{
-    return P == P_MIXED ? kPass1Cap : kStageCap;
-}
 
 template <int D, int P, bool RIEMANN, bool FUSE_INIT_2ND, bool CORR>
 __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> &a, const uint32_t blk, double dt_d)
@@ -432,22 +611,21 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
     __shared__ PolyLDS<T> poly_in;
     __shared__ PolyLDS<T> poly_w[kMaxWalls];
     extern __shared__ __align__(32) unsigned char staged_lds[];
-    stage_poly(poly_in, a.poly, true);
-    for (int k = 0; k < a.n_wall; ++k)
-        stage_poly(poly_w[k], a.wall[k].poly, true);
+    stage_gradients(a, poly_in, poly_w);
     const uint32_t i = blk * kThreads + threadIdx.x;
     // staged neighbour records: (x, y, z|Vol, Vol|0) and p of the block's distinct neighbours
-    Rec4<T> *s_pv = (Rec4<T> *)staged_lds;
-    T *s_p = (T *)(s_pv + pass1_cap<P>());
+    constexpr uint32_t kCap = pass1_cap<D, P>();
+    StagedPV<T, D> s_pv(staged_lds, kCap);
+    T *s_p = (T *)(staged_lds + kCap * StagedPV<T, D>::kBytes);
     const uint32_t n_staged = a.stage_count ? a.stage_count[blk] : kStageOverflow;
-    const bool staged = n_staged <= pass1_cap<P>(); // kStageOverflow is above any cap
+    const bool staged = n_staged <= kCap; // kStageOverflow is above any cap
     if (staged)
     {
         const uint32_t *keys = a.stage_keys + (size_t)blk * a.stage_cap;
         for (uint32_t r = threadIdx.x; r < n_staged; r += kThreads)
         {
             const uint32_t j = keys[r];
-            s_pv[r] = a.posvol[j];
+            s_pv.put(r, a.posvol[j]);
             s_p[r] = a.p[j];
         }
     }
@@ -481,11 +659,19 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
     if (staged)
         walk_pipelined<D, kWalkBatch>(
             a.local_slice, nb, nc, pi, poly_in, x_per_r,
-            [&](uint32_t r) { return Rec{load_pv<T, D>(s_pv, r), s_p[r]}; }, no_late, pair);
+            [&](uint32_t r) { return Rec{s_pv.get(r), s_p[r]}; }, no_late, pair);
     else
         walk_pipelined<D, kWalkBatch>(
             a.slice, nb, nc, pi, poly_in, x_per_r,
             [&](uint32_t j) { return Rec{load_pv<T, D>(a.posvol, j), a.p[j]}; }, no_late, pair);
+    if constexpr (kClosedGradient<T>)
+    {
+        const T grad_scale = a.poly->grad_scale;
+        fx *= grad_scale;
+        fy *= grad_scale;
+        fz *= grad_scale;
+        cd *= grad_scale;
+    }
     const T k_avg = T(2) * a.inv_rho0c0_sum * a.rho0c0; // 2 * AverageP / (p_i + p_j)
     const T vol_i = pi.vol;
     T Fx = a.force[0][i], Fy = a.force[1][i], Fz = D == 3 ? a.force[2][i] : T(0);
@@ -516,7 +702,6 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
         for (int k = 0; k < a.n_wall; ++k)
         {
             const WallArgs<T> &w = a.wall[k];
-            const T w_x_per_r = w.poly->x_per_r;
             T wx = 0, wy = 0, wz = 0, wcd = 0;
             const uint32_t mb = w.chunk[i >> 6] + (i & 63u), mc = w.count[i];
             for (uint32_t k2 = 0; k2 < mc; ++k2)
@@ -527,7 +712,7 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
                 const T r2 = D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy;
                 const T ir = inv_sqrt(r2);
                 const T r = r2 * ir;
-                const T dWV = eval_poly(poly_w[k], r, w_x_per_r) * pj.vol;
+                const T dWV = wall_gradient(poly_w[k], w.poly, r) * pj.vol;
                 const T ex = dx * ir, ey = dy * ir, ez = D == 3 ? dz * ir : T(0);
                 T face = -((apx - w.acc[0][j]) * ex + (apy - w.acc[1][j]) * ey);
                 if (D == 3)
@@ -800,16 +985,8 @@ __device__ __forceinline__ void trav_walk(const TravArgs &t, const TravLane &L, 
 // AcousticTimeStepCK for the next sub-step, max-reduced into the max lanes at max_slot.
 //---------------------------------------------------------------------------
 // CORR (LinearCorrectionCK): the divergence uses B_i e_ij in place of e_ij
-// Pass 2 stages at most kPass2Cap records, as (x, y, z|Vol, Vol|0) plus the
-// three velocity components in separate arrays (28 B a record), so that with
-// the static tables a block takes at most 40 KB of LDS and four blocks fit a
-// CU; a block with a larger staged set reads its neighbours from global
-// memory in this pass only.
-constexpr uint32_t kPass2Cap = 1400;
-static_assert(kPass2Cap <= kStageCap, "pass 2 stages a prefix of the staging capacity");
-
 // FP32-mixed: registers capped for 4 waves per SIMD, which its 40 KB of LDS
-// per block allows; FP64 (not staged) keeps its registers
+// per block allows; FP64 (two blocks a CU by its LDS) keeps its registers
 // TRAV: the inner neighbours by the cell traversal (one-wave blocks, 3D,
 // FP32-mixed, not staged by the stored lists' sets)
 template <int D, int P, bool RIEMANN, bool FUSE_CFL, bool CORR, bool TRAV = false>
@@ -825,29 +1002,22 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
     __shared__ PolyLDS<T> poly_w[kMaxWalls];
     __shared__ double wave_red[kThreads / 64];
     extern __shared__ __align__(32) unsigned char staged_lds[];
-    stage_poly(poly_in, a.poly, true);
-    for (int k = 0; k < a.n_wall; ++k)
-        stage_poly(poly_w[k], a.wall[k].poly, true);
+    stage_gradients(a, poly_in, poly_w);
     const uint32_t i = blk * NT + threadIdx.x;
     // staged neighbour records: (x, y, z|Vol, Vol|0) and the velocity components
-    Rec4<T> *s_pv = (Rec4<T> *)staged_lds;
-    // (no opaque base as in pass 1: its extra register makes this pass spill,
-    // 45% slower measured)
-    T *s_vx = (T *)(s_pv + kPass2Cap), *s_vy = s_vx + kPass2Cap, *s_vz = s_vy + kPass2Cap;
+    constexpr uint32_t kCap = pass2_cap<D, P>();
+    StagedPV<T, D> s_pv(staged_lds, kCap);
+    StagedVec<T, D> s_v(staged_lds + kCap * StagedPV<T, D>::kBytes, kCap);
     const uint32_t n_staged = a.stage_count ? a.stage_count[blk] : kStageOverflow;
-    const bool staged = n_staged <= kPass2Cap; // kStageOverflow is above any cap
+    const bool staged = n_staged <= kCap; // kStageOverflow is above any cap
     if (staged)
     {
         const uint32_t *keys = a.stage_keys + (size_t)blk * a.stage_cap;
         for (uint32_t r = threadIdx.x; r < n_staged; r += kThreads)
         {
             const uint32_t j = keys[r];
-            s_pv[r] = a.posvol[j];
-            const Rec4<T> v = a.vel[j];
-            s_vx[r] = v.x;
-            s_vy[r] = v.y;
-            if (D == 3)
-                s_vz[r] = v.z;
+            s_pv.put(r, a.posvol[j]);
+            s_v.put(r, a.vel[j]);
         }
     }
     // the traversal's staged box: records, particle indices, column starts
@@ -914,14 +1084,20 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
         else if (staged)
             walk_pipelined<D, kWalkBatch>(
                 a.local_slice, nb, nc, pi, poly_in, x_per_r,
-                [&](uint32_t r) {
-                    return Rec{load_pv<T, D>(s_pv, r), Rec4<T>{s_vx[r], s_vy[r], D == 3 ? s_vz[r] : T(0), T(0)}};
-                },
+                [&](uint32_t r) { return Rec{s_pv.get(r), s_v.get(r)}; },
                 no_late, pair);
         else
             walk_pipelined<D, kWalkBatch>(
                 a.slice, nb, nc, pi, poly_in, x_per_r,
                 [&](uint32_t j) { return Rec{load_pv<T, D>(a.posvol, j), a.vel[j]}; }, no_late, pair);
+        if constexpr (kClosedGradient<T>)
+        {
+            const T grad_scale = a.poly->grad_scale;
+            div *= grad_scale;
+            px *= grad_scale;
+            py *= grad_scale;
+            pz *= grad_scale;
+        }
         const T C_i = full_C<P>(a.C[i]);
         const T vol_i = pi.vol;
         T dC = a.dC[i] + div * C_i;
@@ -930,7 +1106,6 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
         for (int k = 0; k < a.n_wall; ++k)
         {
             const WallArgs<T> &w = a.wall[k];
-            const T w_x_per_r = w.poly->x_per_r;
             T wdiv = 0, wx = 0, wy = 0, wz = 0;
             const uint32_t mb = w.chunk[i >> 6] + (i & 63u), mc = w.count[i];
             for (uint32_t k2 = 0; k2 < mc; ++k2)
@@ -940,7 +1115,7 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
                 const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
                 const T r2 = D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy;
                 const T ir = inv_sqrt(r2);
-                const T dWV = eval_poly(poly_w[k], r2 * ir, w_x_per_r) * pj.vol;
+                const T dWV = wall_gradient(poly_w[k], w.poly, r2 * ir) * pj.vol;
                 const T ex = dx * ir, ey = dy * ir, ez = D == 3 ? dz * ir : T(0);
                 const T vdx = T(2) * (vi.x - w.vel[0][j]), vdy = T(2) * (vi.y - w.vel[1][j]);
                 const T vdz = D == 3 ? T(2) * (vi.z - w.vel[2][j]) : T(0);
@@ -1041,9 +1216,10 @@ __device__ __forceinline__ void summation_body(const FluidArgs<typename Prec<P>:
         stage_poly(poly_w[k], a.wall[k].poly, false);
     const uint32_t i = blk * kThreads + threadIdx.x;
     // staged neighbour records: (x, y, z, Vol_ref) of the block's distinct neighbours
-    Rec4<T> *s_pv = (Rec4<T> *)staged_lds;
+    constexpr uint32_t kCap = sum_cap<D, P>();
+    StagedPV<T, D> s_pv(staged_lds, kCap);
     const uint32_t n_staged = a.stage_count ? a.stage_count[blk] : kStageOverflow;
-    const bool staged = n_staged != kStageOverflow;
+    const bool staged = n_staged <= kCap; // kStageOverflow is above any cap
     if (staged)
     {
         const uint32_t *keys = a.stage_keys + (size_t)blk * a.stage_cap;
@@ -1055,7 +1231,7 @@ __device__ __forceinline__ void summation_body(const FluidArgs<typename Prec<P>:
                 rec.w = a.Vol_ref[j];
             else
                 rec.z = a.Vol_ref[j];
-            s_pv[r] = rec;
+            s_pv.put(r, rec);
         }
     }
     __syncthreads();
@@ -1073,7 +1249,7 @@ __device__ __forceinline__ void summation_body(const FluidArgs<typename Prec<P>:
     };
     const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
     if (staged)
-        for_each_neighbor(a.local_slice, nb, nc, [&](uint32_t r) { pair(load_pv<T, D>(s_pv, r)); });
+        for_each_neighbor(a.local_slice, nb, nc, [&](uint32_t r) { pair(s_pv.get(r)); });
     else
         for_each_neighbor(a.slice, nb, nc, [&](uint32_t j) {
             PV<T, D> pj = load_pv<T, D>(a.posvol, j);
@@ -1163,14 +1339,15 @@ __global__ void __launch_bounds__(kThreads) k_correction(FluidArgs<typename Prec
         stage_poly(poly_w[k], a.wall[k].poly, true);
     const uint32_t blk = xcd_block_index();
     const uint32_t i = blk * kThreads + threadIdx.x;
-    Rec4<T> *s_pv = (Rec4<T> *)staged_lds;
+    constexpr uint32_t kCap = sum_cap<D, P>();
+    StagedPV<T, D> s_pv(staged_lds, kCap);
     const uint32_t n_staged = a.stage_count ? a.stage_count[blk] : kStageOverflow;
-    const bool staged = n_staged != kStageOverflow;
+    const bool staged = n_staged <= kCap; // kStageOverflow is above any cap
     if (staged)
     {
         const uint32_t *keys = a.stage_keys + (size_t)blk * a.stage_cap;
         for (uint32_t r = threadIdx.x; r < n_staged; r += kThreads)
-            s_pv[r] = a.posvol[keys[r]];
+            s_pv.put(r, a.posvol[keys[r]]);
     }
     __syncthreads();
     if (i >= a.n)
@@ -1198,7 +1375,7 @@ __global__ void __launch_bounds__(kThreads) k_correction(FluidArgs<typename Prec
     const T x_per_r = a.poly->x_per_r;
     const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
     if (staged)
-        for_each_neighbor(a.local_slice, nb, nc, [&](uint32_t r) { acc(load_pv<T, D>(s_pv, r), poly_in, x_per_r); });
+        for_each_neighbor(a.local_slice, nb, nc, [&](uint32_t r) { acc(s_pv.get(r), poly_in, x_per_r); });
     else
         for_each_neighbor(a.slice, nb, nc, [&](uint32_t j) { acc(load_pv<T, D>(a.posvol, j), poly_in, x_per_r); });
     for (int k = 0; k < a.n_wall; ++k)
@@ -2345,7 +2522,7 @@ struct SummationL
         FluidArgs<T> a = fluid_args<T>(b);
         attach_relations(a, inner, c, nc);
         ProfileScope prof(b->ctx, "compression_summation");
-        const size_t lds = a.stage_count ? (size_t)a.stage_cap * sizeof(Rec4<T>) : 0;
+        const size_t lds = a.stage_count ? sum_lds<D, P>() : 0;
         allow_lds(k_summation<D, P>, lds);
         hipLaunchKernelGGL((k_summation<D, P>), dim3(grid_for(b->n, kThreads)), dim3(kThreads), lds,
                            b->ctx->stream, a);
@@ -2435,7 +2612,7 @@ struct Acoustic1L
         }
         ProfileScope prof(b->ctx, "acoustic_pass1");
         const bool rs = riemann != SPHX_RIEMANN_NONE;
-        const size_t lds = a.stage_count ? (size_t)pass1_cap<P>() * (sizeof(Rec4<T>) + sizeof(T)) : 0;
+        const size_t lds = a.stage_count ? pass1_lds<D, P>() : 0;
         SPHX_PASS_VARIANTS(k_pass1, rs, fuse_init_2nd, corr, a, dt);
         LAUNCH_CHECK();
         return SPHX_OK;
@@ -2463,7 +2640,7 @@ struct Acoustic2L
         ProfileScope prof(b->ctx, "acoustic_pass2");
         const bool rs = riemann != SPHX_RIEMANN_NONE;
         const bool cfl = max_slot != nullptr;
-        const size_t lds = a.stage_count ? (size_t)kPass2Cap * (sizeof(Rec4<T>) + 3 * sizeof(T)) : 0;
+        const size_t lds = a.stage_count ? pass2_lds<D, P>() : 0;
         SPHX_PASS_VARIANTS(k_pass2, rs, cfl, corr, a, dt, max_slot);
         LAUNCH_CHECK();
         return SPHX_OK;
@@ -2473,7 +2650,8 @@ struct Acoustic2L
 sphx_status acoustic_1st_half(sphx_relation *inner, sphx_relation *const *w, int nw, int riemann, double dt,
                               bool fuse_init_2nd)
 {
-    return dispatch<Acoustic1L>(inner->source, inner, w, nw, riemann, dt, fuse_init_2nd, false);
+    sphx_status s = ensure_staged(inner);
+    return s ? s : dispatch<Acoustic1L>(inner->source, inner, w, nw, riemann, dt, fuse_init_2nd, false);
 }
 
 sphx_status acoustic_2nd_half(sphx_relation *inner, sphx_relation *const *w, int nw, int riemann, double dt,
@@ -2481,7 +2659,8 @@ sphx_status acoustic_2nd_half(sphx_relation *inner, sphx_relation *const *w, int
 {
     sphx_body *b = inner->source;
     unsigned long long *slot = fuse_cfl ? b->ctx->scalars_d + SLOT_MAX : nullptr;
-    return dispatch<Acoustic2L>(b, inner, w, nw, riemann, dt, run_init, slot, false);
+    sphx_status s = ensure_staged(inner);
+    return s ? s : dispatch<Acoustic2L>(b, inner, w, nw, riemann, dt, run_init, slot, false);
 }
 
 sphx_status acoustic_2nd_half_traversal(sphx_relation *inner, sphx_relation *const *w, int nw, int riemann, double dt)
@@ -2531,8 +2710,8 @@ sphx_status acoustic_2nd_half_traversal(sphx_relation *inner, sphx_relation *con
 sphx_status acoustic_1st_half_corrected(sphx_relation *inner, sphx_relation *const *w, int nw, int riemann,
                                         double dt, bool fuse_init_2nd)
 {
-    sphx_status s = refresh_grad_sum(inner->source, inner);
-    if (s)
+    sphx_status s = ensure_staged(inner);
+    if (s || (s = refresh_grad_sum(inner->source, inner)))
         return s;
     return dispatch<Acoustic1L>(inner->source, inner, w, nw, riemann, dt, fuse_init_2nd, true);
 }
@@ -2542,7 +2721,8 @@ sphx_status acoustic_2nd_half_corrected(sphx_relation *inner, sphx_relation *con
 {
     sphx_body *b = inner->source;
     unsigned long long *slot = fuse_cfl ? b->ctx->scalars_d + SLOT_MAX : nullptr;
-    return dispatch<Acoustic2L>(b, inner, w, nw, riemann, dt, run_init, slot, true);
+    sphx_status s = ensure_staged(inner);
+    return s ? s : dispatch<Acoustic2L>(b, inner, w, nw, riemann, dt, run_init, slot, true);
 }
 
 template <int D, int P>
@@ -2555,7 +2735,7 @@ struct CorrectionL
             return SPHX_OK;
         FluidArgs<T> a = fluid_args<T>(b);
         attach_relations(a, inner, c, nc);
-        const size_t lds = a.stage_count ? (size_t)a.stage_cap * sizeof(Rec4<T>) : 0;
+        const size_t lds = a.stage_count ? sum_lds<D, P>() : 0;
         allow_lds(k_correction<D, P>, lds);
         hipLaunchKernelGGL((k_correction<D, P>), dim3(grid_for(b->n, kThreads)), dim3(kThreads), lds,
                            b->ctx->stream, a, alpha);
@@ -2567,6 +2747,9 @@ struct CorrectionL
 sphx_status linear_correction_matrix(sphx_relation *inner, sphx_relation *const *c, int nc, double alpha)
 {
     sphx_body *b = inner->source;
+    sphx_status s = ensure_staged(inner);
+    if (s)
+        return s;
     ProfileScope prof(b->ctx, "linear_correction");
     b->state_version++;
     return dispatch<CorrectionL>(b, inner, c, nc, alpha);
@@ -2846,7 +3029,8 @@ static sphx_status build_poly_t(sphx_relation *rel)
     KernelPoly<T> kp;
     expand_table(w, (long double)fW, kp.w, dq);
     expand_table(dw, (long double)fdW, kp.dw, dq);
-    kp.inv_h = T(inv_h);
+    // dW = 0.625 (q - 2)^3 q = 0.625 dq^4 (x - 20)^3 x
+    kp.grad_scale = T(0.625L * dq * dq * dq * dq * (long double)fdW);
     kp.x_per_r = T(inv_h * (1.0 / dq));
     // W0 = src_inv_h^D dimfac W(0); interpolateCubic at q = 0 returns data[1] scaled by the basis
     const double f1 = 0.0, f0 = dq, f2 = -dq, f3 = -2 * dq;
@@ -2938,15 +3122,9 @@ struct BatchL
     using T = typename Prec<P>::T;
     static const SceneArgs<T> *tab(const BatchFluid &b) { return (const SceneArgs<T> *)b.tab; }
     // dynamic LDS of the staged neighbour passes (as the single-scene launchers)
-    static size_t lds_sum(const BatchFluid &b) { return (size_t)b.stage_cap * sizeof(Rec4<T>); }
-    static size_t lds_pass1(const BatchFluid &b)
-    {
-        return b.stage_cap ? (size_t)pass1_cap<P>() * (sizeof(Rec4<T>) + sizeof(T)) : 0;
-    }
-    static size_t lds_pass2(const BatchFluid &b)
-    {
-        return b.stage_cap ? (size_t)kPass2Cap * (sizeof(Rec4<T>) + 3 * sizeof(T)) : 0;
-    }
+    static size_t lds_sum(const BatchFluid &b) { return b.stage_cap ? sum_lds<D, P>() : 0; }
+    static size_t lds_pass1(const BatchFluid &b) { return b.stage_cap ? pass1_lds<D, P>() : 0; }
+    static size_t lds_pass2(const BatchFluid &b) { return b.stage_cap ? pass2_lds<D, P>() : 0; }
     static sphx_status head(const BatchFluid &b)
     {
         const dim3 g(b.blocks), blk(kThreads), gs(grid_for(b.n_scenes, 64)), bs(64);

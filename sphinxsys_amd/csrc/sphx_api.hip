@@ -560,9 +560,6 @@ sphx_status sphx_context_create(int device, sphx_context **out)
         return st;
     std::unique_ptr<sphx_context> ctx(new sphx_context());
     ctx->device = device;
-    int lds = 0;
-    if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) == hipSuccess && lds > 0)
-        ctx->max_lds = (size_t)lds;
     // on a failure below, the stream and the pinned mirror go back to the pools
     struct Release
     {
@@ -1072,23 +1069,16 @@ static sphx_status relation_create(sphx_body *src, sphx_body *tar, sphx_cell_lin
             return st;
     }
     SPHX_HIP(hipMemsetAsync(r->neighbor_size, 0, (size_t)(src->n + 1) * sizeof(uint32_t), src->ctx->stream));
-    if (inner && src->desc.kind == SPHX_BODY_FLUID && src->n > 0)
+    if (inner && src->desc.kind == SPHX_BODY_FLUID && src->n >= (src->P == P_FP64 ? kStageMin64 : 1u))
     {
-        // LDS staging of the acoustic passes: the 2nd pass stages two 4-wide
-        // records per distinct neighbour; keep 8 KiB for the static tables
-        // (MIXED only: FP64 records would halve the occupancy of the passes)
-        const size_t rec2 = 2 * (src->P == P_FP64 ? sizeof(Rec4<double>) : sizeof(Rec4<float>));
-        const size_t cap = kStageCap;
-        if (src->P == P_MIXED && cap * rec2 + 8192 <= std::min<size_t>(src->ctx->max_lds, 65536))
-        {
-            const size_t nblocks = (src->n + kStageBlock - 1) / kStageBlock;
-            r->staged = true;
-            r->stage_cap = (uint32_t)cap;
-            sphx_status st;
-            if ((st = dev_alloc(stream, (void **)&r->stage_count, nblocks * sizeof(uint32_t))) ||
-                (st = dev_alloc(stream, (void **)&r->stage_keys, nblocks * cap * sizeof(uint32_t))))
-                return st;
-        }
+        // LDS staging of the acoustic passes and the sums over the inner neighbours
+        const size_t nblocks = (src->n + kStageBlock - 1) / kStageBlock;
+        r->staged = true;
+        r->stage_cap = kStageCap;
+        sphx_status st;
+        if ((st = dev_alloc(stream, (void **)&r->stage_count, nblocks * sizeof(uint32_t))) ||
+            (st = dev_alloc(stream, (void **)&r->stage_keys, nblocks * kStageCap * sizeof(uint32_t))))
+            return st;
     }
     sphx_status s = build_kernel_poly(r.get());
     if (s)
@@ -1199,9 +1189,7 @@ sphx_status sphx_update_relation(sphx_relation *r)
     }
     r->kmax = kmax;
     r->slice_total = nchunks * kmax * 64;
-    if ((s = relation_stage(r)))
-        return s;
-    r->stage_stale = false;
+    r->stage_stale = true; // the staging sets follow with the first dynamics that reads the lists often
     r->csr_valid = false; // the CSR view (offsets and indices) is built when read
     r->built = true;
     r->builds++;
@@ -1599,7 +1587,8 @@ sphx_status sphx_advection_step(sphx_relation *inner, sphx_relation *const *wall
     sphx_body *b = inner->source;
     sphx_context *ctx = b->ctx;
     SPHX_HIP(hipSetDevice(ctx->device));
-    if ((s = compression_summation(inner, walls, n_wall)) || (s = density_regularization(b, cfg->flow_type)) ||
+    if ((s = ensure_staged(inner)) || (s = compression_summation(inner, walls, n_wall)) ||
+        (s = density_regularization(b, cfg->flow_type)) ||
         (s = advection_step_setup(b)))
         return s;
     // AdvectionTimeStepCK on the device: the loop below runs without host

@@ -60,7 +60,8 @@ struct KernelPoly
 {
     T w[kPolyIntervals][4];  // W  = sum_k w[loc][k]  f^k   (factor inv_h^D dimfac folded in)
     T dw[kPolyIntervals][4]; // dW = sum_k dw[loc][k] f^k   (factor inv_h^(D+1) dimfac folded in)
-    T inv_h, x_per_r, w0;    // x_per_r = inv_h / dq; w0 = W0 of the source with its own factor
+    T x_per_r, w0;           // x_per_r = inv_h / dq; w0 = W0 of the source with its own factor
+    T grad_scale;            // dW = grad_scale kernel_gradient(x): 0.625 dq^4 inv_h^(D+1) dimfac
 };
 
 // Mesh of a cell linked list, base_mesh.cpp:6-16 / base_mesh.hxx:9-26.

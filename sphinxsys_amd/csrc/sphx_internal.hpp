@@ -45,6 +45,11 @@ constexpr int kScalarSlots = 1024;
 constexpr uint32_t kStageBlock = 256;          // source particles per staging block
 constexpr uint32_t kStageOverflow = 0xffffffffu;
 constexpr uint32_t kStageCap = 1536;           // distinct neighbours staged per block (LDS records)
+// FP64 fluid bodies of at least this many particles stage their inner
+// neighbours.  Below, the sets cost what they save or more (per advection step
+// in 3D: 8,000 particles 45 us for the sets, 51 us less in the passes; 800 in 2D
+// 19 against 6; above, 90,000: 67 against 185)
+constexpr uint32_t kStageMin64 = 16384;
 // reported through the relation build's `needed` slot when a search box holds
 // more candidates than the tiled build's masks: rebuild with the scan kernel
 constexpr unsigned long long kTooDense = 1ull << 40;
@@ -75,7 +80,6 @@ struct sphx_context
 {
     int device = 0;
     hipStream_t stream = nullptr;
-    size_t max_lds = 65536; // shared memory per workgroup of the device
     // HIP-event kernel timing (sphx_profile_*)
     bool profiling = false;
     bool profile_passes_only = false; // time only the acoustic pass launches
@@ -179,7 +183,7 @@ struct sphx_relation
     // stage_count[b] of them, or kStageOverflow) and the neighbour entries as
     // 16-bit ranks into that set (local_slice, same slice layout)
     bool staged = false;
-    bool stage_stale = false;             // lists rebuilt without their staging sets (the passes gather directly)
+    bool stage_stale = true;              // lists rebuilt since their staging sets (readers gather directly)
     uint32_t stage_cap = 0;
     uint32_t *stage_count = nullptr;
     uint32_t *stage_keys = nullptr;
@@ -222,6 +226,12 @@ void relation_prefilter(const sphx_relation *rel, float *thr_lo, float *thr_hi, 
 sphx_status relation_build(sphx_relation *rel, uint32_t kmax, unsigned long long *needed, bool scan);
 // the LDS staging sets of a staged relation, from its finished slices
 sphx_status relation_stage(sphx_relation *rel);
+// the same where they are stale.  Made by the first acoustic half step,
+// correction matrix or whole advection step after a list build, not by the
+// build: a density summation alone (a neighbour search without a time loop)
+// gains less from the sets than they cost (2.1M particles FP32-mixed, sort,
+// lists and summation: 3.48 -> 3.34 ms without them)
+sphx_status ensure_staged(sphx_relation *rel);
 // per-cell flags of a target cell list: any particle within the search box
 sphx_status cell_near_flags(sphx_cell_linked_list *cll);
 sphx_status morton_sequence(sphx_body *b, sphx_cell_linked_list *cll);

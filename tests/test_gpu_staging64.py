@@ -1,0 +1,66 @@
+"""The FP64 sums over LDS-staged neighbour records against the oracle: sizes on
+both sides of the smallest staged body, a last block of a few particles, and
+shuffled orders, whose blocks have more distinct neighbours than the kernels
+stage (some of them in a window of 1024, all of them in a full shuffle) and
+read from global memory.
+
+Gate: 1e-10 relative L2, the FP64 gate of the same comparison on smaller
+bodies (sums of 80 terms, summed in the same order with other roundings)."""
+import numpy as np
+import pytest
+
+from sphinxsys_amd import _capi as capi
+from sphinxsys_amd import cases, ck
+from tests.test_gpu_parity import FP64_GATE, Pair, jittered_lattice, rel_l2, shuffled
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dim,m,window", [(2, 127, None), (2, 129, None), (2, 129, 0), (3, 25, None), (3, 26, None),
+                                          (3, 26, 1024), (3, 26, 0)])
+def test_fp64_sums_staged_and_not(hip, oracle, dim, m, window):
+    dp = 0.02
+    fluid = jittered_lattice(dim, m, dp, 3)
+    if window is not None:
+        fluid = shuffled(fluid, window, 4)
+    wall = jittered_lattice(dim, m, dp, 5, jitter=0.0)
+    wall = wall[wall[:, -1] < 3 * dp].copy()
+    wall[:, -1] -= 3 * dp
+    pr = Pair(hip, oracle, fluid, dp, wall, np.tile(np.eye(dim)[-1], (len(wall), 1)), capi.FP64, rho0=1000.0, c0=20.0)
+    rng = np.random.default_rng(6)
+    n = len(fluid)
+    pr.write("Compression", 1.0 + rng.uniform(-0.01, 0.01, n))
+    pr.write("CompressionRate", rng.uniform(-0.5, 0.5, n))
+    pr.write("Velocity", rng.normal(scale=0.3, size=(n, dim)))
+    pr.both(lambda s: ck.CompressionSummation(s["inner"], *s["walls"]).exec())
+    pr.both(lambda s: ck.LinearCorrectionMatrixComplex(s["inner"], *s["walls"], alpha=0.5).exec())
+    names = ["CompressionSummation", "LinearCorrectionMatrix"]
+    for correction in (capi.CORRECTION_NONE, capi.CORRECTION_LINEAR):
+        pr.both(lambda s: ck.AcousticStep1stHalf(s["inner"], *s["walls"], correction=correction).exec(2e-5))
+        pr.both(lambda s: ck.AcousticStep2ndHalf(s["inner"], *s["walls"], correction=correction).exec(2e-5))
+        for name in names + ["Pressure", "Force", "CompressionRate", "Compression", "Velocity", "Displacement"]:
+            g, c = pr.read(name)
+            assert rel_l2(g, c) < FP64_GATE, (correction, name)
+    pr.close()
+
+
+@pytest.mark.parametrize("precision", [capi.FP64, capi.MIXED])
+def test_lists_rebuilt_between_batch_steps(hip, precision):
+    """A caller that rebuilds a scene's lists between two batch steps leaves their
+    staging sets to the next reader: the batched scene still equals itself alone."""
+    geom = cases.dambreak_2d(dp=0.01)  # 20,000 particles: staged in both precisions
+    alone, batched = (cases.DamBreak(hip, geom, precision) for _ in range(2))
+    for sc in (alone, batched):
+        sc.initialize()
+        sc.ctx.synchronize()
+    batch = ck.BatchAdvection(hip, [batched.advection], options=dict(use_graph=1, autotune=0))
+    for _ in range(4):
+        alone.advection_step()
+        batch.exec()
+        batched.complex_relation.exec()
+        batched.ctx.synchronize()
+    for name in ("Position", "Velocity", "Compression", "Force"):
+        assert np.array_equal(alone.fluid.read(name), batched.fluid.read(name)), name
+    batch.close()
+    alone.close()
+    batched.close()
