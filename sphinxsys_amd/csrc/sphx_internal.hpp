@@ -42,6 +42,7 @@ struct Scratch
 };
 
 constexpr int kScalarSlots = 1024;
+constexpr size_t kSmallTransfer = 256u << 10; // field transfers up to this size use the context's own pinned memory
 constexpr uint32_t kStageBlock = 256;          // source particles per staging block
 constexpr uint32_t kStageOverflow = 0xffffffffu;
 constexpr uint32_t kStageCap = 1536;           // distinct neighbours staged per block (LDS records)
@@ -92,7 +93,8 @@ struct sphx_context
     std::vector<hipEvent_t> event_pool; // recorded events ready for reuse
     std::map<std::string, std::pair<double, uint64_t>> profile; // stage -> (ms, launches)
     unsigned long long *scalars_d = nullptr; // kScalarSlots u64 on the device
-    unsigned long long *scalars_h = nullptr; // pinned mirror
+    unsigned long long *scalars_h = nullptr; // pinned mirror, followed by kSmallTransfer bytes for field transfers
+    unsigned char *transfer_h = nullptr;
     sphx::Scratch sort_keys, sort_vals, sort_hist, scan_blocks, reduce_parts, gather_tmp, cll_cursor;
     // while set, the acoustic kernels take dt and their run flag from the SLOT_STEP slots
     bool device_step = false;

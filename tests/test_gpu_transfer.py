@@ -1,0 +1,46 @@
+"""Body.write followed by Body.read returns the written values in the body's
+precision, exactly, for each device layout (three arrays, 4-wide records, one
+array, matrix components, 32-bit integers), with sizes on both sides of the
+context's own pinned buffer (262,144 bytes), of one half of a staging buffer
+(8 MiB) and over more than two halves."""
+import numpy as np
+import pytest
+
+from sphinxsys_amd import _capi as capi
+from sphinxsys_amd import ck
+
+pytestmark = pytest.mark.gpu
+
+# name, values per particle in D dimensions, kept in double in both precisions
+FIELDS = [("Position", lambda d: d, True), ("Velocity", lambda d: d, False), ("Pressure", lambda d: 1, False),
+          ("Compression", lambda d: 1, False), ("Force", lambda d: d, False),
+          ("LinearCorrectionMatrix", lambda d: d * d, False)]
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("precision", [capi.FP64, capi.MIXED])
+@pytest.mark.parametrize("n", [1, 257, 3641, 10923, 32769, 349526, 800001])
+def test_write_read_round_trip(hip, dim, precision, n):
+    rng = np.random.default_rng(n)
+    ctx = ck.Context(hip)
+    body = ck.Body(ctx, dim, n, 0.01, capi.BODY_FLUID, precision)
+    kept = {}
+    for name, width, double in FIELDS:
+        v = rng.normal(size=(n, width(dim)) if width(dim) > 1 else n)
+        v.flat[0] = -0.0
+        if name == "Compression":
+            v = 1.0 + 0.01 * v
+        if name == "LinearCorrectionMatrix":
+            v = v.reshape(n, dim, dim)
+        body.write(name, v)
+        if precision == capi.MIXED and not double:
+            v = (v - 1.0).astype(np.float32).astype(float) + 1.0 if name == "Compression" else v.astype(np.float32)
+        kept[name] = v.astype(float)
+    ids = rng.permutation(n).astype(np.uint32)
+    body.write("OriginalID", ids)
+    for name, v in kept.items():
+        got = body.read(name)
+        assert np.array_equal(got, v) and np.array_equal(np.signbit(got), np.signbit(v)), name
+    assert np.array_equal(body.read("OriginalID"), ids)
+    body.close()
+    ctx.close()
