@@ -64,11 +64,11 @@ struct sphx_batch
     // device buffers
     std::vector<void *> allocations;
     void *scene_tab = nullptr, *cll_tab = nullptr, *build_tab = nullptr, *stage_tab = nullptr;
-    uint32_t *map256 = nullptr, *map_cells = nullptr, *map_tiles = nullptr, *map_chunks[3] = {nullptr, nullptr, nullptr};
+    uint32_t *map256 = nullptr, *map_sums = nullptr, *map_cells = nullptr, *map_tiles = nullptr, *map_chunks[3] = {nullptr, nullptr, nullptr};
     uint32_t *rel_scene = nullptr, *cursor = nullptr, *tile_sums = nullptr, *tail_on = nullptr, *gate = nullptr;
     double *time_d = nullptr;
     unsigned long long *readback = nullptr; // S * STEP_SLOTS step states, then R needed counts
-    uint32_t blocks256 = 0, blocks_cells = 0, blocks_tiles = 0, blocks_chunks[3] = {0, 0, 0};
+    uint32_t blocks256 = 0, blocks_sums = 0, blocks_cells = 0, blocks_tiles = 0, blocks_chunks[3] = {0, 0, 0};
     // pinned host mirrors
     double *time_h = nullptr;
     uint32_t *tail_on_h = nullptr;
@@ -186,7 +186,7 @@ sphx_status build_tables(sphx_batch *b)
 {
     free_tables(b);
     const size_t S = b->scenes.size();
-    std::vector<uint32_t> m256, mcells, mtiles, mchunks[3], rscene;
+    std::vector<uint32_t> m256, msums, mcells, mtiles, mchunks[3], rscene;
     std::vector<unsigned char> cll_h(S * batch_cll_args_bytes());
     size_t cells_total = 0, tiles_total = 0;
     for (size_t s = 0; s < S; ++s)
@@ -200,6 +200,10 @@ sphx_status build_tables(sphx_batch *b)
             return batch_error(SPHX_E_CAPACITY, "a batched scene exceeds 65536 blocks of particles or cells");
         for (uint32_t k = 0; k < b256; ++k)
             m256.push_back((uint32_t)(s << 16) | k);
+        // (at most 512 blocks where a scene has several lanes per particle)
+        const uint64_t bsums = ((uint64_t)n * split_lanes(b->D, b->P, n) + 255u) / 256u;
+        for (uint32_t k = 0; k < bsums; ++k)
+            msums.push_back((uint32_t)(s << 16) | k);
         for (uint32_t k = 0; k < bcells; ++k)
             mcells.push_back((uint32_t)(s << 16) | k);
         for (uint32_t k = 0; k < tiles; ++k)
@@ -231,7 +235,8 @@ sphx_status build_tables(sphx_batch *b)
         (st = alloc_dev(b, (unsigned char **)&b->cll_tab, S * batch_cll_args_bytes())) ||
         (st = alloc_dev(b, (unsigned char **)&b->build_tab, R * batch_build_args_bytes())) ||
         (st = alloc_dev(b, (unsigned char **)&b->stage_tab, S * batch_stage_args_bytes())) ||
-        (st = alloc_dev(b, &b->map256, m256.size())) || (st = alloc_dev(b, &b->map_cells, mcells.size())) ||
+        (st = alloc_dev(b, &b->map256, m256.size())) || (st = alloc_dev(b, &b->map_sums, msums.size())) ||
+        (st = alloc_dev(b, &b->map_cells, mcells.size())) ||
         (st = alloc_dev(b, &b->map_tiles, mtiles.size())) || (st = alloc_dev(b, &b->map_chunks[0], mchunks[0].size())) ||
         (st = alloc_dev(b, &b->map_chunks[1], mchunks[1].size())) ||
         (st = alloc_dev(b, &b->map_chunks[2], mchunks[2].size())) || (st = alloc_dev(b, &b->rel_scene, R)) ||
@@ -252,7 +257,8 @@ sphx_status build_tables(sphx_batch *b)
         SPHX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, b->stream));
         return SPHX_OK;
     };
-    if ((st = up(b->map256, m256.data(), m256.size() * 4)) || (st = up(b->map_cells, mcells.data(), mcells.size() * 4)) ||
+    if ((st = up(b->map256, m256.data(), m256.size() * 4)) || (st = up(b->map_sums, msums.data(), msums.size() * 4)) ||
+        (st = up(b->map_cells, mcells.data(), mcells.size() * 4)) ||
         (st = up(b->map_tiles, mtiles.data(), mtiles.size() * 4)) ||
         (st = up(b->map_chunks[0], mchunks[0].data(), mchunks[0].size() * 4)) ||
         (st = up(b->map_chunks[1], mchunks[1].data(), mchunks[1].size() * 4)) ||
@@ -261,6 +267,7 @@ sphx_status build_tables(sphx_batch *b)
         return st;
     SPHX_HIP(hipStreamSynchronize(b->stream));
     b->blocks256 = (uint32_t)m256.size();
+    b->blocks_sums = (uint32_t)msums.size();
     b->blocks_cells = (uint32_t)mcells.size();
     b->blocks_tiles = (uint32_t)mtiles.size();
     for (int w = 0; w < 3; ++w)
@@ -284,6 +291,8 @@ BatchFluid fluid_launch(sphx_batch *b)
     f.n_scenes = (uint32_t)b->scenes.size();
     f.map = b->map256;
     f.blocks = b->blocks256;
+    f.map_sums = b->map_sums;
+    f.blocks_sums = b->blocks_sums;
     f.stage_cap = 0;
     for (const auto &sc : b->scenes)
         if (sc.staged)

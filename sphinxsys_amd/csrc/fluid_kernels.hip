@@ -239,27 +239,138 @@ __device__ __forceinline__ T wall_gradient(const PolyLDS<T> &lds, const KernelPo
         return eval_poly(lds, r, poly->x_per_r);
 }
 
-// walk the neighbour entries of one particle (slice layout: entry k at
-// base + 64 k); the indices of a batch are loaded before any of them is used
-// so that their latency overlaps
-template <class I, class F>
-__device__ __forceinline__ void for_each_neighbor(const I *entries, uint32_t base, uint32_t count, F &&f)
+// The particle of a thread where S consecutive lanes share one: lane `sub` of
+// them takes every S-th neighbour from its sub-th on, the lanes' sums are added
+// (lane_sum<S>), each lane computes the update and the first one stores it.  A
+// body of few particles then has S times the wavefronts, each with an S-th of
+// the list (split_lanes: which bodies).  S = 1: one thread per particle.
+template <int S>
+struct Lanes
 {
-    constexpr uint32_t kBatch = 8;
-    uint32_t k = 0;
-    for (; k + kBatch <= count; k += kBatch)
+    uint32_t i, sub;
+    __device__ __forceinline__ explicit Lanes(uint32_t blk)
+        : i(blk * (kThreads / S) + threadIdx.x / S), sub(S > 1 ? threadIdx.x % S : 0u)
     {
-        // one pointer per batch: the 8 loads take immediate offsets (64 entries apart)
+    }
+    __device__ __forceinline__ bool first() const { return S == 1 || sub == 0u; }
+};
+
+// f(split_lanes of a body of n particles) with the lanes as a constant
+template <int D, int P, class F>
+__host__ __device__ __forceinline__ void with_lanes(uint32_t n, F &&f)
+{
+    const int lanes = split_lanes(D, P, n);
+    if constexpr (split_lanes(D, P, 0) == 8)
+    {
+        if (lanes == 8)
+            return f(std::integral_constant<int, 8>{});
+    }
+    if constexpr (split_lanes(D, P, 0) > 1)
+    {
+        if (lanes == 4)
+            return f(std::integral_constant<int, 4>{});
+    }
+    f(std::integral_constant<int, 1>{});
+}
+// the same for the sums that several lanes add up as a tree: one lane in FP32
+template <int D, int P, class F>
+__host__ __device__ __forceinline__ void with_tree_lanes(uint32_t n, F &&f)
+{
+    if constexpr (P == P_FP64)
+        with_lanes<D, P>(n, f);
+    else
+        f(std::integral_constant<int, 1>{});
+}
+
+// FP32 sums of several lanes keep the order (and the rounding) of one thread's:
+// each lane evaluates its own pair of S, and all of them then take the S terms
+// in list order from their lanes and accumulate them with the same
+// multiply-adds.  FP64 lanes add their own pairs and then each other's sums.
+template <class T, int S>
+constexpr bool kOrdered = S > 1 && std::is_same<T, float>::value;
+
+// a term (a struct of floats) of lane L of the four lanes of a particle
+template <int L, class Term>
+__device__ __forceinline__ Term quad_term(const Term &t)
+{
+    constexpr int N = sizeof(Term) / 4;
+    int v[N];
+    __builtin_memcpy(v, &t, sizeof(Term));
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        v[k] = __builtin_amdgcn_mov_dpp(v[k], L * 0x55, 0xf, 0xf, true); // quad_perm: every lane from lane L
+    Term out;
+    __builtin_memcpy(&out, v, sizeof(Term));
+    return out;
+}
+
+// Sum the terms of a list of count entries (entry k at base + 64 k):
+// add(eval(entry)), in list order for one lane (S = 1) or ordered lanes.
+template <class T, int S, class I, class Eval, class Add>
+__device__ __forceinline__ void sum_terms(const I *entries, uint32_t base, uint32_t count, uint32_t sub, Eval &&eval,
+                                          Add &&add)
+{
+    if constexpr (kOrdered<T, S>)
+    {
+        static_assert(S == 4, "a quad of lanes");
+        // two entries a lane in flight; past the end entry 0, evaluated and not added
+        constexpr uint32_t kB = 2;
+        for (uint32_t k0 = 0; k0 < count; k0 += S * kB)
+        {
+            uint32_t idx[kB];
+            decltype(eval(0u)) t[kB];
+#pragma unroll
+            for (uint32_t q = 0; q < kB; ++q)
+            {
+                const uint32_t k = k0 + q * S + sub;
+                idx[q] = entries[base + ((k < count ? k : 0u) << 6)];
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < kB; ++q)
+                t[q] = eval(idx[q]);
+#pragma unroll
+            for (uint32_t q = 0; q < kB; ++q)
+            {
+                const uint32_t k = k0 + q * S;
+                const auto t0 = quad_term<0>(t[q]), t1 = quad_term<1>(t[q]);
+                const auto t2 = quad_term<2>(t[q]), t3 = quad_term<3>(t[q]);
+                if (k < count)
+                    add(t0);
+                if (k + 1 < count)
+                    add(t1);
+                if (k + 2 < count)
+                    add(t2);
+                if (k + 3 < count)
+                    add(t3);
+            }
+        }
+    }
+    else
+        for (uint32_t k = sub; k < count; k += S)
+            add(eval((uint32_t)entries[base + (k << 6)]));
+}
+
+// walk the neighbour entries of one particle (slice layout: entry k at
+// base + 64 k), from entry sub on every S-th; the indices of a batch are loaded
+// before any of them is used so that their latency overlaps
+template <int S = 1, class I, class F>
+__device__ __forceinline__ void for_each_neighbor(const I *entries, uint32_t base, uint32_t count, uint32_t sub, F &&f)
+{
+    constexpr uint32_t kBatch = S > 1 ? 4 : 8;
+    uint32_t k = sub;
+    for (; k + S * (kBatch - 1) < count; k += S * kBatch)
+    {
+        // one pointer per batch: the loads take immediate offsets (64 S entries apart)
         const I *row = entries + base + ((size_t)k << 6);
         uint32_t idx[kBatch];
 #pragma unroll
         for (uint32_t q = 0; q < kBatch; ++q)
-            idx[q] = row[q << 6];
+            idx[q] = row[q * S << 6];
 #pragma unroll
         for (uint32_t q = 0; q < kBatch; ++q)
             f(idx[q]);
     }
-    for (; k < count; ++k)
+    for (; k < count; k += S)
         f((uint32_t)entries[base + (k << 6)]);
 }
 
@@ -300,6 +411,31 @@ __device__ __forceinline__ T pair_kernel(const Coef4<T> &c, T f)
     return ((c.c3 * f + c.c2) * f + c.c1) * f + c.c0;
 }
 
+// the geometry of one pair from start to end
+template <int D, class T>
+__device__ __forceinline__ PairGeo<T> pair_geometry_of(const PV<T, D> &pi, const PV<T, D> &pj, const PolyLDS<T> &lds,
+                                                       T x_per_r)
+{
+    PairGeo<T> g;
+    if constexpr (kClosedGradient<T>)
+    {
+        g.dx = pi.x - pj.x;
+        g.dy = pi.y - pj.y;
+        g.dz = D == 3 ? pi.z - pj.z : T(0);
+        const T r2 = D == 3 ? dot3(g.dx, g.dx, g.dy, g.dy, g.dz, g.dz) : mad2(g.dx, g.dx, g.dy, g.dy);
+        g.ir = inv_sqrt(r2);
+        g.w = kernel_gradient(r2 * g.ir, x_per_r);
+    }
+    else
+    {
+        int loc;
+        T f;
+        pair_geometry<D>(pi, pj, x_per_r, g, loc, f);
+        g.w = pair_kernel(*reinterpret_cast<const Coef4<T> *>(lds.c[loc]), f);
+    }
+    return g;
+}
+
 // The neighbour walk of for_each_neighbor with the latencies overlapped: the
 // entries are taken in batches of 8; the list entries of the next batch are
 // loaded while the current one is evaluated, and for each batch the records
@@ -311,9 +447,10 @@ __device__ __forceinline__ T pair_kernel(const Coef4<T> &c, T f)
 // the positions are no longer needed (so the batch's records and geometry do
 // not hold registers at the same time); pair(record, geo) finishes a pair.
 // Pairs are finished in list order with the arithmetic of eval_poly, so the
-// sums are those of the plain walk.  In double the kernel gradient is the closed
+// sums are those of the plain walk.  With S lanes a particle, base and count are
+// those of the lane's own entries (split_count), S apart.  In double the kernel gradient is the closed
 // form over grad_scale, which the caller's sums are multiplied by at the end.
-template <int D, uint32_t KB = 8, class T, class I, class Fetch, class Late, class Pair>
+template <int D, uint32_t KB, int S = 1, class T, class I, class Fetch, class Late, class Pair>
 __device__ __forceinline__ void walk_pipelined(const I *entries, uint32_t base, uint32_t count,
                                                const PV<T, D> &pi, const PolyLDS<T> &lds, T x_per_r,
                                                Fetch &&fetch, Late &&late, Pair &&pair)
@@ -324,10 +461,10 @@ __device__ __forceinline__ void walk_pipelined(const I *entries, uint32_t base, 
     const uint32_t nbatch = (count + kBatch - 1) / kBatch;
     uint32_t next[kBatch];
     auto load_entries = [&](uint32_t b) {
-        const I *row = entries + base + ((size_t)(b * kBatch) << 6);
+        const I *row = entries + base + ((size_t)(b * kBatch * S) << 6);
 #pragma unroll
         for (uint32_t q = 0; q < kBatch; ++q)
-            next[q] = b * kBatch + q < count ? (uint32_t)row[q << 6] : 0u;
+            next[q] = b * kBatch + q < count ? (uint32_t)row[q * S << 6] : 0u;
     };
     // one batch; the last one (FULL false) may hold fewer than kBatch entries
     auto run_batch = [&](uint32_t b, auto full) {
@@ -350,17 +487,7 @@ __device__ __forceinline__ void walk_pipelined(const I *entries, uint32_t base, 
 #pragma unroll
             for (uint32_t q = 0; q < kBatch; ++q)
                 if (FULL || q < rem)
-                {
-                    PairGeo<T> g;
-                    const PV<T, D> &pj = rec[q].pv;
-                    g.dx = pi.x - pj.x;
-                    g.dy = pi.y - pj.y;
-                    g.dz = D == 3 ? pi.z - pj.z : T(0);
-                    const T r2 = D == 3 ? dot3(g.dx, g.dx, g.dy, g.dy, g.dz, g.dz) : mad2(g.dx, g.dx, g.dy, g.dy);
-                    g.ir = inv_sqrt(r2);
-                    g.w = kernel_gradient(r2 * g.ir, x_per_r);
-                    pair(rec[q], g);
-                }
+                    pair(rec[q], pair_geometry_of<D>(pi, rec[q].pv, lds, x_per_r));
             return;
         }
         PairGeo<T> g[kBatch];
@@ -394,6 +521,13 @@ __device__ __forceinline__ void walk_pipelined(const I *entries, uint32_t base, 
         run_batch(b, std::true_type{});
     if (nfull < nbatch)
         run_batch(nfull, std::false_type{});
+}
+
+// entries of lane sub of S in a list of count
+template <int S>
+__device__ __forceinline__ uint32_t split_count(uint32_t count, uint32_t sub)
+{
+    return S == 1 ? count : (count + (S - 1u) - sub) / S;
 }
 
 //---------------------------------------------------------------------------
@@ -602,7 +736,7 @@ static_assert(pass1_cap<3, P_MIXED>() <= kStageCap && pass2_cap<3, P_FP64>() <= 
 // the block's records staged in LDS.
 //---------------------------------------------------------------------------
 
-template <int D, int P, bool RIEMANN, bool FUSE_INIT_2ND, bool CORR>
+template <int D, int P, bool RIEMANN, bool FUSE_INIT_2ND, bool CORR, int S>
 __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> &a, const uint32_t blk, double dt_d)
 {
     using T = typename Prec<P>::T;
@@ -612,12 +746,13 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
     __shared__ PolyLDS<T> poly_w[kMaxWalls];
     extern __shared__ __align__(32) unsigned char staged_lds[];
     stage_gradients(a, poly_in, poly_w);
-    const uint32_t i = blk * kThreads + threadIdx.x;
+    const Lanes<S> lane(blk);
+    const uint32_t i = lane.i;
     // staged neighbour records: (x, y, z|Vol, Vol|0) and p of the block's distinct neighbours
     constexpr uint32_t kCap = pass1_cap<D, P>();
     StagedPV<T, D> s_pv(staged_lds, kCap);
     T *s_p = (T *)(staged_lds + kCap * StagedPV<T, D>::kBytes);
-    const uint32_t n_staged = a.stage_count ? a.stage_count[blk] : kStageOverflow;
+    const uint32_t n_staged = S == 1 && a.stage_count ? a.stage_count[blk] : kStageOverflow;
     const bool staged = n_staged <= kCap; // kStageOverflow is above any cap
     if (staged)
     {
@@ -643,27 +778,49 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
         PV<T, D> pv;
         T p;
     };
-    auto pair = [&](const Rec &rj, const PairGeo<T> &g) {
-        const T dWV = g.w * rj.pv.vol;
-        const T s = (CORR ? rj.p : p_i + rj.p) * dWV * g.ir;
-        fx += s * g.dx;
-        fy += s * g.dy;
-        if (D == 3)
-            fz += s * g.dz;
-        if (RIEMANN)
-            cd += (p_i - rj.p) * dWV;
+    struct Term
+    {
+        T s, dx, dy, dz, dp, dWV;
     };
+    auto term = [&](const Rec &rj, const PairGeo<T> &g) {
+        const T dWV = g.w * rj.pv.vol;
+        return Term{(CORR ? rj.p : p_i + rj.p) * dWV * g.ir, g.dx, g.dy, g.dz, p_i - rj.p, dWV};
+    };
+    auto add = [&](const Term &t) {
+        fx = fma(t.s, t.dx, fx);
+        fy = fma(t.s, t.dy, fy);
+        if (D == 3)
+            fz = fma(t.s, t.dz, fz);
+        if (RIEMANN)
+            cd = fma(t.dp, t.dWV, cd);
+    };
+    auto pair = [&](const Rec &rj, const PairGeo<T> &g) { add(term(rj, g)); };
     const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
     auto no_late = [](uint32_t, Rec &) {};
     constexpr uint32_t kWalkBatch = P == P_MIXED ? 6u : 8u;
-    if (staged)
+    auto global_rec = [&](uint32_t j) { return Rec{load_pv<T, D>(a.posvol, j), a.p[j]}; };
+    if constexpr (kOrdered<T, S>)
+        sum_terms<T, S>(
+            a.slice, nb, nc, lane.sub,
+            [&](uint32_t j) {
+                const Rec rj = global_rec(j);
+                return term(rj, pair_geometry_of<D>(pi, rj.pv, poly_in, x_per_r));
+            },
+            add);
+    else if (staged)
         walk_pipelined<D, kWalkBatch>(
-            a.local_slice, nb, nc, pi, poly_in, x_per_r,
-            [&](uint32_t r) { return Rec{s_pv.get(r), s_p[r]}; }, no_late, pair);
+            a.local_slice, nb, nc, pi, poly_in, x_per_r, [&](uint32_t r) { return Rec{s_pv.get(r), s_p[r]}; }, no_late,
+            pair);
     else
-        walk_pipelined<D, kWalkBatch>(
-            a.slice, nb, nc, pi, poly_in, x_per_r,
-            [&](uint32_t j) { return Rec{load_pv<T, D>(a.posvol, j), a.p[j]}; }, no_late, pair);
+        walk_pipelined<D, kWalkBatch, S>(a.slice, nb + (lane.sub << 6), split_count<S>(nc, lane.sub), pi, poly_in,
+                                         x_per_r, global_rec, no_late, pair);
+    if constexpr (S > 1 && !kOrdered<T, S>)
+    {
+        fx = lane_sum<S>(fx);
+        fy = lane_sum<S>(fy);
+        fz = lane_sum<S>(fz);
+        cd = lane_sum<S>(cd);
+    }
     if constexpr (kClosedGradient<T>)
     {
         const T grad_scale = a.poly->grad_scale;
@@ -704,27 +861,41 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
             const WallArgs<T> &w = a.wall[k];
             T wx = 0, wy = 0, wz = 0, wcd = 0;
             const uint32_t mb = w.chunk[i >> 6] + (i & 63u), mc = w.count[i];
-            for (uint32_t k2 = 0; k2 < mc; ++k2)
+            struct WallTerm
             {
-                const uint32_t j = w.slice[mb + (k2 << 6)];
-                const PV<T, D> pj = load_pv<T, D>(w.posvol, j);
-                const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
-                const T r2 = D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy;
-                const T ir = inv_sqrt(r2);
-                const T r = r2 * ir;
-                const T dWV = wall_gradient(poly_w[k], w.poly, r) * pj.vol;
-                const T ex = dx * ir, ey = dy * ir, ez = D == 3 ? dz * ir : T(0);
-                T face = -((apx - w.acc[0][j]) * ex + (apy - w.acc[1][j]) * ey);
-                if (D == 3)
-                    face -= (apz - w.acc[2][j]) * ez;
-                const T p_w = p_i + rho_i * r * dmax(T(0), face);
-                const T s = (p_i + p_w) * dWV;
-                wx += s * ex;
-                wy += s * ey;
-                if (D == 3)
-                    wz += s * ez;
-                if (RIEMANN)
-                    wcd += (p_i - p_w) * dWV;
+                T s, ex, ey, ez, dp, dWV;
+            };
+            sum_terms<T, S>(
+                w.slice, mb, mc, lane.sub,
+                [&](uint32_t j) {
+                    const PV<T, D> pj = load_pv<T, D>(w.posvol, j);
+                    const T ax = w.acc[0][j], ay = w.acc[1][j], az = D == 3 ? w.acc[2][j] : T(0);
+                    const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
+                    const T r2 = D == 3 ? dot3(dx, dx, dy, dy, dz, dz) : mad2(dx, dx, dy, dy);
+                    const T ir = inv_sqrt(r2);
+                    const T r = r2 * ir;
+                    const T dWV = wall_gradient(poly_w[k], w.poly, r) * pj.vol;
+                    const T ex = dx * ir, ey = dy * ir, ez = D == 3 ? dz * ir : T(0);
+                    T face = -mad2(apx - ax, ex, apy - ay, ey);
+                    if (D == 3)
+                        face = fma(-(apz - az), ez, face);
+                    const T p_w = fma(rho_i * r, dmax(T(0), face), p_i);
+                    return WallTerm{(p_i + p_w) * dWV, ex, ey, ez, p_i - p_w, dWV};
+                },
+                [&](const WallTerm &t) {
+                    wx = fma(t.s, t.ex, wx);
+                    wy = fma(t.s, t.ey, wy);
+                    if (D == 3)
+                        wz = fma(t.s, t.ez, wz);
+                    if (RIEMANN)
+                        wcd = fma(t.dp, t.dWV, wcd);
+                });
+            if constexpr (S > 1 && !kOrdered<T, S>)
+            {
+                wx = lane_sum<S>(wx);
+                wy = lane_sum<S>(wy);
+                wz = lane_sum<S>(wz);
+                wcd = lane_sum<S>(wcd);
             }
             if (CORR)
             {
@@ -740,6 +911,8 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
                 dC += wcd * a.inv_rho0c0_ave * C_i;
         }
     }
+    if (!lane.first())
+        return;
     // inside the device-side sub-step loop the 2nd half, which sets the force
     // anew, runs next whenever this pass runs and nothing reads the force in
     // between: the store is left out there
@@ -778,10 +951,11 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
         a.dpos[2][i] = d2;
 }
 
-template <int D, int P, bool RIEMANN, bool FUSE_INIT_2ND, bool CORR>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(P == P_MIXED ? 5 : 1))) k_pass1(FluidArgs<typename Prec<P>::T> a, double dt_d)
+template <int D, int P, bool RIEMANN, bool FUSE_INIT_2ND, bool CORR, int S>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(P == P_MIXED ? 5 : 1)))
+k_pass1(FluidArgs<typename Prec<P>::T> a, double dt_d)
 {
-    pass1_body<D, P, RIEMANN, FUSE_INIT_2ND, CORR>(a, xcd_block_index(), dt_d);
+    pass1_body<D, P, RIEMANN, FUSE_INIT_2ND, CORR, S>(a, xcd_block_index(), dt_d);
 }
 
 // DissipativePJump of the Riemann solvers divided by rho0c0_geo_ave (the
@@ -989,12 +1163,12 @@ __device__ __forceinline__ void trav_walk(const TravArgs &t, const TravLane &L, 
 // per block allows; FP64 (two blocks a CU by its LDS) keeps its registers
 // TRAV: the inner neighbours by the cell traversal (one-wave blocks, 3D,
 // FP32-mixed, not staged by the stored lists' sets)
-template <int D, int P, bool RIEMANN, bool FUSE_CFL, bool CORR, bool TRAV = false>
+template <int D, int P, bool RIEMANN, bool FUSE_CFL, bool CORR, int S, bool TRAV = false>
 __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> &a, const uint32_t blk, double dt_d,
                                            unsigned long long *max_slot, const TravArgs *trav = nullptr)
 {
     using T = typename Prec<P>::T;
-    static_assert(!TRAV || (D == 3 && P == P_MIXED && !CORR), "the traversal is 3D FP32-mixed, uncorrected");
+    static_assert(!TRAV || (D == 3 && P == P_MIXED && !CORR && S == 1), "the traversal is 3D FP32-mixed, uncorrected");
     constexpr uint32_t NT = TRAV ? 64u : kThreads; // threads per block
     if (!step_dt(a, dt_d)) // block-uniform: before any barrier
         return;
@@ -1003,12 +1177,13 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
     __shared__ double wave_red[kThreads / 64];
     extern __shared__ __align__(32) unsigned char staged_lds[];
     stage_gradients(a, poly_in, poly_w);
-    const uint32_t i = blk * NT + threadIdx.x;
+    const Lanes<S> lane(blk);
+    const uint32_t i = TRAV ? blk * NT + threadIdx.x : lane.i;
     // staged neighbour records: (x, y, z|Vol, Vol|0) and the velocity components
     constexpr uint32_t kCap = pass2_cap<D, P>();
     StagedPV<T, D> s_pv(staged_lds, kCap);
     StagedVec<T, D> s_v(staged_lds + kCap * StagedPV<T, D>::kBytes, kCap);
-    const uint32_t n_staged = a.stage_count ? a.stage_count[blk] : kStageOverflow;
+    const uint32_t n_staged = S == 1 && a.stage_count ? a.stage_count[blk] : kStageOverflow;
     const bool staged = n_staged <= kCap; // kStageOverflow is above any cap
     if (staged)
     {
@@ -1045,7 +1220,11 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
             PV<T, D> pv;
             Rec4<T> v;
         };
-        auto pair = [&](const Rec &rj, const PairGeo<T> &g) {
+        struct Term
+        {
+            T u, dWV, s, ex, ey, ez;
+        };
+        auto term = [&](const Rec &rj, const PairGeo<T> &g) {
             const Rec4<T> &vj = rj.v;
             const T dWV = g.w * rj.pv.vol;
             const T ir = g.ir;
@@ -1053,43 +1232,59 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
             T u = mad2(vi.x - vj.x, ex, vi.y - vj.y, ey);
             if (D == 3)
                 u = fma(vi.z - vj.z, ez, u);
+            T uc = u;
             if (CORR)
             {
                 T bx, by, bz;
                 Bi.apply(ex, ey, ez, bx, by, bz);
-                T uc = mad2(vi.x - vj.x, bx, vi.y - vj.y, by);
+                uc = mad2(vi.x - vj.x, bx, vi.y - vj.y, by);
                 if (D == 3)
                     uc = fma(vi.z - vj.z, bz, uc);
-                div += uc * dWV;
             }
-            else
-                div += u * dWV;
+            return Term{uc, dWV, RIEMANN ? p_jump_scaled(a, u) * dWV : T(0), ex, ey, ez};
+        };
+        auto add = [&](const Term &t) {
+            div = fma(t.u, t.dWV, div);
             if (RIEMANN)
             {
-                const T s = p_jump_scaled(a, u) * dWV;
-                px += s * ex;
-                py += s * ey;
+                px = fma(t.s, t.ex, px);
+                py = fma(t.s, t.ey, py);
                 if (D == 3)
-                    pz += s * ez;
+                    pz = fma(t.s, t.ez, pz);
             }
         };
+        auto pair = [&](const Rec &rj, const PairGeo<T> &g) { add(term(rj, g)); };
         const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
         // whole records up front: loading the velocities late (as pass 1 loads
         // its pressures) makes this pass spill under its register cap
         auto no_late = [](uint32_t, Rec &) {};
         constexpr uint32_t kWalkBatch = P == P_MIXED ? 6u : 8u;
+        auto global_rec = [&](uint32_t j) { return Rec{load_pv<T, D>(a.posvol, j), a.vel[j]}; };
         if constexpr (TRAV)
             trav_walk(*trav, tl, a.posvol, i, pi, poly_in, x_per_r, t_pv, t_j, trav_cols, trav_cols + kTravCols,
                       [&](uint32_t j, const PV<T, D> &pj, const PairGeo<T> &g) { pair(Rec{pj, a.vel[j]}, g); });
+        else if constexpr (kOrdered<T, S>)
+            sum_terms<T, S>(
+                a.slice, nb, nc, lane.sub,
+                [&](uint32_t j) {
+                    const Rec rj = global_rec(j);
+                    return term(rj, pair_geometry_of<D>(pi, rj.pv, poly_in, x_per_r));
+                },
+                add);
         else if (staged)
             walk_pipelined<D, kWalkBatch>(
                 a.local_slice, nb, nc, pi, poly_in, x_per_r,
-                [&](uint32_t r) { return Rec{s_pv.get(r), s_v.get(r)}; },
-                no_late, pair);
+                [&](uint32_t r) { return Rec{s_pv.get(r), s_v.get(r)}; }, no_late, pair);
         else
-            walk_pipelined<D, kWalkBatch>(
-                a.slice, nb, nc, pi, poly_in, x_per_r,
-                [&](uint32_t j) { return Rec{load_pv<T, D>(a.posvol, j), a.vel[j]}; }, no_late, pair);
+            walk_pipelined<D, kWalkBatch, S>(a.slice, nb + (lane.sub << 6), split_count<S>(nc, lane.sub), pi, poly_in,
+                                             x_per_r, global_rec, no_late, pair);
+        if constexpr (S > 1 && !kOrdered<T, S>)
+        {
+            div = lane_sum<S>(div);
+            px = lane_sum<S>(px);
+            py = lane_sum<S>(py);
+            pz = lane_sum<S>(pz);
+        }
         if constexpr (kClosedGradient<T>)
         {
             const T grad_scale = a.poly->grad_scale;
@@ -1108,41 +1303,59 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
             const WallArgs<T> &w = a.wall[k];
             T wdiv = 0, wx = 0, wy = 0, wz = 0;
             const uint32_t mb = w.chunk[i >> 6] + (i & 63u), mc = w.count[i];
-            for (uint32_t k2 = 0; k2 < mc; ++k2)
+            struct WallTerm
             {
-                const uint32_t j = w.slice[mb + (k2 << 6)];
-                const PV<T, D> pj = load_pv<T, D>(w.posvol, j);
-                const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
-                const T r2 = D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy;
-                const T ir = inv_sqrt(r2);
-                const T dWV = wall_gradient(poly_w[k], w.poly, r2 * ir) * pj.vol;
-                const T ex = dx * ir, ey = dy * ir, ez = D == 3 ? dz * ir : T(0);
-                const T vdx = T(2) * (vi.x - w.vel[0][j]), vdy = T(2) * (vi.y - w.vel[1][j]);
-                const T vdz = D == 3 ? T(2) * (vi.z - w.vel[2][j]) : T(0);
-                T bex = ex, bey = ey, bez = ez;
-                if (CORR)
-                    Bi.apply(ex, ey, ez, bex, bey, bez);
-                T ve = vdx * bex + vdy * bey;
-                if (D == 3)
-                    ve += vdz * bez;
-                wdiv += ve * dWV;
-                if (RIEMANN)
-                {
-                    const T nx = w.normal[0][j], ny = w.normal[1][j], nz = D == 3 ? w.normal[2][j] : T(0);
-                    T en = ex * nx + ey * ny;
+                T ve, dWV, s, nx, ny, nz;
+            };
+            sum_terms<T, S>(
+                w.slice, mb, mc, lane.sub,
+                [&](uint32_t j) {
+                    const PV<T, D> pj = load_pv<T, D>(w.posvol, j);
+                    const T vdx = T(2) * (vi.x - w.vel[0][j]), vdy = T(2) * (vi.y - w.vel[1][j]);
+                    const T vdz = D == 3 ? T(2) * (vi.z - w.vel[2][j]) : T(0);
+                    const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
+                    const T r2 = D == 3 ? dot3(dx, dx, dy, dy, dz, dz) : mad2(dx, dx, dy, dy);
+                    const T ir = inv_sqrt(r2);
+                    const T dWV = wall_gradient(poly_w[k], w.poly, r2 * ir) * pj.vol;
+                    const T ex = dx * ir, ey = dy * ir, ez = D == 3 ? dz * ir : T(0);
+                    T bex = ex, bey = ey, bez = ez;
+                    if (CORR)
+                        Bi.apply(ex, ey, ez, bex, bey, bez);
+                    T ve = mad2(vdx, bex, vdy, bey);
                     if (D == 3)
-                        en += ez * nz;
-                    const T sg = en < T(0) ? T(-1) : (en > T(0) ? T(1) : T(0));
-                    const T fnx = sg * nx, fny = sg * ny, fnz = sg * nz;
-                    T u = vdx * fnx + vdy * fny;
-                    if (D == 3)
-                        u += vdz * fnz;
-                    const T s = p_jump_scaled(a, u) * dWV;
-                    wx += s * fnx;
-                    wy += s * fny;
-                    if (D == 3)
-                        wz += s * fnz;
-                }
+                        ve = fma(vdz, bez, ve);
+                    WallTerm t{ve, dWV, T(0), T(0), T(0), T(0)};
+                    if (RIEMANN)
+                    {
+                        const T nx = w.normal[0][j], ny = w.normal[1][j], nz = D == 3 ? w.normal[2][j] : T(0);
+                        T en = mad2(ex, nx, ey, ny);
+                        if (D == 3)
+                            en = fma(ez, nz, en);
+                        const T sg = en < T(0) ? T(-1) : (en > T(0) ? T(1) : T(0));
+                        t.nx = sg * nx, t.ny = sg * ny, t.nz = sg * nz;
+                        T u = mad2(vdx, t.nx, vdy, t.ny);
+                        if (D == 3)
+                            u = fma(vdz, t.nz, u);
+                        t.s = p_jump_scaled(a, u) * dWV;
+                    }
+                    return t;
+                },
+                [&](const WallTerm &t) {
+                    wdiv = fma(t.ve, t.dWV, wdiv);
+                    if (RIEMANN)
+                    {
+                        wx = fma(t.s, t.nx, wx);
+                        wy = fma(t.s, t.ny, wy);
+                        if (D == 3)
+                            wz = fma(t.s, t.nz, wz);
+                    }
+                });
+            if constexpr (S > 1 && !kOrdered<T, S>)
+            {
+                wdiv = lane_sum<S>(wdiv);
+                wx = lane_sum<S>(wx);
+                wy = lane_sum<S>(wy);
+                wz = lane_sum<S>(wz);
             }
             dC += wdiv * C_i;
             Fx += wx * zv;
@@ -1150,15 +1363,18 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
             if (D == 3)
                 Fz += wz * zv;
         }
-        a.dC[i] = dC;
-        a.force[0][i] = Fx;
-        a.force[1][i] = Fy;
-        if (D == 3)
-            a.force[2][i] = Fz;
         // UpdateKernel: C += 0.5 dt dC; rho = C rho0
         T c = a.C[i] + T(0.5) * dt * dC;
-        a.C[i] = c;
-        a.rho[i] = full_C<P>(c) * a.rho0;
+        if (lane.first())
+        {
+            a.dC[i] = dC;
+            a.force[0][i] = Fx;
+            a.force[1][i] = Fy;
+            if (D == 3)
+                a.force[2][i] = Fz;
+            a.C[i] = c;
+            a.rho[i] = full_C<P>(c) * a.rho0;
+        }
         if (FUSE_CFL)
         {
             // AcousticTimeStepCK::reduce (fluid_time_step_ck.hpp:51-57)
@@ -1187,24 +1403,24 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
     }
 }
 
-template <int D, int P, bool RIEMANN, bool FUSE_CFL, bool CORR>
+template <int D, int P, bool RIEMANN, bool FUSE_CFL, bool CORR, int S>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(P == P_MIXED ? 4 : 1)))
 k_pass2(FluidArgs<typename Prec<P>::T> a, double dt_d, unsigned long long *max_slot)
 {
-    pass2_body<D, P, RIEMANN, FUSE_CFL, CORR>(a, xcd_block_index(), dt_d, max_slot);
+    pass2_body<D, P, RIEMANN, FUSE_CFL, CORR, S>(a, xcd_block_index(), dt_d, max_slot);
 }
 
 // pass 2 with the inner neighbours by the cell traversal: one 64-particle chunk per block
 template <bool RIEMANN>
 __global__ void __launch_bounds__(64) k_pass2_traverse(FluidArgs<float> a, TravArgs t, double dt_d)
 {
-    pass2_body<3, P_MIXED, RIEMANN, false, false, true>(a, xcd_block_index(), dt_d, nullptr, &t);
+    pass2_body<3, P_MIXED, RIEMANN, false, false, 1, true>(a, xcd_block_index(), dt_d, nullptr, &t);
 }
 
 //---------------------------------------------------------------------------
 // CompressionSummation<Inner<>> + <Contact<>> (density_regularization.hpp:40-83)
 //---------------------------------------------------------------------------
-template <int D, int P>
+template <int D, int P, int S>
 __device__ __forceinline__ void summation_body(const FluidArgs<typename Prec<P>::T> &a, const uint32_t blk)
 {
     using T = typename Prec<P>::T;
@@ -1214,11 +1430,12 @@ __device__ __forceinline__ void summation_body(const FluidArgs<typename Prec<P>:
     stage_poly(poly_in, a.poly, false);
     for (int k = 0; k < a.n_wall; ++k)
         stage_poly(poly_w[k], a.wall[k].poly, false);
-    const uint32_t i = blk * kThreads + threadIdx.x;
+    const Lanes<S> lane(blk);
+    const uint32_t i = lane.i;
     // staged neighbour records: (x, y, z, Vol_ref) of the block's distinct neighbours
     constexpr uint32_t kCap = sum_cap<D, P>();
     StagedPV<T, D> s_pv(staged_lds, kCap);
-    const uint32_t n_staged = a.stage_count ? a.stage_count[blk] : kStageOverflow;
+    const uint32_t n_staged = S == 1 && a.stage_count ? a.stage_count[blk] : kStageOverflow;
     const bool staged = n_staged <= kCap; // kStageOverflow is above any cap
     if (staged)
     {
@@ -1239,47 +1456,56 @@ __device__ __forceinline__ void summation_body(const FluidArgs<typename Prec<P>:
         return;
     const T x_per_r = a.poly->x_per_r;
     const PV<T, D> pi = load_pv<T, D>(a.posvol, i);
-    T s = a.poly->w0 * a.Vol_ref[i];
+    T s = kOrdered<T, S> || lane.first() ? a.poly->w0 * a.Vol_ref[i] : T(0);
+    struct Term
+    {
+        T W, vol;
+    };
     // W_ij Vref_j (pj.vol carries Vref_j)
-    auto pair = [&](const PV<T, D> &pj) {
+    auto term = [&](const PV<T, D> &pj, const PolyLDS<T> &poly, T per_r) {
         const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
-        const T r2 = D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy;
+        const T r2 = D == 3 ? dot3(dx, dx, dy, dy, dz, dz) : mad2(dx, dx, dy, dy);
         const T r = sqrt(r2);
-        s += eval_poly(poly_in, r, x_per_r) * pj.vol;
+        return Term{eval_poly(poly, r, per_r), pj.vol};
+    };
+    auto add = [&](const Term &t) { s = fma(t.W, t.vol, s); };
+    auto global_term = [&](uint32_t j) {
+        PV<T, D> pj = load_pv<T, D>(a.posvol, j);
+        pj.vol = a.Vol_ref[j];
+        return term(pj, poly_in, x_per_r);
     };
     const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
-    if (staged)
-        for_each_neighbor(a.local_slice, nb, nc, [&](uint32_t r) { pair(s_pv.get(r)); });
+    if constexpr (kOrdered<T, S>)
+        sum_terms<T, S>(a.slice, nb, nc, lane.sub, global_term, add);
+    else if (staged)
+        for_each_neighbor(a.local_slice, nb, nc, 0u, [&](uint32_t r) { add(term(s_pv.get(r), poly_in, x_per_r)); });
     else
-        for_each_neighbor(a.slice, nb, nc, [&](uint32_t j) {
-            PV<T, D> pj = load_pv<T, D>(a.posvol, j);
-            pj.vol = a.Vol_ref[j];
-            pair(pj);
-        });
+        for_each_neighbor<S>(a.slice, nb, nc, lane.sub, [&](uint32_t j) { add(global_term(j)); });
     for (int k = 0; k < a.n_wall; ++k)
     {
         const WallArgs<T> &w = a.wall[k];
         const T w_x_per_r = w.poly->x_per_r;
-        const uint32_t mb = w.chunk[i >> 6] + (i & 63u), mc = w.count[i];
-        for (uint32_t k2 = 0; k2 < mc; ++k2)
-        {
-            const uint32_t j = w.slice[mb + (k2 << 6)];
-            const PV<T, D> pj = load_pv<T, D>(w.posvol, j);
-            const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
-            const T r2 = D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy;
-            const T r = sqrt(r2);
-            s += eval_poly(poly_w[k], r, w_x_per_r) * w.Vol_ref[j];
-        }
+        sum_terms<T, S>(
+            w.slice, w.chunk[i >> 6] + (i & 63u), w.count[i], lane.sub,
+            [&](uint32_t j) {
+                PV<T, D> pj = load_pv<T, D>(w.posvol, j);
+                pj.vol = w.Vol_ref[j];
+                return term(pj, poly_w[k], w_x_per_r);
+            },
+            add);
     }
-    a.S[i] = s;
+    if constexpr (S > 1 && !kOrdered<T, S>)
+        s = lane_sum<S>(s);
+    if (lane.first())
+        a.S[i] = s;
 }
 
 // FP32-mixed: six blocks a CU (26 KB of staged records each, 66 VGPRs)
-template <int D, int P>
+template <int D, int P, int S>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(P == P_MIXED ? 6 : 1)))
 k_summation(FluidArgs<typename Prec<P>::T> a)
 {
-    summation_body<D, P>(a, xcd_block_index());
+    summation_body<D, P, S>(a, xcd_block_index());
 }
 
 //---------------------------------------------------------------------------
@@ -1327,7 +1553,7 @@ __device__ __forceinline__ void inverse_d(const double (&x)[3][3], double (&r)[3
             r[i][j] = cof[j][i] * inv_det;
 }
 
-template <int D, int P>
+template <int D, int P, int S>
 __global__ void __launch_bounds__(kThreads) k_correction(FluidArgs<typename Prec<P>::T> a, double alpha)
 {
     using T = typename Prec<P>::T;
@@ -1338,10 +1564,11 @@ __global__ void __launch_bounds__(kThreads) k_correction(FluidArgs<typename Prec
     for (int k = 0; k < a.n_wall; ++k)
         stage_poly(poly_w[k], a.wall[k].poly, true);
     const uint32_t blk = xcd_block_index();
-    const uint32_t i = blk * kThreads + threadIdx.x;
+    const Lanes<S> lane(blk);
+    const uint32_t i = lane.i;
     constexpr uint32_t kCap = sum_cap<D, P>();
     StagedPV<T, D> s_pv(staged_lds, kCap);
-    const uint32_t n_staged = a.stage_count ? a.stage_count[blk] : kStageOverflow;
+    const uint32_t n_staged = S == 1 && a.stage_count ? a.stage_count[blk] : kStageOverflow;
     const bool staged = n_staged <= kCap; // kStageOverflow is above any cap
     if (staged)
     {
@@ -1375,16 +1602,25 @@ __global__ void __launch_bounds__(kThreads) k_correction(FluidArgs<typename Prec
     const T x_per_r = a.poly->x_per_r;
     const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
     if (staged)
-        for_each_neighbor(a.local_slice, nb, nc, [&](uint32_t r) { acc(s_pv.get(r), poly_in, x_per_r); });
+        for_each_neighbor(a.local_slice, nb, nc, 0u, [&](uint32_t r) { acc(s_pv.get(r), poly_in, x_per_r); });
     else
-        for_each_neighbor(a.slice, nb, nc, [&](uint32_t j) { acc(load_pv<T, D>(a.posvol, j), poly_in, x_per_r); });
+        for_each_neighbor<S>(a.slice, nb, nc, lane.sub,
+                             [&](uint32_t j) { acc(load_pv<T, D>(a.posvol, j), poly_in, x_per_r); });
     for (int k = 0; k < a.n_wall; ++k)
     {
         const WallArgs<T> &w = a.wall[k];
         const uint32_t mb = w.chunk[i >> 6] + (i & 63u), mc = w.count[i];
-        for (uint32_t k2 = 0; k2 < mc; ++k2)
+        for (uint32_t k2 = lane.sub; k2 < mc; k2 += S)
             acc(load_pv<T, D>(w.posvol, w.slice[mb + (k2 << 6)]), poly_w[k], w.poly->x_per_r);
     }
+    if constexpr (S > 1)
+    {
+        bxx = lane_sum<S>(bxx), bxy = lane_sum<S>(bxy), byy = lane_sum<S>(byy);
+        if (D == 3)
+            bxz = lane_sum<S>(bxz), byz = lane_sum<S>(byz), bzz = lane_sum<S>(bzz);
+    }
+    if (!lane.first())
+        return;
     // UpdateKernel::update (kernel_correction_ck.hpp:58-65), in double
     double B[3][3] = {{-(double)bxx, -(double)bxy, -(double)bxz},
                       {-(double)bxy, -(double)byy, -(double)byz},
@@ -1421,20 +1657,21 @@ __global__ void __launch_bounds__(kThreads) k_correction(FluidArgs<typename Prec
 
 // grad_sum_i = sum_j B_j e_ij dW_ij V_j over the inner neighbours (the part of
 // the corrected pressure force that does not change within an advection step)
-template <int D, int P>
+template <int D, int P, int S>
 __global__ void __launch_bounds__(kThreads) k_correction_grad(FluidArgs<typename Prec<P>::T> a)
 {
     using T = typename Prec<P>::T;
     __shared__ PolyLDS<T> poly_in;
     stage_poly(poly_in, a.poly, true);
     __syncthreads();
-    const uint32_t i = xcd_block_index() * kThreads + threadIdx.x;
+    const Lanes<S> lane(xcd_block_index());
+    const uint32_t i = lane.i;
     if (i >= a.n)
         return;
     const PV<T, D> pi = load_pv<T, D>(a.posvol, i);
     const T x_per_r = a.poly->x_per_r;
     T gx = 0, gy = 0, gz = 0;
-    for_each_neighbor(a.slice, a.chunk[i >> 6] + (i & 63u), a.count[i], [&](uint32_t j) {
+    for_each_neighbor<S>(a.slice, a.chunk[i >> 6] + (i & 63u), a.count[i], lane.sub, [&](uint32_t j) {
         const PV<T, D> pj = load_pv<T, D>(a.posvol, j);
         const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
         const T r2 = D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy;
@@ -1449,6 +1686,10 @@ __global__ void __launch_bounds__(kThreads) k_correction_grad(FluidArgs<typename
         if (D == 3)
             gz += bz * dWV;
     });
+    if constexpr (S > 1)
+        gx = lane_sum<S>(gx), gy = lane_sum<S>(gy), gz = lane_sum<S>(gz);
+    if (!lane.first())
+        return;
     a.grad_sum[0][i] = gx;
     a.grad_sum[1][i] = gy;
     if (D == 3)
@@ -1461,7 +1702,7 @@ __global__ void __launch_bounds__(kThreads) k_correction_grad(FluidArgs<typename
 // -sum dW V r, held at twice the threshold for a particle that neither was nor
 // neighbours the previous free surface, then the contact part ...
 //---------------------------------------------------------------------------
-template <int D, int P>
+template <int D, int P, int S>
 __global__ void __launch_bounds__(kThreads) k_surface_div(FluidArgs<typename Prec<P>::T> a)
 {
     using T = typename Prec<P>::T;
@@ -1471,7 +1712,8 @@ __global__ void __launch_bounds__(kThreads) k_surface_div(FluidArgs<typename Pre
     for (int k = 0; k < a.n_wall; ++k)
         stage_poly(poly_w[k], a.wall[k].poly, true);
     __syncthreads();
-    const uint32_t i = xcd_block_index() * kThreads + threadIdx.x;
+    const Lanes<S> lane(xcd_block_index());
+    const uint32_t i = lane.i;
     if (i >= a.n)
         return;
     const T threshold = T(0.75) * T(D);
@@ -1483,13 +1725,17 @@ __global__ void __launch_bounds__(kThreads) k_surface_div(FluidArgs<typename Pre
     };
     const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
     T pos_div = 0;
-    for_each_neighbor(a.slice, nb, nc,
-                      [&](uint32_t j) { pos_div -= term(load_pv<T, D>(a.posvol, j), poly_in, a.poly->x_per_r); });
+    for_each_neighbor<S>(a.slice, nb, nc, lane.sub,
+                         [&](uint32_t j) { pos_div -= term(load_pv<T, D>(a.posvol, j), poly_in, a.poly->x_per_r); });
+    if constexpr (S > 1)
+        pos_div = lane_sum<S>(pos_div);
     if (pos_div < threshold && a.prev_indicator[i] != 1)
     {
-        bool near_previous_surface = false;
-        for (uint32_t k = 0; k < nc; ++k)
-            near_previous_surface |= a.prev_indicator[a.slice[nb + (k << 6)]] == 1;
+        uint32_t near_previous_surface = 0;
+        for_each_neighbor<S>(a.slice, nb, nc, lane.sub,
+                             [&](uint32_t j) { near_previous_surface |= a.prev_indicator[j] == 1 ? 1u : 0u; });
+        if constexpr (S > 1)
+            near_previous_surface = lane_sum<S>(near_previous_surface);
         if (!near_previous_surface)
             pos_div = T(2) * threshold;
     }
@@ -1498,20 +1744,24 @@ __global__ void __launch_bounds__(kThreads) k_surface_div(FluidArgs<typename Pre
         const WallArgs<T> &w = a.wall[k];
         const uint32_t mb = w.chunk[i >> 6] + (i & 63u), mc = w.count[i];
         T wall_div = 0;
-        for (uint32_t k2 = 0; k2 < mc; ++k2)
+        for (uint32_t k2 = lane.sub; k2 < mc; k2 += S)
             wall_div -= term(load_pv<T, D>(w.posvol, w.slice[mb + (k2 << 6)]), poly_w[k], w.poly->x_per_r);
+        if constexpr (S > 1)
+            wall_div = lane_sum<S>(wall_div);
         pos_div += wall_div;
     }
-    a.pos_div[i] = pos_div;
+    if (lane.first())
+        a.pos_div[i] = pos_div;
 }
 
 // ... and the update: Indicator = 0 when the divergence exceeds the threshold and
 // no inner neighbour closer than h is below it, else 1; PreviousSurfaceIndicator = Indicator
-template <int D, int P>
+template <int D, int P, int S>
 __global__ void __launch_bounds__(kThreads) k_surface_update(FluidArgs<typename Prec<P>::T> a)
 {
     using T = typename Prec<P>::T;
-    const uint32_t i = xcd_block_index() * kThreads + threadIdx.x;
+    const Lanes<S> lane(xcd_block_index());
+    const uint32_t i = lane.i;
     if (i >= a.n)
         return;
     const T threshold = T(0.75) * T(D);
@@ -1519,16 +1769,20 @@ __global__ void __launch_bounds__(kThreads) k_surface_update(FluidArgs<typename 
     if (a.pos_div[i] > threshold)
     {
         const PV<T, D> pi = load_pv<T, D>(a.posvol, i);
-        bool very_near_surface = false;
-        for_each_neighbor(a.slice, a.chunk[i >> 6] + (i & 63u), a.count[i], [&](uint32_t j) {
+        uint32_t very_near_surface = 0;
+        for_each_neighbor<S>(a.slice, a.chunk[i >> 6] + (i & 63u), a.count[i], lane.sub, [&](uint32_t j) {
             const PV<T, D> pj = load_pv<T, D>(a.posvol, j);
             const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
             const T r = sqrt(D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy);
-            very_near_surface |= (a.pos_div[j] < threshold) & (r < a.h);
+            very_near_surface |= (a.pos_div[j] < threshold) & (r < a.h) ? 1u : 0u;
         });
+        if constexpr (S > 1)
+            very_near_surface = lane_sum<S>(very_near_surface);
         if (!very_near_surface)
             indicator = 0;
     }
+    if (!lane.first())
+        return;
     a.indicator[i] = indicator;
     a.prev_indicator[i] = indicator;
 }
@@ -1540,7 +1794,7 @@ __global__ void __launch_bounds__(kThreads) k_surface_update(FluidArgs<typename 
 //           + sum_w 2 mu (r.C_i e) 2 (v_i - v_w) / (r^2 + 0.01 h^2) dW V_w ],
 // C = 1 (CORR false) or the correction matrix; ForcePrior += F - F_previous.
 //---------------------------------------------------------------------------
-template <int D, int P, bool CORR>
+template <int D, int P, bool CORR, int S>
 __global__ void __launch_bounds__(kThreads) k_viscous(FluidArgs<typename Prec<P>::T> a, double mu_pair_d,
                                                       double mu_d, double h_sq_d)
 {
@@ -1551,7 +1805,8 @@ __global__ void __launch_bounds__(kThreads) k_viscous(FluidArgs<typename Prec<P>
     for (int k = 0; k < a.n_wall; ++k)
         stage_poly(poly_w[k], a.wall[k].poly, true);
     __syncthreads();
-    const uint32_t i = xcd_block_index() * kThreads + threadIdx.x;
+    const Lanes<S> lane(xcd_block_index());
+    const uint32_t i = lane.i;
     if (i >= a.n)
         return;
     const T mu_pair = T(mu_pair_d), mu = T(mu_d), eps = T(0.01) * T(h_sq_d);
@@ -1562,7 +1817,7 @@ __global__ void __launch_bounds__(kThreads) k_viscous(FluidArgs<typename Prec<P>
         Bi.load(a.corr, i);
     T fx = 0, fy = 0, fz = 0;
     const T x_per_r = a.poly->x_per_r;
-    for_each_neighbor(a.slice, a.chunk[i >> 6] + (i & 63u), a.count[i], [&](uint32_t j) {
+    for_each_neighbor<S>(a.slice, a.chunk[i >> 6] + (i & 63u), a.count[i], lane.sub, [&](uint32_t j) {
         const PV<T, D> pj = load_pv<T, D>(a.posvol, j);
         const Rec4<T> vj = a.vel[j];
         const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
@@ -1590,6 +1845,8 @@ __global__ void __launch_bounds__(kThreads) k_viscous(FluidArgs<typename Prec<P>
         if (D == 3)
             fz += c * (vi.z - vj.z);
     });
+    if constexpr (S > 1)
+        fx = lane_sum<S>(fx), fy = lane_sum<S>(fy), fz = lane_sum<S>(fz);
     const T vol_i = pi.vol;
     T Fx = fx * vol_i, Fy = fy * vol_i, Fz = fz * vol_i;
     for (int k = 0; k < a.n_wall; ++k)
@@ -1598,7 +1855,7 @@ __global__ void __launch_bounds__(kThreads) k_viscous(FluidArgs<typename Prec<P>
         const T w_x_per_r = w.poly->x_per_r;
         T wx = 0, wy = 0, wz = 0;
         const uint32_t mb = w.chunk[i >> 6] + (i & 63u), mc = w.count[i];
-        for (uint32_t k2 = 0; k2 < mc; ++k2)
+        for (uint32_t k2 = lane.sub; k2 < mc; k2 += S)
         {
             const uint32_t j = w.slice[mb + (k2 << 6)];
             const PV<T, D> pj = load_pv<T, D>(w.posvol, j);
@@ -1623,11 +1880,15 @@ __global__ void __launch_bounds__(kThreads) k_viscous(FluidArgs<typename Prec<P>
             if (D == 3)
                 wz += c * (T(2) * (vi.z - w.vel[2][j]));
         }
+        if constexpr (S > 1)
+            wx = lane_sum<S>(wx), wy = lane_sum<S>(wy), wz = lane_sum<S>(wz);
         Fx += wx * vol_i;
         Fy += wy * vol_i;
         if (D == 3)
             Fz += wz * vol_i;
     }
+    if (!lane.first())
+        return;
     // ForcePriorCK::UpdateKernel::update
     a.visc[0][i] = Fx;
     a.visc[1][i] = Fy;
@@ -1647,7 +1908,7 @@ __global__ void __launch_bounds__(kThreads) k_viscous(FluidArgs<typename Prec<P>
 // KernelGradientIntegral<Inner<K>> + <Contact<Boundary, K>> (kernel_gradient_integral.hpp:37-49,72-84):
 // g_i = -sum_j (C_i + C_j) dW V_j e_ij - sum_w 2 C_i dW V_w e_iw
 //---------------------------------------------------------------------------
-template <int D, int P, bool CORR>
+template <int D, int P, bool CORR, int S>
 __global__ void __launch_bounds__(kThreads) k_kernel_gradient_integral(FluidArgs<typename Prec<P>::T> a)
 {
     using T = typename Prec<P>::T;
@@ -1657,7 +1918,8 @@ __global__ void __launch_bounds__(kThreads) k_kernel_gradient_integral(FluidArgs
     for (int k = 0; k < a.n_wall; ++k)
         stage_poly(poly_w[k], a.wall[k].poly, true);
     __syncthreads();
-    const uint32_t i = xcd_block_index() * kThreads + threadIdx.x;
+    const Lanes<S> lane(xcd_block_index());
+    const uint32_t i = lane.i;
     if (i >= a.n)
         return;
     const PV<T, D> pi = load_pv<T, D>(a.posvol, i);
@@ -1666,7 +1928,7 @@ __global__ void __launch_bounds__(kThreads) k_kernel_gradient_integral(FluidArgs
         Bi.load(a.corr, i);
     T gx = 0, gy = 0, gz = 0;
     const T x_per_r = a.poly->x_per_r;
-    for_each_neighbor(a.slice, a.chunk[i >> 6] + (i & 63u), a.count[i], [&](uint32_t j) {
+    for_each_neighbor<S>(a.slice, a.chunk[i >> 6] + (i & 63u), a.count[i], lane.sub, [&](uint32_t j) {
         const PV<T, D> pj = load_pv<T, D>(a.posvol, j);
         const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
         const T r2 = D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy;
@@ -1700,7 +1962,7 @@ __global__ void __launch_bounds__(kThreads) k_kernel_gradient_integral(FluidArgs
         const T w_x_per_r = w.poly->x_per_r;
         T wx = 0, wy = 0, wz = 0;
         const uint32_t mb = w.chunk[i >> 6] + (i & 63u), mc = w.count[i];
-        for (uint32_t k2 = 0; k2 < mc; ++k2)
+        for (uint32_t k2 = lane.sub; k2 < mc; k2 += S)
         {
             const uint32_t j = w.slice[mb + (k2 << 6)];
             const PV<T, D> pj = load_pv<T, D>(w.posvol, j);
@@ -1721,6 +1983,10 @@ __global__ void __launch_bounds__(kThreads) k_kernel_gradient_integral(FluidArgs
         if (D == 3)
             gz += wz;
     }
+    if constexpr (S > 1)
+        gx = lane_sum<S>(gx), gy = lane_sum<S>(gy), gz = lane_sum<S>(gz);
+    if (!lane.first())
+        return;
     a.kgi[0][i] = gx;
     a.kgi[1][i] = gy;
     if (D == 3)
@@ -2024,38 +2290,49 @@ __global__ void k_fill_u64(unsigned long long *p, size_t n, unsigned long long v
 
 // Interpolation<Contact<Real>>::interact (interpolation_dynamics.hpp:46-60).
 // One wave per observer, its neighbours over the lanes: a program has a few
-// probes, so the time is the latency of one observer's list.  One thread walking
-// an observer's 80 neighbours took 44 us for the two probes of a 90k-particle 3D
-// tank; with a wave, five advection steps and their probes take 6.33 ms instead
-// of 6.55.
+// probes, so the time is the latency of one observer's list.  The lanes' kernels
+// and values go through LDS and every lane adds them in list order, so the sums
+// are those of one thread walking the list, which took 44 us for the two probes
+// of a 90k-particle 3D tank: five advection steps and their probes take 6.33 ms
+// instead of 6.55.
 template <int D, class T>
 __global__ void __launch_bounds__(64) k_interpolate(const Rec4<T> *obs, const Rec4<T> *tar, const T *data,
                                                     uint32_t stride, const uint32_t *chunk, const uint32_t *count,
                                                     const uint32_t *slice, const KernelPoly<T> *poly, T *out)
 {
-    const uint32_t i = blockIdx.x;
+    __shared__ T s_W[64], s_vol[64], s_value[64];
+    const uint32_t i = blockIdx.x, lane = threadIdx.x;
     const PV<T, D> pi = load_pv<T, D>(obs, i);
     T q = 0, w = 0;
     const uint32_t nb = chunk[i >> 6] + (i & 63u), nc = count[i];
-    for (uint32_t k = threadIdx.x; k < nc; k += 64u)
+    for (uint32_t k0 = 0; k0 < nc; k0 += 64u)
     {
-        const uint32_t j = slice[nb + (k << 6)];
-        const PV<T, D> pj = load_pv<T, D>(tar, j);
-        const T value = data[(size_t)j * stride];
-        const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
-        const T r2 = D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy;
-        const T x = sqrt(r2) * poly->x_per_r;
-        const int loc = min((int)x, kPolyIntervals - 1);
-        const T f = frac_part(x);
-        const T *c = poly->w[loc];
-        const T W = ((c[3] * f + c[2]) * f + c[1]) * f + c[0];
-        const T weight = W * pj.vol;
-        q += weight * value;
-        w += weight;
+        const uint32_t m = min(64u, nc - k0);
+        if (lane < m)
+        {
+            const uint32_t j = slice[nb + ((k0 + lane) << 6)];
+            const PV<T, D> pj = load_pv<T, D>(tar, j);
+            const T value = data[(size_t)j * stride];
+            const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
+            const T r2 = D == 3 ? dot3(dx, dx, dy, dy, dz, dz) : mad2(dx, dx, dy, dy);
+            const T x = sqrt(r2) * poly->x_per_r;
+            const int loc = min((int)x, kPolyIntervals - 1);
+            const T f = frac_part(x);
+            const T *c = poly->w[loc];
+            const T W = ((c[3] * f + c[2]) * f + c[1]) * f + c[0];
+            s_W[lane] = W;
+            s_vol[lane] = pj.vol;
+            s_value[lane] = value;
+        }
+        __syncthreads();
+        for (uint32_t k = 0; k < m; ++k)
+        {
+            q = fma(s_W[k] * s_vol[k], s_value[k], q);
+            w = fma(s_W[k], s_vol[k], w);
+        }
+        __syncthreads();
     }
-    q = lane_sum(q);
-    w = lane_sum(w);
-    if (threadIdx.x == 0)
+    if (lane == 0)
         out[i] = q / (w + T(2.71051e-20));
 }
 
@@ -2168,7 +2445,8 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(P
 kb_summation(const SceneArgs<typename Prec<P>::T> *__restrict__ tab, const uint32_t *__restrict__ map)
 {
     const uint32_t m = map[xcd_block_index()];
-    summation_body<D, P>(tab[map_scene(m)].f, map_block(m));
+    const FluidArgs<typename Prec<P>::T> &f = tab[map_scene(m)].f;
+    with_lanes<D, P>(f.n, [&](auto lanes) { summation_body<D, P, lanes.value>(f, map_block(m)); });
 }
 
 // DensityRegularization + AdvectionStepSetup, which touch each particle alone
@@ -2241,7 +2519,10 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(P
                                                      const uint32_t *__restrict__ map)
 {
     const uint32_t m = map[xcd_block_index()];
-    pass1_body<D, P, RIEMANN, true, false>(tab[map_scene(m)].f, map_block(m), 0.0);
+    const FluidArgs<typename Prec<P>::T> &f = tab[map_scene(m)].f;
+    with_lanes<D, P>(f.n, [&](auto lanes) {
+        pass1_body<D, P, RIEMANN, true, false, lanes.value>(f, map_block(m), 0.0);
+    });
 }
 
 template <int D, int P, bool RIEMANN>
@@ -2250,7 +2531,9 @@ kb_pass2(const SceneArgs<typename Prec<P>::T> *__restrict__ tab, const uint32_t 
 {
     const uint32_t m = map[xcd_block_index()];
     const SceneArgs<typename Prec<P>::T> &sa = tab[map_scene(m)];
-    pass2_body<D, P, RIEMANN, true, false>(sa.f, map_block(m), 0.0, sa.scalars + SLOT_MAX);
+    with_lanes<D, P>(sa.f.n, [&](auto lanes) {
+        pass2_body<D, P, RIEMANN, true, false, lanes.value>(sa.f, map_block(m), 0.0, sa.scalars + SLOT_MAX);
+    });
 }
 
 // after the captured sub-steps: gate[s] = 1 when scene s finished its loop
@@ -2523,9 +2806,12 @@ struct SummationL
         attach_relations(a, inner, c, nc);
         ProfileScope prof(b->ctx, "compression_summation");
         const size_t lds = a.stage_count ? sum_lds<D, P>() : 0;
-        allow_lds(k_summation<D, P>, lds);
-        hipLaunchKernelGGL((k_summation<D, P>), dim3(grid_for(b->n, kThreads)), dim3(kThreads), lds,
-                           b->ctx->stream, a);
+        with_lanes<D, P>(b->n, [&](auto lanes) {
+            constexpr int S = lanes.value;
+            allow_lds(k_summation<D, P, S>, lds);
+            hipLaunchKernelGGL((k_summation<D, P, S>), dim3(grid_for(b->n, kThreads / S)), dim3(kThreads), lds,
+                               b->ctx->stream, a);
+        });
         LAUNCH_CHECK();
         return SPHX_OK;
     }
@@ -2540,27 +2826,27 @@ sphx_status compression_summation(sphx_relation *inner, sphx_relation *const *c,
     do                                                                                                           \
     {                                                                                                            \
         if (B0 && B1 && B2)                                                                                      \
-            LAUNCH_PASS((K<D, P, true, true, true>), __VA_ARGS__);                                               \
+            LAUNCH_PASS((K<D, P, true, true, true, S>), __VA_ARGS__);                                            \
         else if (B0 && B1)                                                                                       \
-            LAUNCH_PASS((K<D, P, true, true, false>), __VA_ARGS__);                                              \
+            LAUNCH_PASS((K<D, P, true, true, false, S>), __VA_ARGS__);                                           \
         else if (B0 && B2)                                                                                       \
-            LAUNCH_PASS((K<D, P, true, false, true>), __VA_ARGS__);                                              \
+            LAUNCH_PASS((K<D, P, true, false, true, S>), __VA_ARGS__);                                           \
         else if (B0)                                                                                             \
-            LAUNCH_PASS((K<D, P, true, false, false>), __VA_ARGS__);                                             \
+            LAUNCH_PASS((K<D, P, true, false, false, S>), __VA_ARGS__);                                          \
         else if (B1 && B2)                                                                                       \
-            LAUNCH_PASS((K<D, P, false, true, true>), __VA_ARGS__);                                              \
+            LAUNCH_PASS((K<D, P, false, true, true, S>), __VA_ARGS__);                                           \
         else if (B1)                                                                                             \
-            LAUNCH_PASS((K<D, P, false, true, false>), __VA_ARGS__);                                             \
+            LAUNCH_PASS((K<D, P, false, true, false, S>), __VA_ARGS__);                                          \
         else if (B2)                                                                                             \
-            LAUNCH_PASS((K<D, P, false, false, true>), __VA_ARGS__);                                             \
+            LAUNCH_PASS((K<D, P, false, false, true, S>), __VA_ARGS__);                                          \
         else                                                                                                     \
-            LAUNCH_PASS((K<D, P, false, false, false>), __VA_ARGS__);                                            \
+            LAUNCH_PASS((K<D, P, false, false, false, S>), __VA_ARGS__);                                         \
     } while (0)
 #define LAUNCH_PASS(KERNEL, ...)                                                                                 \
     do                                                                                                           \
     {                                                                                                            \
         allow_lds(KERNEL, lds);                                                                                  \
-        hipLaunchKernelGGL(KERNEL, g, blk, lds, b->ctx->stream, __VA_ARGS__);                                   \
+        hipLaunchKernelGGL(KERNEL, gp, blk, lds, b->ctx->stream, __VA_ARGS__);                                  \
     } while (0)
 
 template <int D, int P>
@@ -2573,8 +2859,11 @@ struct CorrectionGradL
             return SPHX_OK;
         FluidArgs<T> a = fluid_args<T>(b);
         attach_relations(a, inner, nullptr, 0);
-        hipLaunchKernelGGL((k_correction_grad<D, P>), dim3(grid_for(b->n, kThreads)), dim3(kThreads), 0,
-                           b->ctx->stream, a);
+        with_tree_lanes<D, P>(b->n, [&](auto lanes) {
+            constexpr int S = lanes.value;
+            hipLaunchKernelGGL((k_correction_grad<D, P, S>), dim3(grid_for(b->n, kThreads / S)), dim3(kThreads), 0,
+                               b->ctx->stream, a);
+        });
         LAUNCH_CHECK();
         return SPHX_OK;
     }
@@ -2613,7 +2902,11 @@ struct Acoustic1L
         ProfileScope prof(b->ctx, "acoustic_pass1");
         const bool rs = riemann != SPHX_RIEMANN_NONE;
         const size_t lds = a.stage_count ? pass1_lds<D, P>() : 0;
-        SPHX_PASS_VARIANTS(k_pass1, rs, fuse_init_2nd, corr, a, dt);
+        with_lanes<D, P>(b->n, [&](auto lanes) {
+            constexpr int S = lanes.value;
+            const dim3 gp(grid_for(b->n, kThreads / S));
+            SPHX_PASS_VARIANTS(k_pass1, rs, fuse_init_2nd, corr, a, dt);
+        });
         LAUNCH_CHECK();
         return SPHX_OK;
     }
@@ -2641,7 +2934,11 @@ struct Acoustic2L
         const bool rs = riemann != SPHX_RIEMANN_NONE;
         const bool cfl = max_slot != nullptr;
         const size_t lds = a.stage_count ? pass2_lds<D, P>() : 0;
-        SPHX_PASS_VARIANTS(k_pass2, rs, cfl, corr, a, dt, max_slot);
+        with_lanes<D, P>(b->n, [&](auto lanes) {
+            constexpr int S = lanes.value;
+            const dim3 gp(grid_for(b->n, kThreads / S));
+            SPHX_PASS_VARIANTS(k_pass2, rs, cfl, corr, a, dt, max_slot);
+        });
         LAUNCH_CHECK();
         return SPHX_OK;
     }
@@ -2736,9 +3033,12 @@ struct CorrectionL
         FluidArgs<T> a = fluid_args<T>(b);
         attach_relations(a, inner, c, nc);
         const size_t lds = a.stage_count ? sum_lds<D, P>() : 0;
-        allow_lds(k_correction<D, P>, lds);
-        hipLaunchKernelGGL((k_correction<D, P>), dim3(grid_for(b->n, kThreads)), dim3(kThreads), lds,
-                           b->ctx->stream, a, alpha);
+        with_tree_lanes<D, P>(b->n, [&](auto lanes) {
+            constexpr int S = lanes.value;
+            allow_lds(k_correction<D, P, S>, lds);
+            hipLaunchKernelGGL((k_correction<D, P, S>), dim3(grid_for(b->n, kThreads / S)), dim3(kThreads), lds,
+                               b->ctx->stream, a, alpha);
+        });
         LAUNCH_CHECK();
         return SPHX_OK;
     }
@@ -2769,11 +3069,14 @@ struct ViscousL
         // Viscosity::getInterParticleViscosity: PairGeomAverageFixed(mu, mu), particle_functors.h:169-170
         const double mu_pair = 2.0 * mu * mu * (1.0 / (mu + mu));
         const double h_sq = std::pow(b->h, 2.0);
-        dim3 g(grid_for(b->n, kThreads)), blk(kThreads);
-        if (corr)
-            hipLaunchKernelGGL((k_viscous<D, P, true>), g, blk, 0, b->ctx->stream, a, mu_pair, mu, h_sq);
-        else
-            hipLaunchKernelGGL((k_viscous<D, P, false>), g, blk, 0, b->ctx->stream, a, mu_pair, mu, h_sq);
+        with_tree_lanes<D, P>(b->n, [&](auto lanes) {
+            constexpr int S = lanes.value;
+            const dim3 g(grid_for(b->n, kThreads / S)), blk(kThreads);
+            if (corr)
+                hipLaunchKernelGGL((k_viscous<D, P, true, S>), g, blk, 0, b->ctx->stream, a, mu_pair, mu, h_sq);
+            else
+                hipLaunchKernelGGL((k_viscous<D, P, false, S>), g, blk, 0, b->ctx->stream, a, mu_pair, mu, h_sq);
+        });
         LAUNCH_CHECK();
         return SPHX_OK;
     }
@@ -2795,11 +3098,14 @@ struct KgiL
             return SPHX_OK;
         FluidArgs<T> a = fluid_args<T>(b);
         attach_relations(a, inner, c, nc);
-        dim3 g(grid_for(b->n, kThreads)), blk(kThreads);
-        if (corr)
-            hipLaunchKernelGGL((k_kernel_gradient_integral<D, P, true>), g, blk, 0, b->ctx->stream, a);
-        else
-            hipLaunchKernelGGL((k_kernel_gradient_integral<D, P, false>), g, blk, 0, b->ctx->stream, a);
+        with_tree_lanes<D, P>(b->n, [&](auto lanes) {
+            constexpr int S = lanes.value;
+            const dim3 g(grid_for(b->n, kThreads / S)), blk(kThreads);
+            if (corr)
+                hipLaunchKernelGGL((k_kernel_gradient_integral<D, P, true, S>), g, blk, 0, b->ctx->stream, a);
+            else
+                hipLaunchKernelGGL((k_kernel_gradient_integral<D, P, false, S>), g, blk, 0, b->ctx->stream, a);
+        });
         LAUNCH_CHECK();
         return SPHX_OK;
     }
@@ -2844,9 +3150,12 @@ struct SurfaceL
             return SPHX_OK;
         FluidArgs<T> a = fluid_args<T>(b);
         attach_relations(a, inner, c, nc);
-        dim3 g(grid_for(b->n, kThreads)), blk(kThreads);
-        hipLaunchKernelGGL((k_surface_div<D, P>), g, blk, 0, b->ctx->stream, a);
-        hipLaunchKernelGGL((k_surface_update<D, P>), g, blk, 0, b->ctx->stream, a);
+        with_tree_lanes<D, P>(b->n, [&](auto lanes) {
+            constexpr int S = lanes.value;
+            const dim3 g(grid_for(b->n, kThreads / S)), blk(kThreads);
+            hipLaunchKernelGGL((k_surface_div<D, P, S>), g, blk, 0, b->ctx->stream, a);
+            hipLaunchKernelGGL((k_surface_update<D, P, S>), g, blk, 0, b->ctx->stream, a);
+        });
         LAUNCH_CHECK();
         return SPHX_OK;
     }
@@ -3129,7 +3438,7 @@ struct BatchL
     {
         const dim3 g(b.blocks), blk(kThreads), gs(grid_for(b.n_scenes, 64)), bs(64);
         allow_lds(kb_summation<D, P>, lds_sum(b));
-        hipLaunchKernelGGL((kb_summation<D, P>), g, blk, lds_sum(b), b.stream, tab(b), b.map);
+        hipLaunchKernelGGL((kb_summation<D, P>), dim3(b.blocks_sums), blk, lds_sum(b), b.stream, tab(b), b.map_sums);
         hipLaunchKernelGGL((kb_regularize_setup<D, P>), g, blk, 0, b.stream, tab(b), b.map);
         hipLaunchKernelGGL((kb_reset_lanes<T>), dim3(b.n_scenes), dim3(64), 0, b.stream, tab(b), b.n_scenes);
         hipLaunchKernelGGL((kb_speed_max<D, P>), g, blk, 0, b.stream, tab(b), b.map);
@@ -3145,8 +3454,8 @@ struct BatchL
         allow_lds(kb_pass2<D, P, RIEMANN>, lds_pass2(b));
         hipLaunchKernelGGL((kb_substep_begin<T>), gs, bs, 0, b.stream, tab(b), b.n_scenes);
         hipLaunchKernelGGL((kb_init_1st<D, P>), g, blk, 0, b.stream, tab(b), b.map);
-        hipLaunchKernelGGL((kb_pass1<D, P, RIEMANN>), g, blk, lds_pass1(b), b.stream, tab(b), b.map);
-        hipLaunchKernelGGL((kb_pass2<D, P, RIEMANN>), g, blk, lds_pass2(b), b.stream, tab(b), b.map);
+        hipLaunchKernelGGL((kb_pass1<D, P, RIEMANN>), dim3(b.blocks_sums), blk, lds_pass1(b), b.stream, tab(b), b.map_sums);
+        hipLaunchKernelGGL((kb_pass2<D, P, RIEMANN>), dim3(b.blocks_sums), blk, lds_pass2(b), b.stream, tab(b), b.map_sums);
         SPHX_HIP(hipGetLastError());
         return SPHX_OK;
     }

@@ -1163,7 +1163,7 @@ static sphx_status relation_create(sphx_body *src, sphx_body *tar, sphx_cell_lin
             return st;
     }
     SPHX_HIP(hipMemsetAsync(r->neighbor_size, 0, (size_t)(src->n + 1) * sizeof(uint32_t), src->ctx->stream));
-    if (inner && src->desc.kind == SPHX_BODY_FLUID && src->n >= (src->P == P_FP64 ? kStageMin64 : 1u))
+    if (inner && src->desc.kind == SPHX_BODY_FLUID && src->n > 0 && split_lanes(src->D, src->P, src->n) == 1)
     {
         // LDS staging of the acoustic passes and the sums over the inner neighbours
         const size_t nblocks = (src->n + kStageBlock - 1) / kStageBlock;

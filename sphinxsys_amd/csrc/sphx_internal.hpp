@@ -46,11 +46,23 @@ constexpr size_t kSmallTransfer = 256u << 10; // field transfers up to this size
 constexpr uint32_t kStageBlock = 256;          // source particles per staging block
 constexpr uint32_t kStageOverflow = 0xffffffffu;
 constexpr uint32_t kStageCap = 1536;           // distinct neighbours staged per block (LDS records)
-// FP64 fluid bodies of at least this many particles stage their inner
-// neighbours.  Below, the sets cost what they save or more (per advection step
-// in 3D: 8,000 particles 45 us for the sets, 51 us less in the passes; 800 in 2D
-// 19 against 6; above, 90,000: 67 against 185)
-constexpr uint32_t kStageMin64 = 16384;
+// Lanes per particle of a fluid body's neighbour sums: several for a body whose
+// wavefronts would not fill the GPU (1,024 SIMDs); such a body is not staged.
+// The passes of a small body are the latency of one thread's list: 800
+// particles in 2D 14 + 16 us with one lane, 9 + 10 with four; 8,000 in 3D
+// corrected 40 + 52 with one, 16 + 20 with four, 12 + 15 with eight; 90,000 51 +
+// 65 with eight, 45 + 58 with four, 58 + 67 staged with one.  The upper lines lie
+// where the whole step is as fast with one lane and staging (FP64: 134,000
+// particles in 3D 1,011 us with four, 1,058 with one; 214,000 1,400 and 1,361;
+// 125,000 in 2D 431 and 423).  One lane in FP32-mixed 3D, whose second half step
+// equals its cell traversal bit for bit.
+constexpr uint32_t kSplitFew3D = 16384, kSplit3D = 163840, kSplit2D = 131072;
+constexpr int split_lanes(int D, int P, uint32_t n)
+{
+    if (D == 2)
+        return n < kSplit2D ? 4 : 1;
+    return P != P_FP64 ? 1 : n < kSplitFew3D ? 8 : n < kSplit3D ? 4 : 1;
+}
 // reported through the relation build's `needed` slot when a search box holds
 // more candidates than the tiled build's masks: rebuild with the scan kernel
 constexpr unsigned long long kTooDense = 1ull << 40;
@@ -297,6 +309,8 @@ struct BatchFluid
     uint32_t n_scenes = 0;
     const uint32_t *map = nullptr;
     uint32_t blocks = 0;
+    const uint32_t *map_sums = nullptr; // as map for the neighbour sums: 256 / split_lanes particles a block
+    uint32_t blocks_sums = 0;
     uint32_t stage_cap = 0;            // staging capacity of the staged scenes (0: none staged)
     const uint32_t *tail_on = nullptr; // per scene: the device runs the step's tail
     uint32_t *gate = nullptr;          // per scene: sub-steps done and tail on (written by the gate)

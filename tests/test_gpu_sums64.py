@@ -1,5 +1,6 @@
-"""The FP64 sums over LDS-staged neighbour records against the oracle: sizes on
-both sides of the smallest staged body, a last block of a few particles, and
+"""The FP64 neighbour sums against the oracle at the sizes where their form
+changes (eight, four and one lanes per particle, the last from LDS-staged
+records), bodies of less than a wave, last blocks of a few particles, and
 shuffled orders, whose blocks have more distinct neighbours than the kernels
 stage (some of them in a window of 1024, all of them in a full shuffle) and
 read from global memory.
@@ -16,8 +17,9 @@ from tests.test_gpu_parity import FP64_GATE, Pair, jittered_lattice, rel_l2, shu
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("dim,m,window", [(2, 127, None), (2, 129, None), (2, 129, 0), (3, 25, None), (3, 26, None),
-                                          (3, 26, 1024), (3, 26, 0)])
+@pytest.mark.parametrize("dim,m,window", [(2, 7, None), (2, 362, None), (2, 363, None), (2, 363, 0),
+                                          (3, 5, None), (3, 25, None), (3, 26, None), (3, 54, None),
+                                          (3, 55, None), (3, 55, 1024), (3, 55, 0)])
 def test_fp64_sums_staged_and_not(hip, oracle, dim, m, window):
     dp = 0.02
     fluid = jittered_lattice(dim, m, dp, 3)
@@ -48,7 +50,7 @@ def test_fp64_sums_staged_and_not(hip, oracle, dim, m, window):
 def test_lists_rebuilt_between_batch_steps(hip, precision):
     """A caller that rebuilds a scene's lists between two batch steps leaves their
     staging sets to the next reader: the batched scene still equals itself alone."""
-    geom = cases.dambreak_2d(dp=0.01)  # 20,000 particles: staged in both precisions
+    geom = cases.dambreak_2d(dp=0.0038)  # 138,000 particles: staged in both precisions
     alone, batched = (cases.DamBreak(hip, geom, precision) for _ in range(2))
     for sc in (alone, batched):
         sc.initialize()
