@@ -620,20 +620,26 @@ __device__ __forceinline__ uint32_t pick(const uint32_t (&v)[R], uint32_t idx)
     return out;
 }
 
-template <int D, int W>
+// With V waves per chunk (W = 1) each wave tests an equal range of the chunk's
+// sources and then writes an equal range of the slice rows: for bodies whose
+// chunks alone would not fill the GPU (tile_split), where the build is the time
+// one wave takes for its 64 sources.
+template <int D, int W, int V = 1>
 __device__ __forceinline__ void relation_tile_body(const BuildArgs &b, const uint32_t blk)
 {
+    static_assert(W == 1 || V == 1, "several chunks or several waves of a chunk per workgroup");
     constexpr int R = D == 3 ? 9 : 3; // cell rows of the search box, l -> m order
     constexpr int QMAX = 8;           // candidates of a cell kept in registers: 64 * QMAX
     const RelationArgs &a = b.r;
     __shared__ unsigned long long masks[W][64][kMaskSlots];
     __shared__ uint32_t any_dense;
     const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63u;
-    const uint32_t chunk = blk * W + wave;
+    const uint32_t part = V > 1 ? wave : 0u; // of the chunk
+    const uint32_t chunk = V > 1 ? blk : blk * W + wave;
     const uint32_t i = chunk * 64u + lane;
     const bool valid = i < a.n_src;
     const uint32_t kmax = b.kmax;
-    unsigned long long(&my_masks)[64][kMaskSlots] = masks[wave];
+    unsigned long long(&my_masks)[64][kMaskSlots] = masks[V > 1 ? 0u : wave];
     if (t == 0)
         any_dense = 0;
     __syncthreads();
@@ -727,6 +733,8 @@ __device__ __forceinline__ void relation_tile_body(const BuildArgs &b, const uin
     // share its candidates), so a particle that left its cell's run since the
     // last sort does not make the wave reload the candidates
     unsigned long long todo = __ballot(my_total > 0u);
+    if (V > 1)
+        todo &= (~0ull >> (64 - 64 / V)) << (part * (64u / V));
     unsigned long long group = 0ull; // sources of the current cell not yet done
     while (todo)
     {
@@ -876,12 +884,14 @@ __device__ __forceinline__ void relation_tile_body(const BuildArgs &b, const uin
             }
         }
     }
+    if (V > 1)
+        __syncthreads(); // every wave's masks
     // each lane counts its own neighbours from its masks (a source's
     // candidate list is its cell's: my_total entries)
     for (uint32_t q = 0; q < (my_total + 63u) >> 6; ++q)
         my_count += (uint32_t)__popcll(my_masks[lane][q]);
     const uint32_t mine = valid ? min(my_count, kmax) : 0u;
-    if (valid)
+    if (valid && part == 0u)
     {
         a.neighbor_size[i] = mine;
         if (my_count > kmax)
@@ -903,11 +913,27 @@ __device__ __forceinline__ void relation_tile_body(const BuildArgs &b, const uin
         }
     }
     const size_t row0 = (size_t)chunk * kmax * 64u + lane;
-    const uint32_t rows = wave_max_u32(mine);
+    const uint32_t all_rows = wave_max_u32(mine);
+    constexpr uint32_t kOutBatch = 8; // index gathers in flight per lane
+    // this wave's rows: all, or a V-th of them in whole batches
+    const uint32_t share = V > 1 ? (all_rows + V * kOutBatch - 1u) / (V * kOutBatch) * kOutBatch : all_rows;
+    const uint32_t row_first = V > 1 ? part * share : 0u;
+    const uint32_t rows = V > 1 ? min(all_rows, row_first + share) : all_rows;
     uint32_t cur_q = 0;
     unsigned long long cur = mine > 0u ? my_masks[lane][0] : 0ull;
-    constexpr uint32_t kOutBatch = 8; // index gathers in flight per lane
-    for (uint32_t r0 = 0; r0 < rows; r0 += kOutBatch)
+    if (V > 1 && row_first < mine)
+    {
+        // the mask with the wave's first neighbour, without the neighbours before it
+        uint32_t skip = row_first;
+        for (uint32_t c2 = (uint32_t)__popcll(cur); skip >= c2; c2 = (uint32_t)__popcll(cur))
+        {
+            skip -= c2;
+            cur = my_masks[lane][++cur_q]; // mine bounds the walk
+        }
+        for (; skip > 0u; --skip)
+            cur &= cur - 1ull;
+    }
+    for (uint32_t r0 = row_first; r0 < rows; r0 += kOutBatch)
     {
         uint32_t jj[kOutBatch];
 #pragma unroll
@@ -935,11 +961,19 @@ __device__ __forceinline__ void relation_tile_body(const BuildArgs &b, const uin
     }
 }
 
-template <int D>
-__global__ void __launch_bounds__(kTileWaves * 64) k_relation_tile(BuildArgs b)
+template <int D, int V>
+__global__ void __launch_bounds__(kTileWaves * V * 64) k_relation_tile(BuildArgs b)
 {
-    relation_tile_body<D, kTileWaves>(b, xcd_block_index());
+    relation_tile_body<D, kTileWaves, V>(b, xcd_block_index());
 }
+// Waves per chunk of a build of nchunks chunks.  Inner build and wall contact,
+// one wave / four: 800 particles in 2D 41 + 24 / 18 + 14 us, 8,000 in 3D 88 + 54 /
+// 47 + 26, 90,000 133 + 68 / 92 + 39, 195,000 149 + 76 / 144 + 59, 415,000 226 +
+// 85 / 280 + 91 (each wave loads the candidates of its cells itself; eight waves
+// are slower from 90,000 on)
+constexpr int kTileSplit = 4;
+constexpr uint32_t kTileSplitBelow = 4096;
+inline bool tile_split(uint32_t nchunks) { return nchunks < kTileSplitBelow; }
 
 //---------------------------------------------------------------------------
 // staging sets of the inner fluid relation, from its finished slices: for each
@@ -1334,8 +1368,8 @@ __global__ void kb_zero_u64(unsigned long long *p, uint32_t n)
         p[i] = 0ull;
 }
 
-template <int D, int W>
-__global__ void __launch_bounds__(W * 64) kb_relation_tile(const BuildArgs *__restrict__ tab,
+template <int D, int W, int V = 1>
+__global__ void __launch_bounds__(W * V * 64) kb_relation_tile(const BuildArgs *__restrict__ tab,
                                                            const uint32_t *__restrict__ map,
                                                            const uint32_t *__restrict__ rel_scene,
                                                            const uint32_t *__restrict__ gate)
@@ -1343,7 +1377,7 @@ __global__ void __launch_bounds__(W * 64) kb_relation_tile(const BuildArgs *__re
     const uint32_t m = map[xcd_block_index()], r = bmap_owner(m);
     if (!gate[rel_scene[r]])
         return;
-    relation_tile_body<D, W>(tab[r], bmap_block(m));
+    relation_tile_body<D, W, V>(tab[r], bmap_block(m));
 }
 
 __global__ void __launch_bounds__(kThreads) kb_stage_sets(const StageArgs *__restrict__ tab,
@@ -1676,8 +1710,11 @@ sphx_status relation_to_csr(sphx_relation *rel)
 template <int D>
 static sphx_status launch_tile(sphx_context *ctx, const BuildArgs &b, uint32_t nchunks)
 {
-    hipLaunchKernelGGL((k_relation_tile<D>), dim3(grid_for(nchunks, kTileWaves)), dim3(kTileWaves * 64), 0, ctx->stream,
-                       b);
+    if (tile_split(nchunks))
+        hipLaunchKernelGGL((k_relation_tile<D, kTileSplit>), dim3(nchunks), dim3(kTileSplit * 64), 0, ctx->stream, b);
+    else
+        hipLaunchKernelGGL((k_relation_tile<D, 1>), dim3(grid_for(nchunks, kTileWaves)), dim3(kTileWaves * 64), 0,
+                           ctx->stream, b);
     SPHX_HIP(hipGetLastError());
     return SPHX_OK;
 }
@@ -1908,7 +1945,17 @@ sphx_status batch_relations(const BatchConfig &b)
         set_error("tiled relation build: 1, 2 or 4 waves per workgroup");
         return SPHX_E_ARG;
     }
-    if (b.D == 2)
+    if (b.split_chunks && tile_split(b.blocks_single))
+    {
+        const dim3 g(b.blocks_single), blk(kTileSplit * 64);
+        if (b.D == 2)
+            hipLaunchKernelGGL((kb_relation_tile<2, 1, kTileSplit>), g, blk, 0, b.stream, (const BuildArgs *)b.build,
+                               b.split_chunks, b.rel_scene, b.gate);
+        else
+            hipLaunchKernelGGL((kb_relation_tile<3, 1, kTileSplit>), g, blk, 0, b.stream, (const BuildArgs *)b.build,
+                               b.split_chunks, b.rel_scene, b.gate);
+    }
+    else if (b.D == 2)
         w == 1 ? launch_batch_tile<2, 1>(b) : w == 2 ? launch_batch_tile<2, 2>(b) : launch_batch_tile<2, 4>(b);
     else
         w == 1 ? launch_batch_tile<3, 1>(b) : w == 2 ? launch_batch_tile<3, 2>(b) : launch_batch_tile<3, 4>(b);
