@@ -78,6 +78,7 @@ struct sphx_batch
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     uint32_t graph_substeps = 0;
+    uint32_t launched = 0; // sub-steps of the last step's launches
     Shape graph_shape;
     bool graph_valid = false;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -310,6 +311,16 @@ BatchConfig config_launch(sphx_batch *b)
     c.stream = b->stream;
     c.gate = b->gate;
     c.cll = b->cll_tab;
+    for (const auto &sc : b->scenes)
+    {
+        const size_t lds = batch_cll_small(sc.cll);
+        if (!lds)
+        {
+            c.small_lds = 0;
+            break;
+        }
+        c.small_lds = std::max(c.small_lds, lds);
+    }
     c.n_scenes = (uint32_t)b->scenes.size();
     c.map_particles = b->map256;
     c.blocks_particles = b->blocks256;
@@ -335,12 +346,12 @@ BatchConfig config_launch(sphx_batch *b)
 }
 
 // the launches of the step's tail: position update, cell lists, relations
-sphx_status enqueue_tail(sphx_batch *b)
+sphx_status enqueue_tail(sphx_batch *b, uint32_t substeps)
 {
     sphx_status s;
     const BatchFluid f = fluid_launch(b);
     const BatchConfig c = config_launch(b);
-    if ((s = batch_step_gate(f)) || (s = batch_position(f)) || (s = batch_cell_linked_list(c)) ||
+    if ((s = batch_step_gate(f, substeps)) || (s = batch_position(f)) || (s = batch_cell_linked_list(c)) ||
         (s = batch_relations(c)))
         return s;
     return SPHX_OK;
@@ -352,8 +363,8 @@ sphx_status enqueue_step(sphx_batch *b, uint32_t substeps)
     const BatchFluid f = fluid_launch(b);
     sphx_status s = batch_step_head(f);
     for (uint32_t k = 0; k < substeps && !s; ++k)
-        s = batch_substep(f);
-    return s ? s : enqueue_tail(b);
+        s = batch_substep(f, k);
+    return s ? s : enqueue_tail(b, substeps);
 }
 
 sphx_status read_back(sphx_batch *b, bool with_needed)
@@ -384,15 +395,15 @@ sphx_status run_direct(sphx_batch *b)
     const BatchFluid f = fluid_launch(b);
     if ((s = batch_step_head(f)))
         return s;
-    uint32_t batch = 1;
+    uint32_t batch = 1, done = 0;
     for (const auto &sc : b->scenes)
         batch = std::max(batch, sc.last);
     while (true)
     {
         for (uint32_t k = 0; k < batch; ++k)
-            if ((s = batch_substep(f)))
+            if ((s = batch_substep(f, done++)))
                 return s;
-        if ((s = batch_step_gate(f)) || (s = read_back(b, false)))
+        if ((s = batch_step_gate(f, done)) || (s = read_back(b, false)))
             return s;
         bool all = true;
         for (size_t i = 0; i < b->scenes.size() && all; ++i)
@@ -401,7 +412,8 @@ sphx_status run_direct(sphx_batch *b)
             break;
         batch = 1;
     }
-    if ((s = enqueue_tail(b)) || (s = read_back(b, true)))
+    b->launched = done;
+    if ((s = enqueue_tail(b, done)) || (s = read_back(b, true)))
         return s;
     b->direct_steps++;
     return SPHX_OK;
@@ -446,6 +458,7 @@ sphx_status run_graph(sphx_batch *b, uint32_t substeps, float *ms)
     if ((s = read_back(b, true)))
         return s;
     SPHX_HIP(hipEventElapsedTime(ms, b->ev0, b->ev1));
+    b->launched = substeps;
     b->graph_launches++;
     return SPHX_OK;
 }
@@ -744,8 +757,7 @@ sphx_status sphx_batch_advection_step(sphx_batch *b, double *time, uint32_t *ste
         {
             // more sub-steps than captured: the single-scene loop goes on from the device state
             body->state_version++;
-            std::memcpy(ctx->scalars_h + SLOT_STEP, st, STEP_SLOTS * sizeof(unsigned long long));
-            if ((s = advection_substeps(sc.inner, sc.walls, sc.n_wall, &sc.cfg, 1u)))
+            if ((s = advection_substeps(sc.inner, sc.walls, sc.n_wall, &sc.cfg, time[i], b->launched, 1u, &st)))
             {
                 if (s != SPHX_E_NONFINITE)
                     return s;
@@ -757,7 +769,6 @@ sphx_status sphx_batch_advection_step(sphx_batch *b, double *time, uint32_t *ste
             b->host_substep_scenes++;
             b->host_tail_scenes++;
             regrown = true; // relations may have been regrown; the records are refreshed
-            st = ctx->scalars_h + SLOT_STEP;
         }
         else if (!b->tail_on_h[i])
         {

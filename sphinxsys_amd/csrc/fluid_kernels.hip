@@ -16,6 +16,7 @@
 // density_regularization.hpp:40-118, fluid_time_step_ck.{h,hpp,cpp}.
 #include "sphx_internal.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -105,8 +106,9 @@ struct FluidArgs
     // device-side sub-step control (null: dt is the kernel argument): the
     // acoustic kernels return at once when STEP_ACTIVE is 0 and take STEP_DT
     const unsigned long long *step;
-    // max lanes of the time-step reductions (batched launches: each scene's own)
-    unsigned long long *lanes;
+    int in_loop; // within the device-side loop
+    // the context's scalar slots, whose max lanes the summation clears (null: it does not)
+    unsigned long long *reset_lanes;
 };
 
 // dt of an acoustic kernel: the argument, or the device-side sub-step's; false
@@ -534,12 +536,9 @@ __device__ __forceinline__ uint32_t split_count(uint32_t count, uint32_t sub)
 // AcousticStep1stHalf::InitializeKernel (acoustic_step_1st_half.hpp:66-74)
 //---------------------------------------------------------------------------
 template <int D, int P>
-__device__ __forceinline__ void init_1st_body(const FluidArgs<typename Prec<P>::T> &a, uint32_t blk, double dt_d)
+__device__ __forceinline__ void init_1st_body(const FluidArgs<typename Prec<P>::T> &a, uint32_t i, double dt_d)
 {
     using T = typename Prec<P>::T;
-    uint32_t i = blk * kThreads + threadIdx.x;
-    if (i >= a.n || !step_dt(a, dt_d))
-        return;
     const T dt = T(dt_d);
     T c = a.C[i] + T(0.5) * dt * a.dC[i];
     a.C[i] = c;
@@ -552,7 +551,111 @@ __device__ __forceinline__ void init_1st_body(const FluidArgs<typename Prec<P>::
 template <int D, int P>
 __global__ void __launch_bounds__(kThreads) k_init_1st(FluidArgs<typename Prec<P>::T> a, double dt_d)
 {
-    init_1st_body<D, P>(a, blockIdx.x, dt_d);
+    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+    if (i < a.n)
+        init_1st_body<D, P>(a, i, dt_d);
+}
+
+//---------------------------------------------------------------------------
+// the same at the start of a sub-step of the device-side dual-time loop of
+// sphx_advection_step (dambreak.cpp:188-207): AdvectionTimeStepCK's dt from the
+// speed max (first sub-step), AcousticTimeStepCK's dt from the signal max and the
+// loop condition relaxation < advection dt, with the host's arithmetic in
+// double, in every block; the first block stores the state
+//---------------------------------------------------------------------------
+// the max of the accumulator lanes, taken by the lanes of a wave
+__device__ __forceinline__ double lanes_max(const unsigned long long *lanes)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    return wave_max(lane < (unsigned)kMaxLanes ? from_ordered_bits(lanes[lane * kMaxStride]) : -1.79769313486231570e308);
+}
+__device__ __forceinline__ void put_double(unsigned long long *slot, double v)
+{
+    *slot = (unsigned long long)__double_as_longlong(v);
+}
+__device__ __forceinline__ double get_double(const unsigned long long *slot)
+{
+    return __longlong_as_double((long long)*slot);
+}
+
+template <int D, int P>
+__device__ __forceinline__ void begin_init_body(const FluidArgs<typename Prec<P>::T> &a, const StepBegin &sb,
+                                                const uint32_t blk, const uint32_t stride)
+{
+    __shared__ double s_dt;
+    __shared__ uint32_t s_active;
+    if (threadIdx.x < 64u)
+    {
+        const unsigned long long *in = sb.scalars + step_slot(sb.parity);
+        const double signal = lanes_max(sb.scalars + signal_slot(sb.parity));
+        double adv_dt, dt = 0.0, relaxation = 0.0, time = sb.time;
+        unsigned long long count = 0, error;
+        if (sb.first)
+        {
+            // AdvectionTimeStepCK::FinishDynamics::Result, fluid_time_step_ck.cpp:23-26
+            const double m = lanes_max(sb.scalars + SLOT_SPEED);
+            adv_dt = sb.advection_cfl * sb.h / (fmax(sqrt(m), sb.u_ref) + 2.71051e-20);
+            // a non-finite velocity made the speed max +inf and the step zero
+            error = isfinite(adv_dt) && adv_dt > 0.0 ? 0ull : 1ull;
+        }
+        else
+        {
+            adv_dt = get_double(in + STEP_ADV_DT);
+            dt = get_double(in + STEP_DT);
+            relaxation = get_double(in + STEP_RELAXATION);
+            time = get_double(in + STEP_TIME);
+            count = in[STEP_COUNT];
+            error = in[STEP_ERROR];
+        }
+        bool active = error == 0 && relaxation < adv_dt;
+        if (active)
+        {
+            // AcousticTimeStepCK::FinishDynamics::Result, fluid_time_step_ck.hpp:30-57
+            const double next = sb.acoustic_cfl * sb.h / (signal + 2.71051e-20);
+            active = isfinite(next) && next > 0.0;
+            if (active)
+            {
+                dt = next;
+                relaxation += dt;
+                time += dt;
+                ++count;
+            }
+            else
+                error = 1;
+        }
+        if (threadIdx.x == 0)
+        {
+            s_dt = dt;
+            s_active = active ? 1u : 0u;
+        }
+        if (blk == 0u)
+        {
+            // the lanes that this sub-step's second pass fills
+            if (threadIdx.x < (unsigned)kMaxLanes)
+                sb.scalars[signal_slot(sb.parity ^ 1u) + threadIdx.x * kMaxStride] = kOrderedLowest;
+            unsigned long long *out = sb.scalars + step_slot(sb.parity ^ 1u);
+            if (threadIdx.x == 0)
+            {
+                put_double(out + STEP_ADV_DT, adv_dt);
+                put_double(out + STEP_DT, dt);
+                put_double(out + STEP_RELAXATION, relaxation);
+                put_double(out + STEP_TIME, time);
+                out[STEP_COUNT] = count;
+                out[STEP_ACTIVE] = active ? 1ull : 0ull;
+                out[STEP_ERROR] = error;
+            }
+        }
+    }
+    __syncthreads();
+    if (s_active)
+        for (uint32_t i = blk * kThreads + threadIdx.x; i < a.n; i += stride)
+            init_1st_body<D, P>(a, i, s_dt);
+}
+
+template <int D, int P>
+__global__ void __launch_bounds__(kThreads) k_begin_init(FluidArgs<typename Prec<P>::T> a, StepBegin sb)
+{
+    begin_init_body<D, P>(a, sb, blockIdx.x, gridDim.x * kThreads);
 }
 
 //---------------------------------------------------------------------------
@@ -916,7 +1019,7 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
     // inside the device-side sub-step loop the 2nd half, which sets the force
     // anew, runs next whenever this pass runs and nothing reads the force in
     // between: the store is left out there
-    if (!a.step)
+    if (!a.in_loop)
     {
         a.force[0][i] = Fx;
         a.force[1][i] = Fy;
@@ -1427,6 +1530,9 @@ __device__ __forceinline__ void summation_body(const FluidArgs<typename Prec<P>:
     __shared__ PolyLDS<T> poly_in;
     __shared__ PolyLDS<T> poly_w[kMaxWalls];
     extern __shared__ __align__(32) unsigned char staged_lds[];
+    if (a.reset_lanes && blk == 0u && threadIdx.x < 2u * kMaxLanes)
+        a.reset_lanes[(threadIdx.x < (unsigned)kMaxLanes ? SLOT_MAX : SLOT_SPEED) + threadIdx.x % kMaxLanes * kMaxStride] =
+            kOrderedLowest;
     stage_poly(poly_in, a.poly, false);
     for (int k = 0; k < a.n_wall; ++k)
         stage_poly(poly_w[k], a.wall[k].poly, false);
@@ -2173,54 +2279,80 @@ __device__ __forceinline__ void block_max_to(double v, unsigned long long *slot)
 }
 
 template <int D, int P>
-__device__ __forceinline__ void signal_body(const FluidArgs<typename Prec<P>::T> &a, uint32_t blk,
-                                            unsigned long long *slot)
+__device__ __forceinline__ double signal_of(const FluidArgs<typename Prec<P>::T> &a, uint32_t i)
 {
     using T = typename Prec<P>::T;
-    uint32_t i = blk * kThreads + threadIdx.x;
-    double v = -1.0;
-    if (i < a.n)
-    {
-        const T m_i = a.mass[i];
-        T gx = a.force[0][i] + a.force_prior[0][i], gy = a.force[1][i] + a.force_prior[1][i];
-        T gz = D == 3 ? a.force[2][i] + a.force_prior[2][i] : T(0);
-        T fn = sqrt(D == 3 ? gx * gx + gy * gy + gz * gz : gx * gx + gy * gy);
-        T acc_scale = sqrt(T(4) * a.h * fn / m_i);
-        Rec4<T> vi = a.vel[i];
-        T vn = sqrt(D == 3 ? vi.x * vi.x + vi.y * vi.y + vi.z * vi.z : vi.x * vi.x + vi.y * vi.y);
-        v = signal_or_inf(a.c0 + vn, acc_scale, T(0));
-    }
-    block_max_to(v, slot);
+    if (i >= a.n)
+        return -1.0;
+    const T m_i = a.mass[i];
+    T gx = a.force[0][i] + a.force_prior[0][i], gy = a.force[1][i] + a.force_prior[1][i];
+    T gz = D == 3 ? a.force[2][i] + a.force_prior[2][i] : T(0);
+    T fn = sqrt(D == 3 ? gx * gx + gy * gy + gz * gz : gx * gx + gy * gy);
+    T acc_scale = sqrt(T(4) * a.h * fn / m_i);
+    Rec4<T> vi = a.vel[i];
+    T vn = sqrt(D == 3 ? vi.x * vi.x + vi.y * vi.y + vi.z * vi.z : vi.x * vi.x + vi.y * vi.y);
+    return signal_or_inf(a.c0 + vn, acc_scale, T(0));
 }
 
 template <int D, int P>
 __global__ void __launch_bounds__(kThreads) k_signal_max(FluidArgs<typename Prec<P>::T> a,
                                                          unsigned long long *slot)
 {
-    signal_body<D, P>(a, blockIdx.x, slot);
+    block_max_to(signal_of<D, P>(a, blockIdx.x * kThreads + threadIdx.x), slot);
 }
 
 template <int D, int P>
-__device__ __forceinline__ void speed_body(const FluidArgs<typename Prec<P>::T> &a, uint32_t blk,
-                                           unsigned long long *slot)
+__device__ __forceinline__ double speed_of(const FluidArgs<typename Prec<P>::T> &a, uint32_t i)
 {
     using T = typename Prec<P>::T;
-    uint32_t i = blk * kThreads + threadIdx.x;
-    double v = -1.0;
-    if (i < a.n)
-    {
-        Rec4<T> vi = a.vel[i];
-        const T v2 = D == 3 ? vi.x * vi.x + vi.y * vi.y + vi.z * vi.z : vi.x * vi.x + vi.y * vi.y;
-        v = isfinite(v2) ? (double)v2 : __builtin_huge_val();
-    }
-    block_max_to(v, slot);
+    if (i >= a.n)
+        return -1.0;
+    Rec4<T> vi = a.vel[i];
+    const T v2 = D == 3 ? vi.x * vi.x + vi.y * vi.y + vi.z * vi.z : vi.x * vi.x + vi.y * vi.y;
+    return isfinite(v2) ? (double)v2 : __builtin_huge_val();
 }
 
 template <int D, int P>
 __global__ void __launch_bounds__(kThreads) k_speed_max(FluidArgs<typename Prec<P>::T> a,
                                                         unsigned long long *slot)
 {
-    speed_body<D, P>(a, blockIdx.x, slot);
+    block_max_to(speed_of<D, P>(a, blockIdx.x * kThreads + threadIdx.x), slot);
+}
+
+// DensityRegularization, AdvectionStepSetup and the maxima of
+// AdvectionTimeStepCK and of the first sub-step's AcousticTimeStepCK, which
+// touch each particle alone (the maxima read nothing that the first two change)
+template <int D, int P>
+__device__ __forceinline__ void head_body(const FluidArgs<typename Prec<P>::T> &a, const PosArgs &pa,
+                                          typename Prec<P>::T *Vol, Rec4<typename Prec<P>::T> *posvol, uint32_t blk,
+                                          int flow, unsigned long long *scalars)
+{
+    __shared__ double red[2][kThreads / 64];
+    const uint32_t i = blk * kThreads + threadIdx.x;
+    regularize_body<D, P>(a, i, flow);
+    setup_body<D, P>(a, pa, Vol, posvol, i);
+    const double speed = wave_max(speed_of<D, P>(a, i)), signal = wave_max(signal_of<D, P>(a, i));
+    if ((threadIdx.x & 63) == 0)
+    {
+        red[0][threadIdx.x >> 6] = speed;
+        red[1][threadIdx.x >> 6] = signal;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2)
+    {
+        double m = red[threadIdx.x][0];
+        for (int w = 1; w < kThreads / 64; ++w)
+            m = fmax(m, red[threadIdx.x][w]);
+        atomic_max_spread(scalars + (threadIdx.x == 0 ? SLOT_SPEED : SLOT_MAX), m);
+    }
+}
+
+template <int D, int P>
+__global__ void __launch_bounds__(kThreads) k_step_head(FluidArgs<typename Prec<P>::T> a, PosArgs pa,
+                                                        typename Prec<P>::T *Vol, Rec4<typename Prec<P>::T> *posvol,
+                                                        int flow, unsigned long long *scalars)
+{
+    head_body<D, P>(a, pa, Vol, posvol, blockIdx.x, flow, scalars);
 }
 
 __global__ void __launch_bounds__(kThreads) k_axis_max(const double *x, uint32_t n, unsigned long long *slot)
@@ -2337,85 +2469,6 @@ __global__ void __launch_bounds__(64) k_interpolate(const Rec4<T> *obs, const Re
 }
 
 //---------------------------------------------------------------------------
-// device-side dual-time loop of sphx_advection_step (dambreak.cpp:188-207):
-// AdvectionTimeStepCK's dt from the speed max, then per sub-step
-// AcousticTimeStepCK's dt from the signal max and the loop condition
-// relaxation < advection dt, with the host's arithmetic in double
-//---------------------------------------------------------------------------
-// the max of the accumulator lanes, which are then reset for the next reduction
-__device__ __forceinline__ double lanes_max_reset(unsigned long long *lanes)
-{
-    unsigned long long m = 0;
-    for (int k = 0; k < kMaxLanes; ++k)
-    {
-        m = m > lanes[k * kMaxStride] ? m : lanes[k * kMaxStride];
-        lanes[k * kMaxStride] = kOrderedLowest;
-    }
-    return from_ordered_bits(m);
-}
-__device__ __forceinline__ void put_double(unsigned long long *slot, double v)
-{
-    *slot = (unsigned long long)__double_as_longlong(v);
-}
-__device__ __forceinline__ double get_double(const unsigned long long *slot)
-{
-    return __longlong_as_double((long long)*slot);
-}
-
-__device__ __forceinline__ void step_begin_body(unsigned long long *scalars, double u_ref, double cfl, double h,
-                                                double time)
-{
-    unsigned long long *st = scalars + SLOT_STEP;
-    const double m = lanes_max_reset(scalars + SLOT_MAX);
-    // AdvectionTimeStepCK::FinishDynamics::Result, fluid_time_step_ck.cpp:23-26
-    const double adv_dt = cfl * h / (fmax(sqrt(m), u_ref) + 2.71051e-20);
-    put_double(st + STEP_ADV_DT, adv_dt);
-    put_double(st + STEP_DT, 0.0);
-    put_double(st + STEP_RELAXATION, 0.0);
-    put_double(st + STEP_TIME, time);
-    st[STEP_COUNT] = 0;
-    st[STEP_ACTIVE] = 0;
-    // a non-finite velocity made the speed max +inf and the step zero
-    st[STEP_ERROR] = isfinite(adv_dt) && adv_dt > 0.0 ? 0ull : 1ull;
-}
-
-__global__ void k_step_begin(unsigned long long *scalars, double u_ref, double cfl, double h, double time)
-{
-    if (threadIdx.x == 0)
-        step_begin_body(scalars, u_ref, cfl, h, time);
-}
-
-__device__ __forceinline__ void substep_begin_body(unsigned long long *scalars, double cfl, double h)
-{
-    unsigned long long *st = scalars + SLOT_STEP;
-    const double relaxation = get_double(st + STEP_RELAXATION);
-    if (st[STEP_ERROR] != 0 || !(relaxation < get_double(st + STEP_ADV_DT)))
-    {
-        st[STEP_ACTIVE] = 0;
-        return;
-    }
-    // AcousticTimeStepCK::FinishDynamics::Result, fluid_time_step_ck.hpp:30-57
-    const double dt = cfl * h / (lanes_max_reset(scalars + SLOT_MAX) + 2.71051e-20);
-    if (!isfinite(dt) || !(dt > 0.0))
-    {
-        st[STEP_ERROR] = 1;
-        st[STEP_ACTIVE] = 0;
-        return;
-    }
-    put_double(st + STEP_DT, dt);
-    put_double(st + STEP_RELAXATION, relaxation + dt);
-    put_double(st + STEP_TIME, get_double(st + STEP_TIME) + dt);
-    st[STEP_COUNT] += 1;
-    st[STEP_ACTIVE] = 1;
-}
-
-__global__ void k_substep_begin(unsigned long long *scalars, double cfl, double h)
-{
-    if (threadIdx.x == 0)
-        substep_begin_body(scalars, cfl, h);
-}
-
-//---------------------------------------------------------------------------
 // Batched launches: one grid over the blocks of every scene of a batch.
 // map[b] = scene << 16 | block of that scene, laid out scene after scene, so
 // that the XCD-aware block order keeps each scene's blocks on one XCD where
@@ -2449,90 +2502,60 @@ kb_summation(const SceneArgs<typename Prec<P>::T> *__restrict__ tab, const uint3
     with_lanes<D, P>(f.n, [&](auto lanes) { summation_body<D, P, lanes.value>(f, map_block(m)); });
 }
 
-// DensityRegularization + AdvectionStepSetup, which touch each particle alone
 template <int D, int P>
-__global__ void __launch_bounds__(kThreads) kb_regularize_setup(const SceneArgs<typename Prec<P>::T> *__restrict__ tab,
-                                                                const uint32_t *__restrict__ map)
-{
-    const uint32_t m = map[blockIdx.x];
-    const SceneArgs<typename Prec<P>::T> &sa = tab[map_scene(m)];
-    const uint32_t i = map_block(m) * kThreads + threadIdx.x;
-    regularize_body<D, P>(sa.f, i, sa.flow);
-    setup_body<D, P>(sa.f, sa.pa, sa.Vol, sa.posvol, i);
-}
-
-// the max lanes of every scene to the lowest value (one block per scene)
-template <class T>
-__global__ void kb_reset_lanes(const SceneArgs<T> *__restrict__ tab, uint32_t n_scenes)
-{
-    if (blockIdx.x < n_scenes && threadIdx.x < (unsigned)kMaxLanes)
-        tab[blockIdx.x].scalars[SLOT_MAX + threadIdx.x * kMaxStride] = kOrderedLowest;
-}
-
-template <int D, int P>
-__global__ void __launch_bounds__(kThreads) kb_speed_max(const SceneArgs<typename Prec<P>::T> *__restrict__ tab,
+__global__ void __launch_bounds__(kThreads) kb_step_head(const SceneArgs<typename Prec<P>::T> *__restrict__ tab,
                                                          const uint32_t *__restrict__ map)
 {
     const uint32_t m = map[blockIdx.x];
     const SceneArgs<typename Prec<P>::T> &sa = tab[map_scene(m)];
-    speed_body<D, P>(sa.f, map_block(m), sa.scalars + SLOT_MAX);
+    head_body<D, P>(sa.f, sa.pa, sa.Vol, sa.posvol, map_block(m), sa.flow, sa.scalars);
 }
 
 template <int D, int P>
-__global__ void __launch_bounds__(kThreads) kb_signal_max(const SceneArgs<typename Prec<P>::T> *__restrict__ tab,
-                                                          const uint32_t *__restrict__ map)
+__global__ void __launch_bounds__(kThreads) kb_begin_init(const SceneArgs<typename Prec<P>::T> *__restrict__ tab,
+                                                          const uint32_t *__restrict__ map, uint32_t k)
 {
     const uint32_t m = map[blockIdx.x];
     const SceneArgs<typename Prec<P>::T> &sa = tab[map_scene(m)];
-    signal_body<D, P>(sa.f, map_block(m), sa.scalars + SLOT_MAX);
-}
-
-// one thread per scene
-template <class T>
-__global__ void kb_step_begin(const SceneArgs<T> *__restrict__ tab, uint32_t n_scenes)
-{
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < n_scenes)
-    {
-        const SceneArgs<T> &sa = tab[s];
-        step_begin_body(sa.scalars, sa.u_ref, sa.advection_cfl, sa.h, *sa.time);
-    }
-}
-template <class T>
-__global__ void kb_substep_begin(const SceneArgs<T> *__restrict__ tab, uint32_t n_scenes)
-{
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < n_scenes)
-        substep_begin_body(tab[s].scalars, tab[s].acoustic_cfl, tab[s].h);
-}
-
-template <int D, int P>
-__global__ void __launch_bounds__(kThreads) kb_init_1st(const SceneArgs<typename Prec<P>::T> *__restrict__ tab,
-                                                        const uint32_t *__restrict__ map)
-{
-    const uint32_t m = map[blockIdx.x];
-    init_1st_body<D, P>(tab[map_scene(m)].f, map_block(m), 0.0);
+    StepBegin sb;
+    sb.scalars = sa.scalars;
+    sb.parity = k & 1u;
+    sb.first = k == 0u;
+    sb.acoustic_cfl = sa.acoustic_cfl;
+    sb.advection_cfl = sa.advection_cfl;
+    sb.u_ref = sa.u_ref;
+    sb.h = sa.h;
+    sb.time = *sa.time;
+    begin_init_body<D, P>(sa.f, sb, map_block(m), ~0u - sa.f.n); // one round
 }
 
 template <int D, int P, bool RIEMANN>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(P == P_MIXED ? 5 : 1))) kb_pass1(const SceneArgs<typename Prec<P>::T> *__restrict__ tab,
-                                                     const uint32_t *__restrict__ map)
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(P == P_MIXED ? 5 : 1)))
+kb_pass1(const SceneArgs<typename Prec<P>::T> *__restrict__ tab, const uint32_t *__restrict__ map, uint32_t k)
 {
     const uint32_t m = map[xcd_block_index()];
-    const FluidArgs<typename Prec<P>::T> &f = tab[map_scene(m)].f;
+    const SceneArgs<typename Prec<P>::T> &sa = tab[map_scene(m)];
+    const FluidArgs<typename Prec<P>::T> &f = sa.f;
+    if (sa.scalars[step_slot(~k & 1u) + STEP_ACTIVE] == 0ull) // block-uniform
+        return;
+    const double dt = get_double(sa.scalars + step_slot(~k & 1u) + STEP_DT);
     with_lanes<D, P>(f.n, [&](auto lanes) {
-        pass1_body<D, P, RIEMANN, true, false, lanes.value>(f, map_block(m), 0.0);
+        pass1_body<D, P, RIEMANN, true, false, lanes.value>(f, map_block(m), dt);
     });
 }
 
 template <int D, int P, bool RIEMANN>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(P == P_MIXED ? 4 : 1)))
-kb_pass2(const SceneArgs<typename Prec<P>::T> *__restrict__ tab, const uint32_t *__restrict__ map)
+kb_pass2(const SceneArgs<typename Prec<P>::T> *__restrict__ tab, const uint32_t *__restrict__ map, uint32_t k)
 {
     const uint32_t m = map[xcd_block_index()];
     const SceneArgs<typename Prec<P>::T> &sa = tab[map_scene(m)];
+    if (sa.scalars[step_slot(~k & 1u) + STEP_ACTIVE] == 0ull) // block-uniform
+        return;
+    const double dt = get_double(sa.scalars + step_slot(~k & 1u) + STEP_DT);
     with_lanes<D, P>(sa.f.n, [&](auto lanes) {
-        pass2_body<D, P, RIEMANN, true, false, lanes.value>(sa.f, map_block(m), 0.0, sa.scalars + SLOT_MAX);
+        pass2_body<D, P, RIEMANN, true, false, lanes.value>(sa.f, map_block(m), dt,
+                                                            sa.scalars + signal_slot(~k & 1u));
     });
 }
 
@@ -2541,12 +2564,14 @@ kb_pass2(const SceneArgs<typename Prec<P>::T> *__restrict__ tab, const uint32_t 
 // state is copied to state[s * STEP_SLOTS ...] for the host
 template <class T>
 __global__ void kb_gate(const SceneArgs<T> *__restrict__ tab, uint32_t n_scenes, const uint32_t *__restrict__ tail_on,
-                        uint32_t *gate, unsigned long long *state)
+                        uint32_t *gate, unsigned long long *state, uint32_t substeps)
 {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n_scenes)
         return;
-    const unsigned long long *st = tab[s].scalars + SLOT_STEP;
+    unsigned long long *st = tab[s].scalars + step_slot(substeps & 1u);
+    if (tab[s].f.n == 0u)
+        st[STEP_ERROR] = 1; // no particle, no time step
     for (int k = 0; k < STEP_SLOTS; ++k)
         state[(size_t)s * STEP_SLOTS + k] = st[k];
     const bool done = st[STEP_ERROR] == 0 && !(get_double(st + STEP_RELAXATION) < get_double(st + STEP_ADV_DT));
@@ -2576,7 +2601,9 @@ static FluidArgs<T> fluid_args(sphx_body *b)
 {
     FluidArgs<T> a{};
     a.n = b->n;
-    a.step = b->ctx->device_step ? b->ctx->scalars_d + SLOT_STEP : nullptr;
+    const StepBegin &sb = b->ctx->step;
+    a.step = sb.scalars ? sb.scalars + step_slot(sb.parity ^ 1u) : nullptr;
+    a.in_loop = a.step != nullptr;
     a.posvol = (const Rec4<T> *)b->posvol;
     a.vel = (Rec4<T> *)b->vel;
     for (int k = 0; k < 3; ++k)
@@ -2797,12 +2824,13 @@ sphx_status update_position(sphx_body *b)
 template <int D, int P>
 struct SummationL
 {
-    static sphx_status run(sphx_body *b, sphx_relation *inner, sphx_relation *const *c, int nc)
+    static sphx_status run(sphx_body *b, sphx_relation *inner, sphx_relation *const *c, int nc, bool reset_lanes)
     {
         using T = typename Prec<P>::T;
         if (!b->n)
             return SPHX_OK;
         FluidArgs<T> a = fluid_args<T>(b);
+        a.reset_lanes = reset_lanes ? b->ctx->scalars_d : nullptr;
         attach_relations(a, inner, c, nc);
         ProfileScope prof(b->ctx, "compression_summation");
         const size_t lds = a.stage_count ? sum_lds<D, P>() : 0;
@@ -2816,9 +2844,30 @@ struct SummationL
         return SPHX_OK;
     }
 };
-sphx_status compression_summation(sphx_relation *inner, sphx_relation *const *c, int nc)
+sphx_status compression_summation(sphx_relation *inner, sphx_relation *const *c, int nc, bool reset_lanes)
 {
-    return dispatch<SummationL>(inner->source, inner, c, nc);
+    return dispatch<SummationL>(inner->source, inner, c, nc, reset_lanes);
+}
+
+template <int D, int P>
+struct HeadL
+{
+    static sphx_status run(sphx_body *b, int flow)
+    {
+        using T = typename Prec<P>::T;
+        if (!b->n)
+            return SPHX_OK;
+        ProfileScope prof(b->ctx, "state_update");
+        hipLaunchKernelGGL((k_step_head<D, P>), dim3(grid_for(b->n, kThreads)), dim3(kThreads), 0, b->ctx->stream,
+                           fluid_args<T>(b), pos_args(b), (T *)b->Vol, (Rec4<T> *)b->posvol, flow, b->ctx->scalars_d);
+        LAUNCH_CHECK();
+        return SPHX_OK;
+    }
+};
+sphx_status advection_step_head(sphx_body *b, int flow)
+{
+    b->state_version++;
+    return dispatch<HeadL>(b, flow);
 }
 
 // launch one of the eight boolean instantiations of a pass kernel
@@ -2897,7 +2946,13 @@ struct Acoustic1L
         dim3 g(grid_for(b->n, kThreads)), blk(kThreads);
         {
             ProfileScope prof(b->ctx, "acoustic_init");
-            hipLaunchKernelGGL((k_init_1st<D, P>), g, blk, 0, b->ctx->stream, a, dt);
+            if (a.step)
+                // at most eight blocks a CU: each of them reads the lanes (8M particles in one
+                // round of 31,283 blocks 44 us, in 2,048 blocks 32)
+                hipLaunchKernelGGL((k_begin_init<D, P>), dim3(std::min(g.x, 2048u)), blk, 0, b->ctx->stream, a,
+                                   b->ctx->step);
+            else
+                hipLaunchKernelGGL((k_init_1st<D, P>), g, blk, 0, b->ctx->stream, a, dt);
         }
         ProfileScope prof(b->ctx, "acoustic_pass1");
         const bool rs = riemann != SPHX_RIEMANN_NONE;
@@ -2955,7 +3010,7 @@ sphx_status acoustic_2nd_half(sphx_relation *inner, sphx_relation *const *w, int
                               bool run_init, bool fuse_cfl)
 {
     sphx_body *b = inner->source;
-    unsigned long long *slot = fuse_cfl ? b->ctx->scalars_d + SLOT_MAX : nullptr;
+    unsigned long long *slot = fuse_cfl ? b->ctx->scalars_d + signal_slot(b->ctx->step.parity ^ 1u) : nullptr;
     sphx_status s = ensure_staged(inner);
     return s ? s : dispatch<Acoustic2L>(b, inner, w, nw, riemann, dt, run_init, slot, false);
 }
@@ -3017,7 +3072,7 @@ sphx_status acoustic_2nd_half_corrected(sphx_relation *inner, sphx_relation *con
                                         double dt, bool run_init, bool fuse_cfl)
 {
     sphx_body *b = inner->source;
-    unsigned long long *slot = fuse_cfl ? b->ctx->scalars_d + SLOT_MAX : nullptr;
+    unsigned long long *slot = fuse_cfl ? b->ctx->scalars_d + signal_slot(b->ctx->step.parity ^ 1u) : nullptr;
     sphx_status s = ensure_staged(inner);
     return s ? s : dispatch<Acoustic2L>(b, inner, w, nw, riemann, dt, run_init, slot, true);
 }
@@ -3364,21 +3419,6 @@ sphx_status build_kernel_poly(sphx_relation *rel)
     return rel->source->P == P_FP64 ? build_poly_t<double>(rel) : build_poly_t<float>(rel);
 }
 
-sphx_status step_begin(sphx_context *ctx, double u_ref, double advection_cfl, double h, double time)
-{
-    hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(64), 0, ctx->stream, ctx->scalars_d, u_ref, advection_cfl, h,
-                       time);
-    SPHX_HIP(hipGetLastError());
-    return SPHX_OK;
-}
-
-sphx_status substep_begin(sphx_context *ctx, double acoustic_cfl, double h)
-{
-    hipLaunchKernelGGL(k_substep_begin, dim3(1), dim3(64), 0, ctx->stream, ctx->scalars_d, acoustic_cfl, h);
-    SPHX_HIP(hipGetLastError());
-    return SPHX_OK;
-}
-
 //=============================================================================
 // batched launches (host side)
 //=============================================================================
@@ -3391,8 +3431,9 @@ static void fill_scene_args(void *dst, sphx_relation *inner, sphx_relation *cons
     sphx_body *b = inner->source;
     SceneArgs<T> a{};
     a.f = fluid_args<T>(b);
-    a.f.step = b->ctx->scalars_d + SLOT_STEP;
-    a.f.lanes = b->ctx->scalars_d + SLOT_MAX;
+    a.f.step = nullptr; // the batched passes read the loop state themselves
+    a.f.in_loop = 1;
+    a.f.reset_lanes = b->ctx->scalars_d;
     a.f.riemann = cfg->riemann;
     attach_relations(a.f, inner, w, nw);
     if (!staged)
@@ -3436,33 +3477,28 @@ struct BatchL
     static size_t lds_pass2(const BatchFluid &b) { return b.stage_cap ? pass2_lds<D, P>() : 0; }
     static sphx_status head(const BatchFluid &b)
     {
-        const dim3 g(b.blocks), blk(kThreads), gs(grid_for(b.n_scenes, 64)), bs(64);
+        const dim3 g(b.blocks), blk(kThreads);
         allow_lds(kb_summation<D, P>, lds_sum(b));
         hipLaunchKernelGGL((kb_summation<D, P>), dim3(b.blocks_sums), blk, lds_sum(b), b.stream, tab(b), b.map_sums);
-        hipLaunchKernelGGL((kb_regularize_setup<D, P>), g, blk, 0, b.stream, tab(b), b.map);
-        hipLaunchKernelGGL((kb_reset_lanes<T>), dim3(b.n_scenes), dim3(64), 0, b.stream, tab(b), b.n_scenes);
-        hipLaunchKernelGGL((kb_speed_max<D, P>), g, blk, 0, b.stream, tab(b), b.map);
-        hipLaunchKernelGGL((kb_step_begin<T>), gs, bs, 0, b.stream, tab(b), b.n_scenes);
-        hipLaunchKernelGGL((kb_signal_max<D, P>), g, blk, 0, b.stream, tab(b), b.map);
+        hipLaunchKernelGGL((kb_step_head<D, P>), g, blk, 0, b.stream, tab(b), b.map);
         SPHX_HIP(hipGetLastError());
         return SPHX_OK;
     }
-    static sphx_status substep(const BatchFluid &b)
+    static sphx_status substep(const BatchFluid &b, uint32_t k)
     {
-        const dim3 g(b.blocks), blk(kThreads), gs(grid_for(b.n_scenes, 64)), bs(64);
+        const dim3 g(b.blocks), blk(kThreads);
         allow_lds(kb_pass1<D, P, RIEMANN>, lds_pass1(b));
         allow_lds(kb_pass2<D, P, RIEMANN>, lds_pass2(b));
-        hipLaunchKernelGGL((kb_substep_begin<T>), gs, bs, 0, b.stream, tab(b), b.n_scenes);
-        hipLaunchKernelGGL((kb_init_1st<D, P>), g, blk, 0, b.stream, tab(b), b.map);
-        hipLaunchKernelGGL((kb_pass1<D, P, RIEMANN>), dim3(b.blocks_sums), blk, lds_pass1(b), b.stream, tab(b), b.map_sums);
-        hipLaunchKernelGGL((kb_pass2<D, P, RIEMANN>), dim3(b.blocks_sums), blk, lds_pass2(b), b.stream, tab(b), b.map_sums);
+        hipLaunchKernelGGL((kb_begin_init<D, P>), g, blk, 0, b.stream, tab(b), b.map, k);
+        hipLaunchKernelGGL((kb_pass1<D, P, RIEMANN>), dim3(b.blocks_sums), blk, lds_pass1(b), b.stream, tab(b), b.map_sums, k);
+        hipLaunchKernelGGL((kb_pass2<D, P, RIEMANN>), dim3(b.blocks_sums), blk, lds_pass2(b), b.stream, tab(b), b.map_sums, k);
         SPHX_HIP(hipGetLastError());
         return SPHX_OK;
     }
-    static sphx_status gate(const BatchFluid &b)
+    static sphx_status gate(const BatchFluid &b, uint32_t substeps)
     {
         hipLaunchKernelGGL((kb_gate<T>), dim3(grid_for(b.n_scenes, 64)), dim3(64), 0, b.stream, tab(b), b.n_scenes,
-                           b.tail_on, b.gate, b.state);
+                           b.tail_on, b.gate, b.state, substeps);
         SPHX_HIP(hipGetLastError());
         return SPHX_OK;
     }
@@ -3499,13 +3535,13 @@ sphx_status batch_step_head(const BatchFluid &b)
 {
     return BatchDispatch<BatchL>::run(b, [&](auto l) { return decltype(l)::head(b); });
 }
-sphx_status batch_substep(const BatchFluid &b)
+sphx_status batch_substep(const BatchFluid &b, uint32_t k)
 {
-    return BatchDispatch<BatchL>::run(b, [&](auto l) { return decltype(l)::substep(b); });
+    return BatchDispatch<BatchL>::run(b, [&](auto l) { return decltype(l)::substep(b, k); });
 }
-sphx_status batch_step_gate(const BatchFluid &b)
+sphx_status batch_step_gate(const BatchFluid &b, uint32_t substeps)
 {
-    return BatchDispatch<BatchL>::run(b, [&](auto l) { return decltype(l)::gate(b); });
+    return BatchDispatch<BatchL>::run(b, [&](auto l) { return decltype(l)::gate(b, substeps); });
 }
 sphx_status batch_position(const BatchFluid &b)
 {

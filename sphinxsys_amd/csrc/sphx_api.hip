@@ -558,31 +558,43 @@ namespace sphx
 {
 // dambreak.cpp:196-207: while (relaxation < advection dt) { dt = acoustic dt; 1st
 // half; 2nd half; relaxation += dt }.  Each sub-step's dt, the loop condition
-// and the time are evaluated on the device (k_substep_begin); launches past
-// the end of the loop return at once.  The first batch has `batch` sub-steps;
-// when it was too short the loop goes on one sub-step at a time.  On return
-// the step state is in the context's pinned mirror (SLOT_STEP).
+// and the time are evaluated on the device (k_begin_init); launches past the end
+// of the loop return at once.  The first batch has `batch` sub-steps; when it was
+// too short the loop goes on one sub-step at a time.  `done` sub-steps of this
+// advection step were launched before.  On return the step state is in the
+// context's pinned mirror, at *state.
 sphx_status advection_substeps(sphx_relation *inner, sphx_relation *const *walls, int n_wall,
-                               const sphx_advection_config *cfg, uint32_t batch)
+                               const sphx_advection_config *cfg, double time, uint32_t done, uint32_t batch,
+                               const unsigned long long **state)
 {
     sphx_body *b = inner->source;
     sphx_context *ctx = b->ctx;
+    if (b->n == 0)
+    {
+        set_error("non-finite acoustic time step: the fluid body has no particles");
+        return SPHX_E_NONFINITE;
+    }
     const bool corrected = cfg->correction == SPHX_CORRECTION_LINEAR;
     struct DeviceStep
     {
         sphx_context *c;
-        explicit DeviceStep(sphx_context *c) : c(c) { c->device_step = true; }
-        ~DeviceStep() { c->device_step = false; }
+        explicit DeviceStep(sphx_context *c) : c(c) {}
+        ~DeviceStep() { c->step = StepBegin(); }
     } device_step(ctx);
-    const unsigned long long *st = ctx->scalars_h + SLOT_STEP;
+    StepBegin &sb = ctx->step;
+    sb.scalars = ctx->scalars_d;
+    sb.acoustic_cfl = cfg->acoustic_cfl;
+    sb.advection_cfl = cfg->advection_cfl;
+    sb.u_ref = cfg->u_ref;
+    sb.h = b->h;
+    sb.time = time;
     sphx_status s;
     while (true)
     {
-        for (uint32_t k = 0; k < batch; ++k)
+        for (uint32_t k = 0; k < batch; ++k, ++done)
         {
-            if ((s = substep_begin(ctx, cfg->acoustic_cfl, b->h)))
-                return s;
-            // k_substep_begin read the signal max and reset the lanes for pass 2
+            sb.parity = done & 1u;
+            sb.first = done == 0u;
             if (corrected)
                 s = acoustic_1st_half_corrected(inner, walls, n_wall, cfg->riemann, 0.0, true);
             else
@@ -596,7 +608,9 @@ sphx_status advection_substeps(sphx_relation *inner, sphx_relation *const *walls
             if (s)
                 return s;
         }
-        if ((s = read_scalars(ctx, SLOT_STEP, STEP_SLOTS)))
+        const unsigned long long *st = ctx->scalars_h + step_slot(done & 1u);
+        *state = st;
+        if ((s = read_scalars(ctx, step_slot(done & 1u), STEP_SLOTS)))
             return s;
         if (st[STEP_ERROR])
         {
@@ -612,6 +626,108 @@ sphx_status advection_substeps(sphx_relation *inner, sphx_relation *const *walls
     }
 }
 
+// the slices of a relation for lists of up to kmax entries
+static sphx_status reserve_slices(sphx_relation *r, uint32_t kmax)
+{
+    hipStream_t stream = r->source->ctx->stream;
+    const size_t nchunks = ((size_t)r->source->n + 63) / 64;
+    const size_t need = std::max<size_t>(nchunks * kmax * 64, 64);
+    if (need >= (1ull << 32))
+    {
+        set_error("neighbour slices exceed 2^32 entries");
+        return SPHX_E_CAPACITY;
+    }
+    if (need <= r->slice_capacity && r->slice)
+        return SPHX_OK;
+    // released after the kernels already queued on the stream
+    dev_free(stream, r->slice);
+    r->slice = nullptr;
+    dev_free(stream, r->local_slice);
+    r->local_slice = nullptr;
+    r->slice_capacity = 0;
+    sphx_status s;
+    if ((s = dev_alloc(stream, (void **)&r->slice, need * sizeof(uint32_t))))
+        return s;
+    if (r->staged && (s = dev_alloc(stream, (void **)&r->local_slice, need * sizeof(uint16_t))))
+        return s;
+    r->slice_capacity = need;
+    return SPHX_OK;
+}
+
+// UpdateRelation of several relations of one context: every build is launched,
+// then the neighbour counts that did not fit are read back once.  A relation
+// whose slice width was too small is rebuilt with a larger one, as the
+// reference grows NeighborIndex on overflow (update_body_relation.hpp:145-155).
+static sphx_status update_relations(sphx_relation *const *rels, int count)
+{
+    sphx_context *ctx = rels[0]->source->ctx;
+    SPHX_HIP(hipSetDevice(ctx->device));
+    unsigned long long *slots = ctx->scalars_d + SLOT_NEEDED;
+    sphx_status s;
+    struct Work
+    {
+        uint32_t kmax;
+        bool scan, done;
+    } work[kMaxRelations];
+    for (int k = 0; k < count; ++k)
+    {
+        sphx_relation *r = rels[k];
+        work[k] = {r->kmax ? r->kmax : (r->source->D == 3 ? 96u : 32u), false, false};
+        if (!r->inner && (s = cell_near_flags(r->cll)))
+            return s;
+    }
+    for (int attempt = 0; attempt < 5; ++attempt)
+    {
+        if ((s = fill_u64(ctx, slots, (size_t)count, 0ull)))
+            return s;
+        for (int k = 0; k < count; ++k)
+            if (!work[k].done && ((s = reserve_slices(rels[k], work[k].kmax)) ||
+                                  (s = relation_build(rels[k], work[k].kmax, slots + k, work[k].scan))))
+                return s;
+        if ((s = read_scalars(ctx, SLOT_NEEDED, count)))
+            return s;
+        bool all = true;
+        for (int k = 0; k < count; ++k)
+        {
+            const unsigned long long needed = ctx->scalars_h[SLOT_NEEDED + k];
+            if (work[k].done || needed <= work[k].kmax)
+            {
+                work[k].done = true;
+                continue;
+            }
+            all = false;
+            if (needed >= kTooDense)
+            {
+                work[k].scan = true; // a cell row too dense for the tiled build's row code
+                continue;
+            }
+            if (needed > 60000)
+            {
+                set_error("a particle has more than 60000 neighbours: positions collapsed");
+                return SPHX_E_CAPACITY;
+            }
+            work[k].kmax = (uint32_t)((needed + needed / 4 + 7) / 8 * 8);
+        }
+        if (!all)
+            continue;
+        for (int k = 0; k < count; ++k)
+        {
+            sphx_relation *r = rels[k];
+            r->kmax = work[k].kmax;
+            r->slice_total = ((size_t)r->source->n + 63) / 64 * work[k].kmax * 64;
+            r->stage_stale = true; // the staging sets follow with the first dynamics that reads the lists often
+            r->csr_valid = false;  // the CSR view (offsets and indices) is built when read
+            r->built = true;
+            r->builds++;
+            r->built_version = r->source->config_version;
+            r->target_version = r->target->config_version;
+        }
+        return SPHX_OK;
+    }
+    set_error("neighbour lists did not fit after growing the slice width");
+    return SPHX_E_CAPACITY;
+}
+
 // the end of an advection step: position update, ParticleSortCK when due, the
 // fluid cell linked list and the relations
 sphx_status advection_tail(sphx_relation *inner, sphx_relation *const *walls, int n_wall,
@@ -623,12 +739,17 @@ sphx_status advection_tail(sphx_relation *inner, sphx_relation *const *walls, in
         return s;
     if (sort_now && (s = sphx_particle_sort(b, cll)))
         return s;
-    if ((s = sphx_update_cell_linked_list(cll)) || (s = sphx_update_relation(inner)))
+    if ((s = sphx_update_cell_linked_list(cll)))
         return s;
+    sphx_relation *rels[kMaxRelations] = {inner};
     for (int k = 0; k < n_wall; ++k)
-        if ((s = sphx_update_relation(walls[k])))
-            return s;
-    return SPHX_OK;
+    {
+        rels[k + 1] = walls[k];
+        const sphx_cell_linked_list *c = walls[k]->cll;
+        if (!c->built || c->built_version != c->body->config_version)
+            return state_error("target cell linked list not updated since the last configuration change");
+    }
+    return update_relations(rels, 1 + n_wall);
 }
 } // namespace sphx
 
@@ -1220,76 +1341,7 @@ sphx_status sphx_update_relation(sphx_relation *r)
     sphx_cell_linked_list *c = r->cll;
     if (!c->built || c->built_version != c->body->config_version)
         return state_error("target cell linked list not updated since the last configuration change");
-    sphx_context *ctx = r->source->ctx;
-    SPHX_HIP(hipSetDevice(ctx->device));
-    sphx_status s;
-    // one scan builds the slices (and the staging sets); grow the slice width
-    // and rebuild when a particle has more neighbours than it, as the
-    // reference grows NeighborIndex on overflow (update_body_relation.hpp:145-155)
-    const size_t n = r->source->n;
-    const size_t nchunks = (n + 63) / 64;
-    uint32_t kmax = r->kmax ? r->kmax : (r->source->D == 3 ? 96u : 32u);
-    if (!r->inner && (s = cell_near_flags(c)))
-        return s;
-    bool scan = false, done = false;
-    for (int attempt = 0; attempt < 5 && !done; ++attempt)
-    {
-        const size_t need = std::max<size_t>(nchunks * kmax * 64, 64);
-        if (need >= (1ull << 32))
-        {
-            set_error("neighbour slices exceed 2^32 entries");
-            return SPHX_E_CAPACITY;
-        }
-        if (need > r->slice_capacity || !r->slice)
-        {
-            // released after the kernels already queued on the stream
-            dev_free(ctx->stream, r->slice);
-            r->slice = nullptr;
-            dev_free(ctx->stream, r->local_slice);
-            r->local_slice = nullptr;
-            r->slice_capacity = 0;
-            if ((s = dev_alloc(ctx->stream, (void **)&r->slice, need * sizeof(uint32_t))))
-                return s;
-            if (r->staged && (s = dev_alloc(ctx->stream, (void **)&r->local_slice, need * sizeof(uint16_t))))
-                return s;
-            r->slice_capacity = need;
-        }
-        if ((s = fill_u64(ctx, ctx->scalars_d + SLOT_NEEDED, 1, 0ull)) ||
-            (s = relation_build(r, kmax, ctx->scalars_d + SLOT_NEEDED, scan)) ||
-            (s = read_scalars(ctx, SLOT_NEEDED, 1)))
-            return s;
-        const unsigned long long needed = ctx->scalars_h[SLOT_NEEDED];
-        if (needed <= kmax)
-        {
-            done = true;
-            break;
-        }
-        if (needed >= kTooDense)
-        {
-            scan = true; // a cell row too dense for the tiled build's row code
-            continue;
-        }
-        if (needed > 60000)
-        {
-            set_error("a particle has more than 60000 neighbours: positions collapsed");
-            return SPHX_E_CAPACITY;
-        }
-        kmax = (uint32_t)((needed + needed / 4 + 7) / 8 * 8);
-    }
-    if (!done)
-    {
-        set_error("neighbour lists did not fit after growing the slice width");
-        return SPHX_E_CAPACITY;
-    }
-    r->kmax = kmax;
-    r->slice_total = nchunks * kmax * 64;
-    r->stage_stale = true; // the staging sets follow with the first dynamics that reads the lists often
-    r->csr_valid = false; // the CSR view (offsets and indices) is built when read
-    r->built = true;
-    r->builds++;
-    r->built_version = r->source->config_version;
-    r->target_version = r->target->config_version;
-    return SPHX_OK;
+    return update_relations(&r, 1);
 }
 
 sphx_status sphx_relation_read(sphx_relation *r, uint32_t *size, uint32_t *offset, uint32_t *index, size_t capacity,
@@ -1681,14 +1733,8 @@ sphx_status sphx_advection_step(sphx_relation *inner, sphx_relation *const *wall
     sphx_body *b = inner->source;
     sphx_context *ctx = b->ctx;
     SPHX_HIP(hipSetDevice(ctx->device));
-    if ((s = ensure_staged(inner)) || (s = compression_summation(inner, walls, n_wall)) ||
-        (s = density_regularization(b, cfg->flow_type)) ||
-        (s = advection_step_setup(b)))
-        return s;
-    // AdvectionTimeStepCK on the device: the loop below runs without host
-    // round trips, the host reads the loop state once per batch of sub-steps
-    if ((s = reset_max(ctx)) || (s = advection_speed_max(b, ctx->scalars_d + SLOT_MAX)) ||
-        (s = step_begin(ctx, cfg->u_ref, cfg->advection_cfl, b->h, *time)))
+    if ((s = ensure_staged(inner)) || (s = compression_summation(inner, walls, n_wall, true)) ||
+        (s = advection_step_head(b, cfg->flow_type)))
         return s;
     // dambreak.cpp:192-193
     if (cfg->surface_indication && (s = free_surface_indication(inner, walls, n_wall)))
@@ -1696,13 +1742,11 @@ sphx_status sphx_advection_step(sphx_relation *inner, sphx_relation *const *wall
     const bool corrected = cfg->correction == SPHX_CORRECTION_LINEAR;
     if (corrected && (s = linear_correction_matrix(inner, walls, n_wall, cfg->correction_alpha)))
         return s;
-    // AcousticTimeStepCK of the first sub-step from the current state (k_step_begin
-    // left the max lanes reset)
-    if ((s = acoustic_signal_max(b, ctx->scalars_d + SLOT_MAX)))
+    // AdvectionTimeStepCK and the sub-steps on the device: the loop runs without
+    // host round trips, the host reads its state once per batch of sub-steps
+    const unsigned long long *st = nullptr;
+    if ((s = advection_substeps(inner, walls, n_wall, cfg, *time, 0u, ctx->last_substeps ? ctx->last_substeps : 1u, &st)))
         return s;
-    if ((s = advection_substeps(inner, walls, n_wall, cfg, ctx->last_substeps ? ctx->last_substeps : 1u)))
-        return s;
-    const unsigned long long *st = ctx->scalars_h + SLOT_STEP;
     const uint32_t count = (uint32_t)st[STEP_COUNT];
     std::memcpy(time, st + STEP_TIME, sizeof(double));
     ctx->last_substeps = count;

@@ -41,7 +41,8 @@ struct Scratch
     void release();
 };
 
-constexpr int kScalarSlots = 1024;
+constexpr int kScalarSlots = 2048;
+constexpr int kMaxRelations = 5; // inner and 0..4 walls
 constexpr size_t kSmallTransfer = 256u << 10; // field transfers up to this size use the context's own pinned memory
 constexpr uint32_t kStageBlock = 256;          // source particles per staging block
 constexpr uint32_t kStageOverflow = 0xffffffffu;
@@ -69,13 +70,19 @@ constexpr unsigned long long kTooDense = 1ull << 40;
 enum ScalarSlot
 {
     SLOT_TOTAL = 2,      // u32 totals returned by scans (stored as u64)
-    SLOT_NEEDED = 4,     // u64: neighbour count beyond the slice width
     SLOT_SUM_BASE = 8,   // double partial sums region start (reduce_sum final)
-    SLOT_STEP = 16,      // device-side sub-step control of sphx_advection_step (StepSlot offsets)
-    SLOT_MAX = 512       // kMaxLanes ordered-bits max accumulators, kMaxStride apart
+    SLOT_NEEDED = 32,    // u64 per relation of an update: neighbour count beyond the slice width
+    SLOT_STEP = 16,      // device-side sub-step control of sphx_advection_step: two states (step_slot)
+    SLOT_MAX = 512,      // kMaxLanes ordered-bits max accumulators, kMaxStride apart: signal speeds, even sub-steps
+    SLOT_MAX_ODD = 1024, // ... odd sub-steps
+    SLOT_SPEED = 1536    // ... advection speeds
 };
-// offsets from SLOT_STEP: the dual-time loop state kept on the device so that
-// the acoustic sub-steps of an advection step run without host round trips
+// Offsets from a state: the dual-time loop kept on the device so that the
+// acoustic sub-steps of an advection step run without host round trips.  Every
+// block of a sub-step's first kernel works the sub-step's state out of the
+// previous one, so that no launch of a single thread is needed for it; the
+// states and the signal lanes alternate, since some blocks still read the
+// previous ones while others write.
 enum StepSlot
 {
     STEP_ADV_DT = 0,     // double: advection dt of the step
@@ -86,6 +93,18 @@ enum StepSlot
     STEP_ACTIVE = 5,     // u64: 1 while the current sub-step runs
     STEP_ERROR = 6,      // u64: 1 when a non-finite acoustic dt stopped the loop
     STEP_SLOTS = 7
+};
+// the state that sub-step `parity` (its number's lowest bit) starts from, and the
+// lanes with the signal speeds it takes its dt from
+constexpr int step_slot(uint32_t parity) { return SLOT_STEP + (parity ? 8 : 0); }
+constexpr int signal_slot(uint32_t parity) { return parity ? SLOT_MAX_ODD : SLOT_MAX; }
+// arguments of the device-side loop
+struct StepBegin
+{
+    unsigned long long *scalars = nullptr; // the context's scalar slots (null: no device-side loop)
+    uint32_t parity = 0;
+    int first = 0;                         // the step's first sub-step: its state from the speed lanes
+    double acoustic_cfl = 0, advection_cfl = 0, u_ref = 0, h = 0, time = 0;
 };
 } // namespace sphx
 
@@ -108,8 +127,8 @@ struct sphx_context
     unsigned long long *scalars_h = nullptr; // pinned mirror, followed by kSmallTransfer bytes for field transfers
     unsigned char *transfer_h = nullptr;
     sphx::Scratch sort_keys, sort_vals, sort_hist, scan_blocks, reduce_parts, gather_tmp, cll_cursor;
-    // while set, the acoustic kernels take dt and their run flag from the SLOT_STEP slots
-    bool device_step = false;
+    // while its scalars are set, the acoustic kernels take dt and their run flag from the device-side loop
+    sphx::StepBegin step;
     uint32_t last_substeps = 0; // sub-steps of the previous sphx_advection_step
 };
 
@@ -262,16 +281,16 @@ sphx_status gravity_force(sphx_body *b, const double *g);
 sphx_status density_regularization(sphx_body *b, int flow);
 sphx_status advection_step_setup(sphx_body *b);
 sphx_status update_position(sphx_body *b);
-sphx_status compression_summation(sphx_relation *inner, sphx_relation *const *c, int nc);
+// reset_lanes: also clears the max lanes of an advection step (signal of sub-step 0, speed)
+sphx_status compression_summation(sphx_relation *inner, sphx_relation *const *c, int nc, bool reset_lanes = false);
+// density_regularization and advection_step_setup, and the maxima of
+// AdvectionTimeStepCK and AcousticTimeStepCK into the speed and signal lanes
+sphx_status advection_step_head(sphx_body *b, int flow);
 // fuse_init_2nd: pass 1 also runs AcousticStep2ndHalf's initialize
 sphx_status acoustic_1st_half(sphx_relation *inner, sphx_relation *const *w, int nw, int riemann,
                               double dt, bool fuse_init_2nd);
 // run_init: launch the 2nd half's initialize (false when pass 1 fused it);
-// device-side dual-time loop: the step state from the advection speed max in
-// the SLOT_MAX lanes, then per sub-step its dt from the signal max there
-sphx_status step_begin(sphx_context *ctx, double u_ref, double advection_cfl, double h, double time);
-sphx_status substep_begin(sphx_context *ctx, double acoustic_cfl, double h);
-// fuse_cfl: max-reduce the next sub-step's signal speed into the SLOT_MAX lanes
+// fuse_cfl: max-reduce the next sub-step's signal speed into its lanes
 sphx_status acoustic_2nd_half(sphx_relation *inner, sphx_relation *const *w, int nw, int riemann,
                               double dt, bool run_init, bool fuse_cfl);
 // the same with the inner neighbours found by a cell traversal (3D FP32-mixed)
@@ -323,9 +342,9 @@ void batch_scene_args(void *dst, sphx_relation *inner, sphx_relation *const *w, 
                       const sphx_advection_config *cfg, const double *time_dev, bool staged);
 // compression summation, regularization + setup, advection dt, first acoustic signal max
 sphx_status batch_step_head(const BatchFluid &b);
-// one acoustic sub-step: its dt and loop flag, 1st half (with the 2nd half's initialize), 2nd half + CFL
-sphx_status batch_substep(const BatchFluid &b);
-sphx_status batch_step_gate(const BatchFluid &b);
+// acoustic sub-step k: its dt and loop flag, 1st half (with the 2nd half's initialize), 2nd half + CFL
+sphx_status batch_substep(const BatchFluid &b, uint32_t k);
+sphx_status batch_step_gate(const BatchFluid &b, uint32_t substeps);
 sphx_status batch_position(const BatchFluid &b);
 
 // ---- batched configuration update (config_kernels.hip) ----
@@ -340,6 +359,7 @@ struct BatchConfig
     // cell lists: table, 256-particle map (as BatchFluid), 256-cell map over
     // ncells + 1, scan-tile map over ncells + 1
     const void *cll = nullptr;
+    size_t small_lds = 0; // every scene's list is updated by one workgroup with this much LDS (0: not)
     uint32_t n_scenes = 0;
     const uint32_t *map_particles = nullptr;
     uint32_t blocks_particles = 0;
@@ -364,6 +384,8 @@ size_t batch_cll_args_bytes();
 // cursor: ncells words, tile_sums: scan tiles of ncells + 1 (device, owned by the batch)
 void batch_cll_args(void *dst, sphx_cell_linked_list *cll, uint32_t *cursor, uint32_t *tile_sums);
 uint32_t batch_cll_tiles(const sphx_cell_linked_list *cll);
+// LDS of the one-workgroup update of a small scene's cell list (0: not small)
+size_t batch_cll_small(const sphx_cell_linked_list *cll);
 size_t batch_build_args_bytes();
 void batch_build_args(void *dst, sphx_relation *rel, unsigned long long *needed);
 size_t batch_stage_args_bytes();
@@ -374,10 +396,11 @@ sphx_status batch_relations(const BatchConfig &b);
 // ---- pieces of the advection step driver (sphx_api.hip) ----
 bool relation_ready(sphx_relation *r);
 sphx_status check_fluid_relations(sphx_relation *inner, sphx_relation *const *walls, int n_wall, bool need_built);
-// the device-side sub-step loop from the current step state until it ends;
-// the state is then in the context's pinned mirror
+// the device-side sub-step loop of an advection step, after its first `done`
+// sub-steps, until it ends; its state is then in the context's pinned mirror
 sphx_status advection_substeps(sphx_relation *inner, sphx_relation *const *walls, int n_wall,
-                               const sphx_advection_config *cfg, uint32_t batch);
+                               const sphx_advection_config *cfg, double time, uint32_t done, uint32_t batch,
+                               const unsigned long long **state);
 // position update, [ParticleSortCK], cell linked list, relations
 sphx_status advection_tail(sphx_relation *inner, sphx_relation *const *walls, int n_wall,
                            sphx_cell_linked_list *cll, bool sort_now);
