@@ -129,28 +129,8 @@ sphx_status alloc_dev(sphx_batch *b, T **p, size_t count)
     return SPHX_OK;
 }
 
-// the per-scene records of the scene, build and staging tables for the current shape
-void fill_records(sphx_batch *b)
-{
-    const size_t sa = batch_scene_args_bytes(b->P), ba = batch_build_args_bytes(), st = batch_stage_args_bytes();
-    unsigned long long *needed = b->readback + (size_t)b->scenes.size() * STEP_SLOTS;
-    for (size_t s = 0; s < b->scenes.size(); ++s)
-    {
-        sphx_batch::Scene &sc = b->scenes[s];
-        sc.staged = sc.inner->staged && sc.inner->source->n >= b->shape.stage_min;
-        batch_scene_args(b->scene_tab_h.data() + s * sa, sc.inner, sc.walls, sc.n_wall, &sc.cfg, b->time_d + s,
-                         sc.staged);
-        batch_stage_args(b->stage_tab_h.data() + s * st, sc.staged ? sc.inner : nullptr);
-        batch_build_args(b->build_tab_h.data() + (size_t)sc.rel0 * ba, sc.inner, needed + sc.rel0);
-        for (int k = 0; k < sc.n_wall; ++k)
-            batch_build_args(b->build_tab_h.data() + (size_t)(sc.rel0 + 1 + k) * ba, sc.walls[k],
-                             needed + sc.rel0 + 1 + k);
-    }
-    b->tables_dirty = true;
-}
-
 // scenes staged under the current shape whose staging sets are stale (their
-// lists were last rebuilt without them) get them rebuilt on their own stream
+// lists were rebuilt since) get them made on their own stream
 sphx_status refresh_staging(sphx_batch *b)
 {
     for (auto &sc : b->scenes)
@@ -161,6 +141,31 @@ sphx_status refresh_staging(sphx_batch *b)
                 return s;
             SPHX_HIP(hipStreamSynchronize(sc.inner->source->ctx->stream));
         }
+    return SPHX_OK;
+}
+
+// the per-scene records of the scene, build and staging tables for the current shape
+sphx_status fill_records(sphx_batch *b)
+{
+    const size_t sa = batch_scene_args_bytes(b->P), ba = batch_build_args_bytes(), st = batch_stage_args_bytes();
+    unsigned long long *needed = b->readback + (size_t)b->scenes.size() * STEP_SLOTS;
+    for (auto &sc : b->scenes)
+        sc.staged = sc.inner->staged && sc.inner->source->n >= b->shape.stage_min;
+    sphx_status status = refresh_staging(b); // the records hold the sets' addresses
+    if (status)
+        return status;
+    for (size_t s = 0; s < b->scenes.size(); ++s)
+    {
+        sphx_batch::Scene &sc = b->scenes[s];
+        batch_scene_args(b->scene_tab_h.data() + s * sa, sc.inner, sc.walls, sc.n_wall, &sc.cfg, b->time_d + s,
+                         sc.staged);
+        batch_stage_args(b->stage_tab_h.data() + s * st, sc.staged ? sc.inner : nullptr);
+        batch_build_args(b->build_tab_h.data() + (size_t)sc.rel0 * ba, sc.inner, needed + sc.rel0);
+        for (int k = 0; k < sc.n_wall; ++k)
+            batch_build_args(b->build_tab_h.data() + (size_t)(sc.rel0 + 1 + k) * ba, sc.walls[k],
+                             needed + sc.rel0 + 1 + k);
+    }
+    b->tables_dirty = true;
     return SPHX_OK;
 }
 
@@ -276,7 +281,8 @@ sphx_status build_tables(sphx_batch *b)
     b->scene_tab_h.assign(S * batch_scene_args_bytes(b->P), 0);
     b->build_tab_h.assign(R * batch_build_args_bytes(), 0);
     b->stage_tab_h.assign(S * batch_stage_args_bytes(), 0);
-    fill_records(b);
+    if ((st = fill_records(b)))
+        return st;
     b->tables = true;
     return upload_records(b);
 }
@@ -710,7 +716,8 @@ sphx_status sphx_batch_advection_step(sphx_batch *b, double *time, uint32_t *ste
             if (!(b->shape == b->candidates[b->next_candidate]))
             {
                 b->shape = b->candidates[b->next_candidate];
-                fill_records(b);
+                if ((s = fill_records(b)))
+                    return s;
             }
             timing = true;
         }
@@ -803,7 +810,8 @@ sphx_status sphx_batch_advection_step(sphx_batch *b, double *time, uint32_t *ste
     {
         for (auto &sc : b->scenes)
             SPHX_HIP(hipStreamSynchronize(sc.inner->source->ctx->stream));
-        fill_records(b);
+        if ((s = fill_records(b)))
+            return s;
     }
     if (timing)
     {
@@ -824,7 +832,8 @@ sphx_status sphx_batch_advection_step(sphx_batch *b, double *time, uint32_t *ste
             if (!(b->shape == b->candidates[best]))
             {
                 b->shape = b->candidates[best];
-                fill_records(b);
+                if ((s = fill_records(b)))
+                    return s;
             }
         }
     }

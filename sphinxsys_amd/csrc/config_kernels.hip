@@ -1513,21 +1513,116 @@ __global__ void k_chunk_stride(uint32_t *chunk, uint32_t nchunks, uint32_t strid
 }
 
 //---------------------------------------------------------------------------
-// gathers of the particle sort (UpdateSortableVariables,
-// base_configuration_dynamics.h:74-128): out[i] = in[perm[i]]
+// the particle sort's permutation (UpdateSortableVariables,
+// base_configuration_dynamics.h:74-128): every evolving variable by one kernel
+// into a scratch copy, out[i] = in[perm[i]], and by another one back to its
+// place, with the (x, y, z, Vol) records and SortedID made on the way.  A field at
+// a time (a gather and a copy each) the whole sort took 349 us for 989k particles
+// FP32-mixed in 3D and 167 for 90k, now 248 and 119.
 //---------------------------------------------------------------------------
-template <class E>
-__global__ void k_gather(const E *in, E *out, const uint32_t *perm, uint32_t n)
+template <class T>
+struct SortFields
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        out[i] = in[perm[i]];
+    static constexpr int kDoubles = 3, kReals = 11, kWords = 2;
+    uint32_t n;
+    const uint32_t *perm;
+    double *d[kDoubles];   // Position
+    T *t[kReals];          // Vol first, then the other evolving reals (null: not carried)
+    uint32_t *w[kWords];   // OriginalID first
+    Rec4<T> *vel;
+    double *d_tmp;         // n values per field, one after another
+    T *t_tmp;
+    uint32_t *w_tmp;
+    Rec4<T> *vel_tmp;
+    Rec4<T> *posvol;
+    Rec4<float> *pos_f32;
+    uint32_t *sorted_id;
+};
+
+template <class T>
+__global__ void __launch_bounds__(kThreads) k_sort_gather(SortFields<T> f)
+{
+    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+    if (i >= f.n)
+        return;
+    const uint32_t j = f.perm[i];
+#pragma unroll
+    for (int k = 0; k < SortFields<T>::kDoubles; ++k)
+        if (f.d[k])
+            f.d_tmp[(size_t)k * f.n + i] = f.d[k][j];
+#pragma unroll
+    for (int k = 0; k < SortFields<T>::kReals; ++k)
+        if (f.t[k])
+            f.t_tmp[(size_t)k * f.n + i] = f.t[k][j];
+#pragma unroll
+    for (int k = 0; k < SortFields<T>::kWords; ++k)
+        if (f.w[k])
+            f.w_tmp[(size_t)k * f.n + i] = f.w[k][j];
+    f.vel_tmp[i] = f.vel[j];
 }
-__global__ void k_sorted_id(const uint32_t *original_id, uint32_t *sorted_id, uint32_t n)
+template <int D, class T>
+__global__ void __launch_bounds__(kThreads) k_sort_store(SortFields<T> f)
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        sorted_id[original_id[i]] = i;
+    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+    if (i >= f.n)
+        return;
+    double x[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < D; ++k)
+        f.d[k][i] = x[k] = f.d_tmp[(size_t)k * f.n + i];
+    const T vol = f.t_tmp[i];
+#pragma unroll
+    for (int k = 0; k < SortFields<T>::kReals; ++k)
+        if (f.t[k])
+            f.t[k][i] = f.t_tmp[(size_t)k * f.n + i];
+    const uint32_t id = f.w_tmp[i];
+#pragma unroll
+    for (int k = 0; k < SortFields<T>::kWords; ++k)
+        if (f.w[k])
+            f.w[k][i] = f.w_tmp[(size_t)k * f.n + i];
+    f.vel[i] = f.vel_tmp[i];
+    const Rec4<T> r = D == 3 ? Rec4<T>{T(x[0]), T(x[1]), T(x[2]), vol} : Rec4<T>{T(x[0]), T(x[1]), vol, T(0)};
+    f.posvol[i] = r;
+    if (f.pos_f32 != (Rec4<float> *)f.posvol)
+        f.pos_f32[i] = Rec4<float>{(float)r.x, (float)r.y, D == 3 ? (float)r.z : 0.0f, 0.0f};
+    f.sorted_id[id] = i;
+}
+
+//---------------------------------------------------------------------------
+// The stable sort of a small body's keys in one workgroup: a bitonic network in
+// LDS over (key, index) as one 64-bit value, instead of a histogram, a scan and
+// a scatter per digit (the values are the indices, so equal keys keep their
+// order).  With the permutation above the sort takes 37 us for 800 particles in
+// 2D instead of 156, 57 for 3,200, 92 for 8,000; at 13,861 the digits take 114.
+//---------------------------------------------------------------------------
+constexpr uint32_t kSortSmall = 8192, kSortThreads = 1024;
+__global__ void __launch_bounds__(kSortThreads) k_sort_small(uint32_t *keys, uint32_t *vals, uint32_t n, uint32_t size)
+{
+    extern __shared__ unsigned long long sort_lds[];
+    const uint32_t t = threadIdx.x;
+    for (uint32_t k = t; k < size; k += kSortThreads)
+        sort_lds[k] = k < n ? (unsigned long long)keys[k] << 32 | vals[k] : ~0ull;
+    for (uint32_t len = 2; len <= size; len <<= 1)
+        for (uint32_t step = len >> 1; step > 0; step >>= 1)
+        {
+            __syncthreads();
+            for (uint32_t q = t; q < size / 2u; q += kSortThreads)
+            {
+                const uint32_t lo = 2u * (q & ~(step - 1u)) + (q & (step - 1u)), hi = lo + step;
+                const unsigned long long x = sort_lds[lo], y = sort_lds[hi];
+                if ((x > y) == ((lo & len) == 0u))
+                {
+                    sort_lds[lo] = y;
+                    sort_lds[hi] = x;
+                }
+            }
+        }
+    __syncthreads();
+    for (uint32_t k = t; k < n; k += kSortThreads)
+    {
+        keys[k] = (uint32_t)(sort_lds[k] >> 32);
+        vals[k] = (uint32_t)sort_lds[k];
+    }
 }
 } // namespace
 
@@ -1583,6 +1678,16 @@ sphx_status radix_sort_pairs(sphx_context *ctx, uint32_t *keys, uint32_t *vals, 
 {
     if (n <= 1 || bits <= 0)
         return SPHX_OK;
+    if (n <= kSortSmall)
+    {
+        uint32_t size = 2;
+        while (size < n)
+            size *= 2;
+        hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kSortThreads), size * sizeof(unsigned long long), ctx->stream,
+                           keys, vals, (uint32_t)n, size);
+        SPHX_HIP(hipGetLastError());
+        return SPHX_OK;
+    }
     sphx_status s;
     uint32_t ntiles = grid_for(n, kTile);
     size_t nhist = (size_t)kBuckets * ntiles;
@@ -1914,7 +2019,19 @@ sphx_status ensure_staged(sphx_relation *rel)
 {
     if (!rel->staged || !rel->stage_stale)
         return SPHX_OK;
-    sphx_status s = relation_stage(rel);
+    // their memory with the first use: a search without a time loop has none
+    hipStream_t stream = rel->source->ctx->stream;
+    const size_t nblocks = ((size_t)rel->source->n + kStageBlock - 1) / kStageBlock;
+    sphx_status s;
+    if (!rel->stage_count && (s = dev_alloc(stream, (void **)&rel->stage_count, nblocks * sizeof(uint32_t))))
+        return s;
+    if (!rel->stage_keys &&
+        (s = dev_alloc(stream, (void **)&rel->stage_keys, nblocks * kStageCap * sizeof(uint32_t))))
+        return s;
+    if (!rel->local_slice &&
+        (s = dev_alloc(stream, (void **)&rel->local_slice, rel->slice_capacity * sizeof(uint16_t))))
+        return s;
+    s = relation_stage(rel);
     if (!s)
         rel->stage_stale = false;
     return s;
@@ -1942,51 +2059,60 @@ sphx_status morton_sequence(sphx_body *b, sphx_cell_linked_list *cll)
     return radix_sort_pairs(ctx, b->sequence, b->perm, b->n, 3 * axis_bits);
 }
 
-template <class E>
-static sphx_status gather_into(sphx_context *ctx, E *field, const uint32_t *perm, uint32_t n)
+template <class T>
+static sphx_status sort_fields(sphx_body *b)
 {
-    sphx_status s = ctx->gather_tmp.reserve((size_t)n * sizeof(E));
+    sphx_context *ctx = b->ctx;
+    const uint32_t n = b->n;
+    SortFields<T> f{};
+    f.n = n;
+    f.perm = b->perm;
+    for (int k = 0; k < b->D; ++k)
+        f.d[k] = b->pos[k];
+    int nt = 0, nw = 0;
+    // Vol, ForcePrior, Mass, Compression, CompressionRate, VolumetricMeasureRef
+    for (void *p : {b->Vol, b->mass, b->C, b->dC, b->Vol_ref})
+        f.t[nt++] = (T *)p;
+    for (int k = 0; k < b->D; ++k)
+        f.t[nt++] = (T *)b->force_prior[k];
+    f.w[nw++] = b->original_id;
+    if (b->desc.kind == SPHX_BODY_FLUID)
+    {
+        // evolving once a free-surface indication exists (surface_indication_ck.hpp:43)
+        f.w[nw++] = (uint32_t *)b->prev_indicator;
+        // evolving with a viscous force (force_prior_ck.cpp:14)
+        for (int k = 0; k < b->D; ++k)
+            f.t[nt++] = (T *)b->prev_visc[k];
+    }
+    f.vel = (Rec4<T> *)b->vel;
+    f.posvol = (Rec4<T> *)b->posvol;
+    f.pos_f32 = b->pos_f32;
+    f.sorted_id = b->sorted_id;
+    const size_t vel_bytes = (size_t)n * sizeof(Rec4<T>), d_bytes = (size_t)n * 8 * b->D;
+    const size_t t_bytes = ((size_t)n * sizeof(T) * nt + 15) / 16 * 16;
+    sphx_status s = ctx->gather_tmp.reserve(vel_bytes + d_bytes + t_bytes + (size_t)n * 4 * nw);
     if (s)
         return s;
-    E *tmp = (E *)ctx->gather_tmp.ptr;
-    hipLaunchKernelGGL(k_gather<E>, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, field, tmp, perm, n);
+    unsigned char *tmp = (unsigned char *)ctx->gather_tmp.ptr;
+    f.vel_tmp = (Rec4<T> *)tmp;
+    f.d_tmp = (double *)(tmp + vel_bytes);
+    f.t_tmp = (T *)(tmp + vel_bytes + d_bytes);
+    f.w_tmp = (uint32_t *)(tmp + vel_bytes + d_bytes + t_bytes);
+    const dim3 g(grid_for(n, kThreads)), blk(kThreads);
+    hipLaunchKernelGGL(k_sort_gather<T>, g, blk, 0, ctx->stream, f);
+    if (b->D == 2)
+        hipLaunchKernelGGL((k_sort_store<2, T>), g, blk, 0, ctx->stream, f);
+    else
+        hipLaunchKernelGGL((k_sort_store<3, T>), g, blk, 0, ctx->stream, f);
     SPHX_HIP(hipGetLastError());
-    SPHX_HIP(hipMemcpyAsync(field, tmp, (size_t)n * sizeof(E), hipMemcpyDeviceToDevice, ctx->stream));
+    b->state_version++;
     return SPHX_OK;
 }
-
-sphx_status gather_u32(sphx_context *ctx, uint32_t *field, const uint32_t *perm, size_t n)
-{
-    return n ? gather_into(ctx, field, perm, (uint32_t)n) : SPHX_OK;
-}
-sphx_status gather_real(sphx_body *b, void **field, const uint32_t *perm)
+sphx_status sort_variables(sphx_body *b)
 {
     if (!b->n)
         return SPHX_OK;
-    if (b->P == P_FP64)
-        return gather_into(b->ctx, (double *)*field, perm, b->n);
-    return gather_into(b->ctx, (float *)*field, perm, b->n);
-}
-sphx_status gather_double(sphx_body *b, double **field, const uint32_t *perm)
-{
-    return b->n ? gather_into(b->ctx, *field, perm, b->n) : SPHX_OK;
-}
-sphx_status gather_rec4(sphx_body *b, void **field, const uint32_t *perm)
-{
-    if (!b->n)
-        return SPHX_OK;
-    if (b->P == P_FP64)
-        return gather_into(b->ctx, (Rec4<double> *)*field, perm, b->n);
-    return gather_into(b->ctx, (Rec4<float> *)*field, perm, b->n);
-}
-sphx_status sorted_id_update(sphx_body *b)
-{
-    if (!b->n)
-        return SPHX_OK;
-    hipLaunchKernelGGL(k_sorted_id, dim3(grid_for(b->n, 256)), dim3(256), 0, b->ctx->stream, b->original_id,
-                       b->sorted_id, b->n);
-    SPHX_HIP(hipGetLastError());
-    return SPHX_OK;
+    return b->P == P_FP64 ? sort_fields<double>(b) : sort_fields<float>(b);
 }
 } // namespace sphx
 

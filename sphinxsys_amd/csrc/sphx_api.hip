@@ -648,8 +648,6 @@ static sphx_status reserve_slices(sphx_relation *r, uint32_t kmax)
     sphx_status s;
     if ((s = dev_alloc(stream, (void **)&r->slice, need * sizeof(uint32_t))))
         return s;
-    if (r->staged && (s = dev_alloc(stream, (void **)&r->local_slice, need * sizeof(uint16_t))))
-        return s;
     r->slice_capacity = need;
     return SPHX_OK;
 }
@@ -1270,8 +1268,7 @@ static sphx_status relation_create(sphx_body *src, sphx_body *tar, sphx_cell_lin
         {
             if (!r)
                 return;
-            for (void *p : {(void *)r->neighbor_size, (void *)r->particle_offset, (void *)r->chunk_offset,
-                            (void *)r->stage_count, (void *)r->stage_keys, r->poly})
+            for (void *p : {(void *)r->neighbor_size, (void *)r->particle_offset, (void *)r->chunk_offset, r->poly})
                 if (p)
                     dev_free(s, p);
         }
@@ -1287,13 +1284,8 @@ static sphx_status relation_create(sphx_body *src, sphx_body *tar, sphx_cell_lin
     if (inner && src->desc.kind == SPHX_BODY_FLUID && src->n > 0 && split_lanes(src->D, src->P, src->n) == 1)
     {
         // LDS staging of the acoustic passes and the sums over the inner neighbours
-        const size_t nblocks = (src->n + kStageBlock - 1) / kStageBlock;
         r->staged = true;
         r->stage_cap = kStageCap;
-        sphx_status st;
-        if ((st = dev_alloc(stream, (void **)&r->stage_count, nblocks * sizeof(uint32_t))) ||
-            (st = dev_alloc(stream, (void **)&r->stage_keys, nblocks * kStageCap * sizeof(uint32_t))))
-            return st;
     }
     sphx_status s = build_kernel_poly(r.get());
     if (s)
@@ -1408,22 +1400,9 @@ sphx_status sphx_particle_sort(sphx_body *b, sphx_cell_linked_list *c)
     sphx_status s;
     if ((s = morton_sequence(b, c)))
         return s;
-    // UpdateSortableVariables over the evolving variables only
-    for (int k = 0; k < b->D; ++k)
-        if ((s = gather_double(b, &b->pos[k], b->perm)) || (s = gather_real(b, &b->force_prior[k], b->perm)))
-            return s;
-    if ((s = gather_real(b, &b->Vol, b->perm)) || (s = gather_u32(b->ctx, b->original_id, b->perm, b->n)) ||
-        (s = gather_rec4(b, &b->vel, b->perm)) || (s = gather_real(b, &b->mass, b->perm)) ||
-        (s = gather_real(b, &b->C, b->perm)) || (s = gather_real(b, &b->dC, b->perm)) ||
-        (s = gather_real(b, &b->Vol_ref, b->perm)) || (s = sorted_id_update(b)) || (s = refresh_posvol(b)))
+    // UpdateSortableVariables over the evolving variables only, SortedID
+    if ((s = sort_variables(b)))
         return s;
-    // evolving once a free-surface indication exists (surface_indication_ck.hpp:43)
-    if (b->desc.kind == SPHX_BODY_FLUID && (s = gather_u32(b->ctx, (uint32_t *)b->prev_indicator, b->perm, b->n)))
-        return s;
-    // evolving with a viscous force (force_prior_ck.cpp:14)
-    for (int k = 0; b->desc.kind == SPHX_BODY_FLUID && k < b->D; ++k)
-        if ((s = gather_real(b, &b->prev_visc[k], b->perm)))
-            return s;
     b->config_version++;
     return SPHX_OK;
 }

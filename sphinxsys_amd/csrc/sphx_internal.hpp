@@ -268,11 +268,8 @@ sphx_status ensure_staged(sphx_relation *rel);
 // per-cell flags of a target cell list: any particle within the search box
 sphx_status cell_near_flags(sphx_cell_linked_list *cll);
 sphx_status morton_sequence(sphx_body *b, sphx_cell_linked_list *cll);
-sphx_status gather_u32(sphx_context *ctx, uint32_t *field, const uint32_t *perm, size_t n);
-sphx_status gather_real(sphx_body *b, void **field, const uint32_t *perm);
-sphx_status gather_double(sphx_body *b, double **field, const uint32_t *perm);
-sphx_status gather_rec4(sphx_body *b, void **field, const uint32_t *perm);
-sphx_status sorted_id_update(sphx_body *b);
+// the evolving variables in the order of b->perm, with the records and SortedID that follow from them
+sphx_status sort_variables(sphx_body *b);
 sphx_status fill_iota(sphx_context *ctx, uint32_t *a, size_t n);
 
 // ---- fluid kernels (fluid_kernels.hip) ----
