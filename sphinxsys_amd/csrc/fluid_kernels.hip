@@ -1761,37 +1761,119 @@ __global__ void __launch_bounds__(kThreads) k_correction(FluidArgs<typename Prec
         }
 }
 
+// the staged correction matrices of a block's neighbours, as rows of four values
+// (a lane reads its neighbours' at random: 16-byte elements, then what is left)
+template <class T, int D>
+struct StagedMat
+{
+    static constexpr int kRows = D == 3 ? 2 : 1;                                    // of four values
+    static constexpr size_t kBytes = kRows * sizeof(Rec4<T>) + (D == 3 ? sizeof(T) : 0);
+    Rec4<T> *rows[kRows];
+    T *last;
+    __device__ __forceinline__ StagedMat(unsigned char *lds, uint32_t cap)
+    {
+        rows[0] = (Rec4<T> *)lds;
+        if constexpr (D == 3)
+            rows[1] = rows[0] + cap;
+        last = (T *)(rows[0] + kRows * cap);
+    }
+    __device__ __forceinline__ void put(uint32_t r, const Mat3<D, T> &B)
+    {
+        if constexpr (D == 3)
+        {
+            rows[0][r] = Rec4<T>{B.m[0][0], B.m[0][1], B.m[0][2], B.m[1][0]};
+            rows[1][r] = Rec4<T>{B.m[1][1], B.m[1][2], B.m[2][0], B.m[2][1]};
+            last[r] = B.m[2][2];
+        }
+        else
+            rows[0][r] = Rec4<T>{B.m[0][0], B.m[0][1], B.m[1][0], B.m[1][1]};
+    }
+    __device__ __forceinline__ Mat3<D, T> get(uint32_t r) const
+    {
+        Mat3<D, T> B;
+        const Rec4<T> x = rows[0][r];
+        if constexpr (D == 3)
+        {
+            const Rec4<T> y = rows[1][r];
+            B.m[0][0] = x.x, B.m[0][1] = x.y, B.m[0][2] = x.z, B.m[1][0] = x.w;
+            B.m[1][1] = y.x, B.m[1][2] = y.y, B.m[2][0] = y.z, B.m[2][1] = y.w;
+            B.m[2][2] = last[r];
+        }
+        else
+            B.m[0][0] = x.x, B.m[0][1] = x.y, B.m[1][0] = x.z, B.m[1][1] = x.w;
+        return B;
+    }
+};
+// LDS of the correction's neighbour sum: two blocks a CU in FP32-mixed 3D (52 B a
+// record); an FP64 record in 3D has 104 B, which would leave one block, and is
+// not staged
+template <int D, int P>
+constexpr bool kStageMat = P == P_MIXED || D == 2;
+template <int D, int P>
+constexpr size_t mat_lds()
+{
+    using T = typename Prec<P>::T;
+    return sum_cap<D, P>() * (StagedPV<T, D>::kBytes + StagedMat<T, D>::kBytes);
+}
+
 // grad_sum_i = sum_j B_j e_ij dW_ij V_j over the inner neighbours (the part of
-// the corrected pressure force that does not change within an advection step)
+// the corrected pressure force that does not change within an advection step).
+// From nine scattered loads per neighbour 416 us a launch for 512k particles
+// FP32-mixed in 3D, from staged records 87.
 template <int D, int P, int S>
 __global__ void __launch_bounds__(kThreads) k_correction_grad(FluidArgs<typename Prec<P>::T> a)
 {
     using T = typename Prec<P>::T;
     __shared__ PolyLDS<T> poly_in;
+    extern __shared__ __align__(32) unsigned char staged_lds[];
     stage_poly(poly_in, a.poly, true);
+    const uint32_t blk = xcd_block_index();
+    constexpr uint32_t kCap = sum_cap<D, P>();
+    StagedPV<T, D> s_pv(staged_lds, kCap);
+    StagedMat<T, D> s_mat(staged_lds + kCap * StagedPV<T, D>::kBytes, kCap);
+    const uint32_t n_staged = S == 1 && kStageMat<D, P> && a.stage_count ? a.stage_count[blk] : kStageOverflow;
+    const bool staged = n_staged <= kCap; // kStageOverflow is above any cap
+    if (staged)
+    {
+        const uint32_t *keys = a.stage_keys + (size_t)blk * a.stage_cap;
+        for (uint32_t r = threadIdx.x; r < n_staged; r += kThreads)
+        {
+            const uint32_t j = keys[r];
+            Mat3<D, T> B;
+            B.load(a.corr, j);
+            s_pv.put(r, a.posvol[j]);
+            s_mat.put(r, B);
+        }
+    }
     __syncthreads();
-    const Lanes<S> lane(xcd_block_index());
+    const Lanes<S> lane(blk);
     const uint32_t i = lane.i;
     if (i >= a.n)
         return;
     const PV<T, D> pi = load_pv<T, D>(a.posvol, i);
     const T x_per_r = a.poly->x_per_r;
     T gx = 0, gy = 0, gz = 0;
-    for_each_neighbor<S>(a.slice, a.chunk[i >> 6] + (i & 63u), a.count[i], lane.sub, [&](uint32_t j) {
-        const PV<T, D> pj = load_pv<T, D>(a.posvol, j);
+    auto add = [&](const PV<T, D> &pj, const Mat3<D, T> &Bj) {
         const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
-        const T r2 = D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy;
+        const T r2 = D == 3 ? dot3(dx, dx, dy, dy, dz, dz) : mad2(dx, dx, dy, dy);
         const T ir = inv_sqrt(r2);
         const T dWV = eval_poly(poly_in, r2 * ir, x_per_r) * pj.vol;
-        Mat3<D, T> Bj;
-        Bj.load(a.corr, j);
         T bx, by, bz;
         Bj.apply(dx * ir, dy * ir, D == 3 ? dz * ir : T(0), bx, by, bz);
-        gx += bx * dWV;
-        gy += by * dWV;
+        gx = fma(bx, dWV, gx);
+        gy = fma(by, dWV, gy);
         if (D == 3)
-            gz += bz * dWV;
-    });
+            gz = fma(bz, dWV, gz);
+    };
+    const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
+    if (staged)
+        for_each_neighbor(a.local_slice, nb, nc, 0u, [&](uint32_t r) { add(s_pv.get(r), s_mat.get(r)); });
+    else
+        for_each_neighbor<S>(a.slice, nb, nc, lane.sub, [&](uint32_t j) {
+            Mat3<D, T> Bj;
+            Bj.load(a.corr, j);
+            add(load_pv<T, D>(a.posvol, j), Bj);
+        });
     if constexpr (S > 1)
         gx = lane_sum<S>(gx), gy = lane_sum<S>(gy), gz = lane_sum<S>(gz);
     if (!lane.first())
@@ -1817,22 +1899,40 @@ __global__ void __launch_bounds__(kThreads) k_surface_div(FluidArgs<typename Pre
     stage_poly(poly_in, a.poly, true);
     for (int k = 0; k < a.n_wall; ++k)
         stage_poly(poly_w[k], a.wall[k].poly, true);
+    extern __shared__ __align__(32) unsigned char staged_lds[];
+    const uint32_t blk = xcd_block_index();
+    constexpr uint32_t kCap = sum_cap<D, P>();
+    StagedPV<T, D> s_pv(staged_lds, kCap);
+    const uint32_t n_staged = S == 1 && a.stage_count ? a.stage_count[blk] : kStageOverflow;
+    const bool staged = n_staged <= kCap; // kStageOverflow is above any cap
+    if (staged)
+    {
+        const uint32_t *keys = a.stage_keys + (size_t)blk * a.stage_cap;
+        for (uint32_t r = threadIdx.x; r < n_staged; r += kThreads)
+            s_pv.put(r, a.posvol[keys[r]]);
+    }
     __syncthreads();
-    const Lanes<S> lane(xcd_block_index());
+    const Lanes<S> lane(blk);
     const uint32_t i = lane.i;
     if (i >= a.n)
         return;
     const T threshold = T(0.75) * T(D);
     const PV<T, D> pi = load_pv<T, D>(a.posvol, i);
-    auto term = [&](const PV<T, D> &pj, const PolyLDS<T> &poly, T x_per_r) {
+    // sum -= dW V r
+    auto subtract = [&](T &sum, const PV<T, D> &pj, const PolyLDS<T> &poly, T x_per_r) {
         const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
-        const T r = sqrt(D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy);
-        return eval_poly(poly, r, x_per_r) * pj.vol * r;
+        const T r = sqrt(D == 3 ? dot3(dx, dx, dy, dy, dz, dz) : mad2(dx, dx, dy, dy));
+        sum = fma(-(eval_poly(poly, r, x_per_r) * pj.vol), r, sum);
     };
     const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
+    const T x_per_r = a.poly->x_per_r;
     T pos_div = 0;
-    for_each_neighbor<S>(a.slice, nb, nc, lane.sub,
-                         [&](uint32_t j) { pos_div -= term(load_pv<T, D>(a.posvol, j), poly_in, a.poly->x_per_r); });
+    if (staged)
+        for_each_neighbor(a.local_slice, nb, nc, 0u,
+                          [&](uint32_t r) { subtract(pos_div, s_pv.get(r), poly_in, x_per_r); });
+    else
+        for_each_neighbor<S>(a.slice, nb, nc, lane.sub,
+                             [&](uint32_t j) { subtract(pos_div, load_pv<T, D>(a.posvol, j), poly_in, x_per_r); });
     if constexpr (S > 1)
         pos_div = lane_sum<S>(pos_div);
     if (pos_div < threshold && a.prev_indicator[i] != 1)
@@ -1851,7 +1951,7 @@ __global__ void __launch_bounds__(kThreads) k_surface_div(FluidArgs<typename Pre
         const uint32_t mb = w.chunk[i >> 6] + (i & 63u), mc = w.count[i];
         T wall_div = 0;
         for (uint32_t k2 = lane.sub; k2 < mc; k2 += S)
-            wall_div -= term(load_pv<T, D>(w.posvol, w.slice[mb + (k2 << 6)]), poly_w[k], w.poly->x_per_r);
+            subtract(wall_div, load_pv<T, D>(w.posvol, w.slice[mb + (k2 << 6)]), poly_w[k], w.poly->x_per_r);
         if constexpr (S > 1)
             wall_div = lane_sum<S>(wall_div);
         pos_div += wall_div;
@@ -1866,7 +1966,25 @@ template <int D, int P, int S>
 __global__ void __launch_bounds__(kThreads) k_surface_update(FluidArgs<typename Prec<P>::T> a)
 {
     using T = typename Prec<P>::T;
-    const Lanes<S> lane(xcd_block_index());
+    extern __shared__ __align__(32) unsigned char staged_lds[];
+    const uint32_t blk = xcd_block_index();
+    constexpr uint32_t kCap = pass1_cap<D, P>();
+    StagedPV<T, D> s_pv(staged_lds, kCap);
+    T *s_div = (T *)(staged_lds + kCap * StagedPV<T, D>::kBytes);
+    const uint32_t n_staged = S == 1 && a.stage_count ? a.stage_count[blk] : kStageOverflow;
+    const bool staged = n_staged <= kCap; // kStageOverflow is above any cap
+    if (staged)
+    {
+        const uint32_t *keys = a.stage_keys + (size_t)blk * a.stage_cap;
+        for (uint32_t r = threadIdx.x; r < n_staged; r += kThreads)
+        {
+            const uint32_t j = keys[r];
+            s_pv.put(r, a.posvol[j]);
+            s_div[r] = a.pos_div[j];
+        }
+    }
+    __syncthreads();
+    const Lanes<S> lane(blk);
     const uint32_t i = lane.i;
     if (i >= a.n)
         return;
@@ -1876,12 +1994,17 @@ __global__ void __launch_bounds__(kThreads) k_surface_update(FluidArgs<typename 
     {
         const PV<T, D> pi = load_pv<T, D>(a.posvol, i);
         uint32_t very_near_surface = 0;
-        for_each_neighbor<S>(a.slice, a.chunk[i >> 6] + (i & 63u), a.count[i], lane.sub, [&](uint32_t j) {
-            const PV<T, D> pj = load_pv<T, D>(a.posvol, j);
+        auto test = [&](const PV<T, D> &pj, T div) {
             const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
-            const T r = sqrt(D == 3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy);
-            very_near_surface |= (a.pos_div[j] < threshold) & (r < a.h) ? 1u : 0u;
-        });
+            const T r = sqrt(D == 3 ? dot3(dx, dx, dy, dy, dz, dz) : mad2(dx, dx, dy, dy));
+            very_near_surface |= (div < threshold) & (r < a.h) ? 1u : 0u;
+        };
+        const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
+        if (staged)
+            for_each_neighbor(a.local_slice, nb, nc, 0u, [&](uint32_t r) { test(s_pv.get(r), s_div[r]); });
+        else
+            for_each_neighbor<S>(a.slice, nb, nc, lane.sub,
+                                 [&](uint32_t j) { test(load_pv<T, D>(a.posvol, j), a.pos_div[j]); });
         if constexpr (S > 1)
             very_near_surface = lane_sum<S>(very_near_surface);
         if (!very_near_surface)
@@ -2910,7 +3033,9 @@ struct CorrectionGradL
         attach_relations(a, inner, nullptr, 0);
         with_tree_lanes<D, P>(b->n, [&](auto lanes) {
             constexpr int S = lanes.value;
-            hipLaunchKernelGGL((k_correction_grad<D, P, S>), dim3(grid_for(b->n, kThreads / S)), dim3(kThreads), 0,
+            const size_t lds = kStageMat<D, P> && a.stage_count ? mat_lds<D, P>() : 0;
+            allow_lds(k_correction_grad<D, P, S>, lds);
+            hipLaunchKernelGGL((k_correction_grad<D, P, S>), dim3(grid_for(b->n, kThreads / S)), dim3(kThreads), lds,
                                b->ctx->stream, a);
         });
         LAUNCH_CHECK();
@@ -3208,8 +3333,10 @@ struct SurfaceL
         with_tree_lanes<D, P>(b->n, [&](auto lanes) {
             constexpr int S = lanes.value;
             const dim3 g(grid_for(b->n, kThreads / S)), blk(kThreads);
-            hipLaunchKernelGGL((k_surface_div<D, P, S>), g, blk, 0, b->ctx->stream, a);
-            hipLaunchKernelGGL((k_surface_update<D, P, S>), g, blk, 0, b->ctx->stream, a);
+            const size_t lds = a.stage_count ? sum_lds<D, P>() : 0, lds_update = a.stage_count ? pass1_lds<D, P>() : 0;
+            allow_lds(k_surface_div<D, P, S>, lds);
+            hipLaunchKernelGGL((k_surface_div<D, P, S>), g, blk, lds, b->ctx->stream, a);
+            hipLaunchKernelGGL((k_surface_update<D, P, S>), g, blk, lds_update, b->ctx->stream, a);
         });
         LAUNCH_CHECK();
         return SPHX_OK;
@@ -3218,6 +3345,9 @@ struct SurfaceL
 
 sphx_status free_surface_indication(sphx_relation *inner, sphx_relation *const *c, int nc)
 {
+    sphx_status s = ensure_staged(inner);
+    if (s)
+        return s;
     ProfileScope prof(inner->source->ctx, "surface_indication");
     return dispatch<SurfaceL>(inner->source, inner, c, nc);
 }

@@ -36,7 +36,10 @@ def test_fp64_sums_staged_and_not(hip, oracle, dim, m, window):
     pr.write("Velocity", rng.normal(scale=0.3, size=(n, dim)))
     pr.both(lambda s: ck.CompressionSummation(s["inner"], *s["walls"]).exec())
     pr.both(lambda s: ck.LinearCorrectionMatrixComplex(s["inner"], *s["walls"], alpha=0.5).exec())
-    names = ["CompressionSummation", "LinearCorrectionMatrix"]
+    pr.both(lambda s: ck.FreeSurfaceIndicationComplexSpatialTemporalCK(s["inner"], *s["walls"]).exec())
+    g, c = pr.read("Indicator")
+    assert np.array_equal(g, c)
+    names = ["CompressionSummation", "LinearCorrectionMatrix", "PositionDivergence"]
     for correction in (capi.CORRECTION_NONE, capi.CORRECTION_LINEAR):
         pr.both(lambda s: ck.AcousticStep1stHalf(s["inner"], *s["walls"], correction=correction).exec(2e-5))
         pr.both(lambda s: ck.AcousticStep2ndHalf(s["inner"], *s["walls"], correction=correction).exec(2e-5))
