@@ -457,8 +457,10 @@ __device__ __forceinline__ void walk_pipelined(const I *entries, uint32_t base, 
                                                const PV<T, D> &pi, const PolyLDS<T> &lds, T x_per_r,
                                                Fetch &&fetch, Late &&late, Pair &&pair)
 {
-    // pairs per batch: 8 in double; 6 is faster for the FP32-mixed passes: pass 2
-    // spills at 8 under its register cap, pass 1 at 6 fits five waves per SIMD
+    // pairs per batch: 8 in double, 4 where several lanes share a particle (short
+    // lists, more waves: 90,000 particles in 3D 45 + 58 -> 43 + 54 us); 6 is faster
+    // for the FP32-mixed passes: pass 2 spills at 8 under its register cap, pass 1
+    // at 6 fits five waves per SIMD
     constexpr uint32_t kBatch = KB;
     const uint32_t nbatch = (count + kBatch - 1) / kBatch;
     uint32_t next[kBatch];
@@ -900,7 +902,7 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
     auto pair = [&](const Rec &rj, const PairGeo<T> &g) { add(term(rj, g)); };
     const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
     auto no_late = [](uint32_t, Rec &) {};
-    constexpr uint32_t kWalkBatch = P == P_MIXED ? 6u : 8u;
+    constexpr uint32_t kWalkBatch = P == P_MIXED ? 6u : S > 1 ? 4u : 8u;
     auto global_rec = [&](uint32_t j) { return Rec{load_pv<T, D>(a.posvol, j), a.p[j]}; };
     if constexpr (kOrdered<T, S>)
         sum_terms<T, S>(
@@ -1361,7 +1363,7 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
         // whole records up front: loading the velocities late (as pass 1 loads
         // its pressures) makes this pass spill under its register cap
         auto no_late = [](uint32_t, Rec &) {};
-        constexpr uint32_t kWalkBatch = P == P_MIXED ? 6u : 8u;
+        constexpr uint32_t kWalkBatch = P == P_MIXED ? 6u : S > 1 ? 4u : 8u;
         auto global_rec = [&](uint32_t j) { return Rec{load_pv<T, D>(a.posvol, j), a.vel[j]}; };
         if constexpr (TRAV)
             trav_walk(*trav, tl, a.posvol, i, pi, poly_in, x_per_r, t_pv, t_j, trav_cols, trav_cols + kTravCols,
