@@ -403,7 +403,7 @@ sphx_status sphx_batch_tuning(const sphx_batch *batch, char *json, size_t capaci
  * "relation_build" (tiled list build of inner relations), "relation_build_contact"
  * (tiled list build of contact relations), "relation_scan" (per-lane scan build,
  * used when a list outgrows the LDS tile), "relation_stage" (LDS staging sets
- * of the FP32-mixed inner relation), "cell_linked_list", "particle_sort",
+ * of an inner relation), "cell_linked_list", "particle_sort",
  * "time_step_reduce", "state_update", "linear_correction" (correction matrix and
  * its neighbour sum), "surface_indication".  Reading synchronises the stream and
  * returns the accumulated milliseconds and launch count since enabling.

@@ -221,7 +221,6 @@ struct sphx_relation
     uint32_t *stage_count = nullptr;
     uint32_t *stage_keys = nullptr;
     uint16_t *local_slice = nullptr;
-    size_t local_capacity = 0;
     bool built = false;
     uint64_t builds = 0;                  // completed list builds
     uint64_t built_version = 0, target_version = 0; // config versions the lists were built for

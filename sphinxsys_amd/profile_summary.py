@@ -34,7 +34,8 @@ import sys
 SIMDS = 256 * 4          # MI355X: 256 CUs of 4 SIMDs
 CLOCK_HZ = 2.4e9         # peak engine clock
 COPY_BYTES = 1 << 30     # bench.py copy calibration: 1 GiB device-to-device copies
-STAGES = {"acoustic_pass1": r"k_pass1<3, 1, true, true, false>", "acoustic_pass2": r"k_pass2<3, 1, true, true, false>"}
+# (the fields after the flags, where there are any, are the lanes per particle)
+STAGES = {"acoustic_pass1": "k_pass1<3, 1, true, true, false", "acoustic_pass2": "k_pass2<3, 1, true, true, false"}
 
 
 def short_name(name):
@@ -217,7 +218,7 @@ def summarize(args):
               f"{valu} | {hit} | {rd / 1e6 if rd is not None else float('nan'):,.0f} | "
               f"{wr / 1e6 if wr is not None else float('nan'):,.0f} | {gbs} |")
             for stage, pat in STAGES.items():
-                if k == pat and rd is not None and wr is not None:
+                if k in (pat + ">", pat + ", 1>") and rd is not None and wr is not None:
                     traffic[stage] = rd + wr
         if traffic:
             w("\nPer-launch HBM bytes of the acoustic passes (read by bench.py):\n")
