@@ -2019,7 +2019,7 @@ sphx_status ensure_staged(sphx_relation *rel)
 {
     if (!rel->staged || !rel->stage_stale)
         return SPHX_OK;
-    // their memory with the first use: a search without a time loop has none
+    // their memory with the first use: an FP64 search without a time loop has none
     hipStream_t stream = rel->source->ctx->stream;
     const size_t nblocks = ((size_t)rel->source->n + kStageBlock - 1) / kStageBlock;
     sphx_status s;

@@ -713,13 +713,17 @@ static sphx_status update_relations(sphx_relation *const *rels, int count)
             sphx_relation *r = rels[k];
             r->kmax = work[k].kmax;
             r->slice_total = ((size_t)r->source->n + 63) / 64 * work[k].kmax * 64;
-            r->stage_stale = true; // the staging sets follow with the first dynamics that reads the lists often
+            r->stage_stale = true;
             r->csr_valid = false;  // the CSR view (offsets and indices) is built when read
             r->built = true;
             r->builds++;
             r->built_version = r->source->config_version;
             r->target_version = r->target->config_version;
         }
+        // FP32-mixed: every dynamics over the inner neighbours reads the sets
+        for (int k = 0; k < count; ++k)
+            if (rels[k]->source->P == P_MIXED && (s = ensure_staged(rels[k])))
+                return s;
         return SPHX_OK;
     }
     set_error("neighbour lists did not fit after growing the slice width");
@@ -747,7 +751,9 @@ sphx_status advection_tail(sphx_relation *inner, sphx_relation *const *walls, in
         if (!c->built || c->built_version != c->body->config_version)
             return state_error("target cell linked list not updated since the last configuration change");
     }
-    return update_relations(rels, 1 + n_wall);
+    if ((s = update_relations(rels, 1 + n_wall)))
+        return s;
+    return ensure_staged(inner); // for the next step's summation and passes
 }
 } // namespace sphx
 

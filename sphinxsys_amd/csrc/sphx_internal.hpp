@@ -258,11 +258,10 @@ void relation_prefilter(const sphx_relation *rel, float *thr_lo, float *thr_hi, 
 sphx_status relation_build(sphx_relation *rel, uint32_t kmax, unsigned long long *needed, bool scan);
 // the LDS staging sets of a staged relation, from its finished slices
 sphx_status relation_stage(sphx_relation *rel);
-// the same where they are stale.  Made by the first acoustic half step,
-// correction matrix or whole advection step after a list build, not by the
-// build: a density summation alone (a neighbour search without a time loop)
-// gains less from the sets than they cost (2.1M particles FP32-mixed, sort,
-// lists and summation: 3.48 -> 3.34 ms without them)
+// the same where they are stale.  In FP32-mixed the list build makes them (left
+// to the first reader, a density summation without them takes 3.27 ms instead
+// of 1.19 for 16.8M particles), in FP64 the end of an advection step or else the
+// first dynamics that gains from them: not a density summation alone
 sphx_status ensure_staged(sphx_relation *rel);
 // per-cell flags of a target cell list: any particle within the search box
 sphx_status cell_near_flags(sphx_cell_linked_list *cll);

@@ -51,8 +51,8 @@ def test_fp64_sums_staged_and_not(hip, oracle, dim, m, window):
 
 @pytest.mark.parametrize("precision", [capi.FP64, capi.MIXED])
 def test_lists_rebuilt_between_batch_steps(hip, precision):
-    """A caller that rebuilds a scene's lists between two batch steps leaves their
-    staging sets to the next reader: the batched scene still equals itself alone."""
+    """A caller that rebuilds a scene's lists between two batch steps may leave
+    their staging sets (FP64) to the next reader: the batched scene still equals itself alone."""
     geom = cases.dambreak_2d(dp=0.0038)  # 138,000 particles: staged in both precisions
     alone, batched = (cases.DamBreak(hip, geom, precision) for _ in range(2))
     for sc in (alone, batched):
