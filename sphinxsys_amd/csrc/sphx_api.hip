@@ -390,8 +390,8 @@ sphx_status transfer_rows(sphx_body *b, const FieldComponents<E> &f, H *host, bo
         return st;
     const size_t per = kStagingHalf / row, chunks = (n + per - 1) / per;
     auto rows_of = [&](size_t k) { return std::min(per, n - k * per); };
-    // the kernels of a half end before the host touches it, and the last before
-    // the buffer is given back (also on an error)
+    // the kernels of a half end before the host touches it, and on an error the
+    // last before the buffer is given back
     struct Wait
     {
         hipStream_t s;
@@ -430,6 +430,7 @@ sphx_status transfer_rows(sphx_body *b, const FieldComponents<E> &f, H *host, bo
             copy_host(host + (k - 1) * per * K, half[(k - 1) & 1], rows_of(k - 1) * row);
         }
     }
+    SPHX_HIP(hipStreamSynchronize(s)); // a failed kernel of a write is reported here
     return SPHX_OK;
 }
 

@@ -1,0 +1,168 @@
+// host_errors_check.cpp -- the host side of the HIP library on a stand-in for
+// the HIP runtime: memory is host memory, kernels do not run, and a named call
+// fails on demand.  The program's own HIP functions come before the runtime's
+// when the library given on the command line is loaded, so nothing here needs
+// or touches a GPU.  What the host paths do with an error, and which launches
+// they issue on which device, is checked without making a GPU fail.
+//
+//   host_errors_check LIBRARY CASE
+//
+// Prints the first check that does not hold and returns 1, otherwise returns 0.
+#include "../../include/sphx.h"
+
+#include <hip/hip_runtime_api.h>
+
+#include <dlfcn.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+#include <vector>
+
+namespace
+{
+struct Stream
+{
+    int device;
+};
+int g_device = 0;            // the calling thread's current device
+int g_sync_error = 0;        // stream synchronizations that fail from now on
+int g_uploads = 0;           // host-to-device copies
+int g_other_device = 0;      // launches on a stream of a device that is not current
+int g_captures = 0;          // stream captures begun
+std::map<const void *, std::string> g_names;
+std::map<std::string, int> g_launches; // kernel -> launches
+dim3 g_grid, g_block;
+size_t g_lds;
+hipStream_t g_stream;
+} // namespace
+
+#define OK(...)                                                                                                  \
+    {                                                                                                            \
+        __VA_ARGS__;                                                                                             \
+        return hipSuccess;                                                                                       \
+    }
+extern "C" {
+void **__hipRegisterFatBinary(const void *) { return new void *(nullptr); }
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *, void *, dim3 *,
+                           dim3 *, int *)
+{
+    g_names[host] = name;
+}
+void __hipRegisterVar(void **, void *, char *, const char *, int, size_t, int, int) {}
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s)
+    OK(g_grid = g; g_block = b; g_lds = lds; g_stream = s)
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t *s)
+    OK(*g = g_grid; *b = g_block; *lds = g_lds; *s = g_stream)
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3, void **, size_t, hipStream_t s)
+{
+    if (g.x == 0)
+        return hipErrorInvalidConfiguration;
+    ++g_launches[g_names[f]];
+    if (((Stream *)s)->device != g_device)
+        ++g_other_device;
+    return hipSuccess;
+}
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) OK()
+hipError_t hipGetLastError(void) OK()
+const char *hipGetErrorString(hipError_t) { return "the stand-in's error"; }
+hipError_t hipGetDeviceCount(int *n) OK(*n = 2)
+hipError_t hipSetDevice(int d) OK(g_device = d)
+hipError_t hipGetSymbolAddress(void **p, const void *) OK(*p = std::calloc(1, 64))
+hipError_t hipMalloc(void **p, size_t n) OK(*p = std::calloc(1, n))
+hipError_t hipFree(void *p) OK(std::free(p))
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) OK(*p = std::calloc(1, n))
+hipError_t hipHostFree(void *p) OK(std::free(p))
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t)
+    OK(std::memcpy(d, s, n); g_uploads += k == hipMemcpyHostToDevice)
+hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) OK(std::memset(d, v, n))
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) OK(*s = (hipStream_t) new Stream{g_device})
+hipError_t hipStreamDestroy(hipStream_t s) OK(delete (Stream *)s)
+hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t *d) OK(*d = ((Stream *)s)->device)
+hipError_t hipStreamSynchronize(hipStream_t) { return g_sync_error ? hipErrorLaunchFailure : hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t *e) OK(*e = (hipEvent_t)std::calloc(1, 8))
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) OK(*e = (hipEvent_t)std::calloc(1, 8))
+hipError_t hipEventDestroy(hipEvent_t e) OK(std::free(e))
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) OK()
+hipError_t hipEventSynchronize(hipEvent_t) OK()
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) OK(*ms = 1.0f)
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) OK(++g_captures)
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) OK(*g = (hipGraph_t)std::calloc(1, 8))
+hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t)
+    OK(*e = (hipGraphExec_t)std::calloc(1, 8))
+hipError_t hipGraphDestroy(hipGraph_t g) OK(std::free(g))
+hipError_t hipGraphExecDestroy(hipGraphExec_t e) OK(std::free(e))
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) OK()
+}
+
+namespace
+{
+void *g_lib;
+#define API(name) ((decltype(&name))dlsym(g_lib, #name))
+
+#define REQUIRE(cond)                                                                                            \
+    do                                                                                                           \
+    {                                                                                                            \
+        if (!(cond))                                                                                             \
+        {                                                                                                        \
+            std::printf("line %d: %s (%s)\n", __LINE__, #cond, API(sphx_last_error)());                          \
+            std::exit(1);                                                                                        \
+        }                                                                                                        \
+    } while (0)
+
+// a fluid body of n particles with its cell list and inner relation, built
+struct Scene
+{
+    sphx_context *ctx = nullptr;
+    sphx_body *body = nullptr;
+    sphx_cell_linked_list *cll = nullptr;
+    sphx_relation *inner = nullptr;
+
+    Scene(int device, int dim, int precision, uint32_t n)
+    {
+        REQUIRE(API(sphx_context_create)(device, &ctx) == SPHX_OK);
+        sphx_body_desc d{};
+        d.dim = dim;
+        d.precision = precision;
+        d.kind = SPHX_BODY_FLUID;
+        d.n_particles = n;
+        d.spacing_ref = 0.01;
+        d.h_spacing_ratio = 1.3;
+        d.rho0 = 1.0;
+        d.c0 = 10.0;
+        REQUIRE(API(sphx_body_create)(ctx, &d, &body) == SPHX_OK);
+        const double lo[3] = {0, 0, 0}, up[3] = {1, 1, 1};
+        REQUIRE(API(sphx_cell_linked_list_create)(body, lo, up, 0.026, 2, &cll) == SPHX_OK);
+        REQUIRE(API(sphx_relation_create_inner)(body, cll, &inner) == SPHX_OK);
+        REQUIRE(API(sphx_update_cell_linked_list)(cll) == SPHX_OK);
+        REQUIRE(API(sphx_update_relation)(inner) == SPHX_OK);
+    }
+};
+
+// a large write whose kernels fail says so
+void large_write()
+{
+    Scene s(0, 2, SPHX_FP64, 100000);
+    std::vector<double> v(100000, 1.0);
+    REQUIRE(API(sphx_body_write)(s.body, SPHX_FIELD_PRESSURE, v.data(), v.size()) == SPHX_OK);
+    g_sync_error = 1;
+    REQUIRE(API(sphx_body_write)(s.body, SPHX_FIELD_PRESSURE, v.data(), v.size()) == SPHX_E_HIP);
+    g_sync_error = 0;
+    REQUIRE(API(sphx_body_write)(s.body, SPHX_FIELD_PRESSURE, v.data(), v.size()) == SPHX_OK);
+}
+} // namespace
+
+int main(int argc, char **argv)
+{
+    const std::map<std::string, void (*)()> cases = {{"large_write", large_write}};
+    if (argc != 3 || !cases.count(argv[2]) || !(g_lib = dlopen(argv[1], RTLD_NOW)))
+    {
+        std::printf("usage: %s LIBRARY CASE\n", argv[0]);
+        return 2;
+    }
+    cases.at(argv[2])();
+    return 0;
+}
