@@ -144,7 +144,9 @@ sphx_status refresh_staging(sphx_batch *b)
     return SPHX_OK;
 }
 
-// the per-scene records of the scene, build and staging tables for the current shape
+// The per-scene records of the scene, build and staging tables for the current
+// shape.  Where the staging sets cannot be made the tables are given up (the
+// scenes' `staged` is already the new shape's) and the next step makes them anew.
 sphx_status fill_records(sphx_batch *b)
 {
     const size_t sa = batch_scene_args_bytes(b->P), ba = batch_build_args_bytes(), st = batch_stage_args_bytes();
@@ -153,7 +155,10 @@ sphx_status fill_records(sphx_batch *b)
         sc.staged = sc.inner->staged && sc.inner->source->n >= b->shape.stage_min;
     sphx_status status = refresh_staging(b); // the records hold the sets' addresses
     if (status)
+    {
+        free_tables(b);
         return status;
+    }
     for (size_t s = 0; s < b->scenes.size(); ++s)
     {
         sphx_batch::Scene &sc = b->scenes[s];
@@ -603,9 +608,7 @@ sphx_status sphx_batch_set_options(sphx_batch *b, const sphx_batch_options *o)
     b->opt = *o;
     b->shape = Shape{o->tile_waves, o->stage_min};
     tuning_candidates(b);
-    if (b->tables)
-        fill_records(b);
-    return SPHX_OK;
+    return b->tables ? fill_records(b) : SPHX_OK;
 }
 
 sphx_status sphx_batch_add_scene(sphx_batch *b, sphx_relation *inner, sphx_relation *const *walls, int n_wall,

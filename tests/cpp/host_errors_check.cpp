@@ -37,6 +37,15 @@ std::map<std::string, int> g_launches; // kernel -> launches
 dim3 g_grid, g_block;
 size_t g_lds;
 hipStream_t g_stream;
+
+int launches(const char *kernel)
+{
+    int n = 0;
+    for (const auto &k : g_launches)
+        if (k.first.find(kernel) != std::string::npos)
+            n += k.second;
+    return n;
+}
 } // namespace
 
 #define OK(...)                                                                                                  \
@@ -153,11 +162,40 @@ void large_write()
     g_sync_error = 0;
     REQUIRE(API(sphx_body_write)(s.body, SPHX_FIELD_PRESSURE, v.data(), v.size()) == SPHX_OK);
 }
+
+// A batch whose options are changed between two steps: an error of the staging
+// sets that the new options ask for is the call's, and the next step makes the
+// batch's tables anew instead of going on with half of them
+void options_error()
+{
+    Scene s(0, 3, SPHX_MIXED, 5000);
+    sphx_batch *batch = nullptr;
+    sphx_advection_config cfg{1.0, 0.25, 0.6, SPHX_RIEMANN_ACOUSTIC, SPHX_FLOW_FREE_SURFACE, 0, 0, 0.0, 0};
+    sphx_batch_options o{0, 0, 1, 1u << 30, 1};
+    REQUIRE(API(sphx_batch_create)(0, &batch) == SPHX_OK);
+    REQUIRE(API(sphx_batch_set_options)(batch, &o) == SPHX_OK);
+    REQUIRE(API(sphx_batch_add_scene)(batch, s.inner, nullptr, 0, s.cll, &cfg) == SPHX_OK);
+    double t = 0.0;
+    for (int k = 0; k < 2; ++k)
+    {
+        g_uploads = 0;
+        REQUIRE(API(sphx_batch_advection_step)(batch, &t, nullptr, nullptr, nullptr) == SPHX_OK);
+    }
+    REQUIRE(g_uploads == 2 && launches("kb_stage_sets") == 0); // times and sort flags
+    o.stage_min = 0;
+    g_sync_error = 1;
+    REQUIRE(API(sphx_batch_set_options)(batch, &o) == SPHX_E_HIP);
+    g_sync_error = 0;
+    g_uploads = 0;
+    REQUIRE(API(sphx_batch_advection_step)(batch, &t, nullptr, nullptr, nullptr) == SPHX_OK);
+    REQUIRE(g_uploads > 2 && launches("kb_stage_sets") == 1);
+    REQUIRE(API(sphx_batch_destroy)(batch) == SPHX_OK);
+}
 } // namespace
 
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> cases = {{"large_write", large_write}};
+    const std::map<std::string, void (*)()> cases = {{"large_write", large_write}, {"options_error", options_error}};
     if (argc != 3 || !cases.count(argv[2]) || !(g_lib = dlopen(argv[1], RTLD_NOW)))
     {
         std::printf("usage: %s LIBRARY CASE\n", argv[0]);
