@@ -605,6 +605,7 @@ sphx_status sphx_batch_set_options(sphx_batch *b, const sphx_batch_options *o)
         return batch_error(SPHX_E_ARG, "null argument");
     if (o->tile_waves != 1 && o->tile_waves != 2 && o->tile_waves != 4)
         return batch_error(SPHX_E_ARG, "tile_waves must be 1, 2 or 4");
+    SPHX_HIP(hipSetDevice(b->device));
     b->opt = *o;
     b->shape = Shape{o->tile_waves, o->stage_min};
     tuning_candidates(b);

@@ -191,11 +191,34 @@ void options_error()
     REQUIRE(g_uploads > 2 && launches("kb_stage_sets") == 1);
     REQUIRE(API(sphx_batch_destroy)(batch) == SPHX_OK);
 }
+
+// Options changed by a thread whose current device is another than the batch's:
+// the staging sets are made on the batch's
+void options_device()
+{
+    Scene s(1, 3, SPHX_MIXED, 5000);
+    sphx_batch *batch = nullptr;
+    sphx_advection_config cfg{1.0, 0.25, 0.6, SPHX_RIEMANN_ACOUSTIC, SPHX_FLOW_FREE_SURFACE, 0, 0, 0.0, 0};
+    sphx_batch_options o{0, 0, 1, 1u << 30, 1};
+    REQUIRE(API(sphx_batch_create)(1, &batch) == SPHX_OK);
+    REQUIRE(API(sphx_batch_set_options)(batch, &o) == SPHX_OK);
+    REQUIRE(API(sphx_batch_add_scene)(batch, s.inner, nullptr, 0, s.cll, &cfg) == SPHX_OK);
+    double t = 0.0;
+    REQUIRE(API(sphx_batch_advection_step)(batch, &t, nullptr, nullptr, nullptr) == SPHX_OK);
+    REQUIRE(g_other_device == 0);
+    const int before = launches("k_stage_sets");
+    o.stage_min = 0;
+    g_device = 0;
+    REQUIRE(API(sphx_batch_set_options)(batch, &o) == SPHX_OK);
+    REQUIRE(launches("k_stage_sets") == before + 1 && g_other_device == 0);
+    REQUIRE(API(sphx_batch_destroy)(batch) == SPHX_OK);
+}
 } // namespace
 
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> cases = {{"large_write", large_write}, {"options_error", options_error}};
+    const std::map<std::string, void (*)()> cases = {
+        {"large_write", large_write}, {"options_error", options_error}, {"options_device", options_device}};
     if (argc != 3 || !cases.count(argv[2]) || !(g_lib = dlopen(argv[1], RTLD_NOW)))
     {
         std::printf("usage: %s LIBRARY CASE\n", argv[0]);
