@@ -52,9 +52,13 @@ struct sphx_batch
         sphx_cell_linked_list *cll = nullptr;
         sphx_advection_config cfg{};
         uint32_t last = 0;     // sub-steps of the previous step
+        sphx_relation *relation(int r) const { return r == 0 ? inner : walls[r - 1]; } // 0..n_wall
         bool failed = false;   // diverged: stays without advancing
         bool staged = false;   // passes from LDS-staged records under the current shape
         uint32_t rel0 = 0;     // index of its inner relation in the relation table
+        // its relations' lists that the records hold the addresses of
+        const uint32_t *slice[kMaxRelations] = {};
+        uint32_t kmax[kMaxRelations] = {};
     };
     std::vector<Scene> scenes;
     uint32_t n_rel = 0;
@@ -165,12 +169,26 @@ sphx_status fill_records(sphx_batch *b)
         batch_scene_args(b->scene_tab_h.data() + s * sa, sc.inner, sc.walls, sc.n_wall, &sc.cfg, b->time_d + s,
                          sc.staged);
         batch_stage_args(b->stage_tab_h.data() + s * st, sc.staged ? sc.inner : nullptr);
-        batch_build_args(b->build_tab_h.data() + (size_t)sc.rel0 * ba, sc.inner, needed + sc.rel0);
-        for (int k = 0; k < sc.n_wall; ++k)
-            batch_build_args(b->build_tab_h.data() + (size_t)(sc.rel0 + 1 + k) * ba, sc.walls[k],
-                             needed + sc.rel0 + 1 + k);
+        for (int r = 0; r <= sc.n_wall; ++r)
+        {
+            sphx_relation *rel = sc.relation(r);
+            batch_build_args(b->build_tab_h.data() + (size_t)(sc.rel0 + r) * ba, rel, needed + sc.rel0 + r);
+            sc.slice[r] = rel->slice;
+            sc.kmax[r] = rel->kmax;
+        }
     }
     b->tables_dirty = true;
+    return SPHX_OK;
+}
+
+// the records again where a caller rebuilt a scene's lists between two steps and
+// they outgrew their memory
+sphx_status renew_records(sphx_batch *b)
+{
+    for (const auto &sc : b->scenes)
+        for (int r = 0; r <= sc.n_wall; ++r)
+            if (sc.slice[r] != sc.relation(r)->slice || sc.kmax[r] != sc.relation(r)->kmax)
+                return fill_records(b);
     return SPHX_OK;
 }
 
@@ -488,7 +506,7 @@ sphx_status finish_device_tail(sphx_batch *b, sphx_batch::Scene &sc, bool *regro
     const unsigned long long *needed = b->readback_h + b->scenes.size() * STEP_SLOTS;
     for (int r = 0; r <= sc.n_wall; ++r)
     {
-        sphx_relation *rel = r == 0 ? sc.inner : sc.walls[r - 1];
+        sphx_relation *rel = sc.relation(r);
         if (needed[sc.rel0 + r] > rel->kmax)
         {
             sphx_status s = sphx_update_relation(rel); // grows the width (or takes the scan build) and rebuilds
@@ -711,6 +729,8 @@ sphx_status sphx_batch_advection_step(sphx_batch *b, double *time, uint32_t *ste
         if ((s = build_tables(b)))
             return s;
     }
+    else if ((s = renew_records(b)))
+        return s;
     // the tuning step's shape
     bool timing = false;
     if (b->opt.autotune && !b->tuned && b->steps > 0 && b->opt.use_graph)

@@ -32,6 +32,7 @@ int g_sync_error = 0;        // stream synchronizations that fail from now on
 int g_uploads = 0;           // host-to-device copies
 int g_other_device = 0;      // launches on a stream of a device that is not current
 int g_captures = 0;          // stream captures begun
+unsigned long long g_needed = 0; // what the next read of a single device word returns
 std::map<const void *, std::string> g_names;
 std::map<std::string, int> g_launches; // kernel -> launches
 dim3 g_grid, g_block;
@@ -86,7 +87,16 @@ hipError_t hipFree(void *p) OK(std::free(p))
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) OK(*p = std::calloc(1, n))
 hipError_t hipHostFree(void *p) OK(std::free(p))
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t)
-    OK(std::memcpy(d, s, n); g_uploads += k == hipMemcpyHostToDevice)
+{
+    std::memcpy(d, s, n);
+    g_uploads += k == hipMemcpyHostToDevice;
+    if (k == hipMemcpyDeviceToHost && n == sizeof(g_needed) && g_needed)
+    {
+        std::memcpy(d, &g_needed, n);
+        g_needed = 0;
+    }
+    return hipSuccess;
+}
 hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) OK(std::memset(d, v, n))
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) OK(*s = (hipStream_t) new Stream{g_device})
 hipError_t hipStreamDestroy(hipStream_t s) OK(delete (Stream *)s)
@@ -213,12 +223,40 @@ void options_device()
     REQUIRE(launches("k_stage_sets") == before + 1 && g_other_device == 0);
     REQUIRE(API(sphx_batch_destroy)(batch) == SPHX_OK);
 }
+
+// A caller that rebuilds a scene's lists between two batch steps and finds more
+// neighbours than before: the lists get new memory, and the next step's tables
+// hold its address
+void regrown_lists()
+{
+    Scene s(0, 3, SPHX_FP64, 5000);
+    sphx_batch *batch = nullptr;
+    sphx_advection_config cfg{1.0, 0.25, 0.6, SPHX_RIEMANN_ACOUSTIC, SPHX_FLOW_FREE_SURFACE, 0, 0, 0.0, 0};
+    sphx_batch_options o{0, 0, 1, 0, 1};
+    REQUIRE(API(sphx_batch_create)(0, &batch) == SPHX_OK);
+    REQUIRE(API(sphx_batch_set_options)(batch, &o) == SPHX_OK);
+    REQUIRE(API(sphx_batch_add_scene)(batch, s.inner, nullptr, 0, s.cll, &cfg) == SPHX_OK);
+    double t = 0.0;
+    REQUIRE(API(sphx_batch_advection_step)(batch, &t, nullptr, nullptr, nullptr) == SPHX_OK);
+    REQUIRE(API(sphx_update_relation)(s.inner) == SPHX_OK); // as wide as before
+    g_uploads = 0;
+    REQUIRE(API(sphx_batch_advection_step)(batch, &t, nullptr, nullptr, nullptr) == SPHX_OK);
+    REQUIRE(g_uploads == 2); // times and sort flags
+    g_needed = 200;
+    REQUIRE(API(sphx_update_relation)(s.inner) == SPHX_OK);
+    REQUIRE(g_needed == 0);
+    g_uploads = 0;
+    REQUIRE(API(sphx_batch_advection_step)(batch, &t, nullptr, nullptr, nullptr) == SPHX_OK);
+    REQUIRE(g_uploads == 5); // and the three tables
+    REQUIRE(API(sphx_batch_destroy)(batch) == SPHX_OK);
+}
 } // namespace
 
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
-        {"large_write", large_write}, {"options_error", options_error}, {"options_device", options_device}};
+        {"large_write", large_write}, {"options_error", options_error}, {"options_device", options_device},
+        {"regrown_lists", regrown_lists}};
     if (argc != 3 || !cases.count(argv[2]) || !(g_lib = dlopen(argv[1], RTLD_NOW)))
     {
         std::printf("usage: %s LIBRARY CASE\n", argv[0]);

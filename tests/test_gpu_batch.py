@@ -216,3 +216,38 @@ def test_batch_3d_unstaged_bit_identical_to_staged_alone(hip):
         batch.close()
         alone.close()
         other.close()
+
+
+@pytest.mark.parametrize("precision", [capi.FP64, capi.MIXED])
+def test_lists_regrown_by_the_caller_between_batch_steps(hip, precision):
+    """A caller that moves particles closer together between two batch steps and
+    rebuilds the lists, which outgrow their width: the batched scene stays
+    bit-identical to itself alone."""
+    spec = specs_small(count=1, seed=16)[0]
+    alone, batched = (make(hip, spec, precision) for _ in range(2))
+    batch = ck.BatchAdvection(hip, [batched.advection], options=dict(use_graph=1, autotune=0))
+    try:
+        for s in range(4):
+            if s == 2:
+                for sc in (alone, batched):
+                    x = sc.fluid.read("Position")
+                    near = np.argsort(np.linalg.norm(x - x[len(x) // 2], axis=1))[:60]
+                    x[near] = x[near[0]] + 0.7 * (x[near] - x[near[0]])
+                    sc.fluid.write("Position", x)
+                    for name in ("Mass", "VolumetricMeasure", "VolumetricMeasureRef"):  # as dense as before
+                        v = sc.fluid.read(name)
+                        v[near] *= 0.49
+                        sc.fluid.write(name, v)
+                    sc.fluid_cell_linked_list.exec()
+                    sc.complex_relation.exec()
+                    sc.ctx.synchronize()
+                    widest = sc.inner.read()[0].max()
+                    assert widest > 32, widest  # the width of a 2D list at first
+            alone.advection_step()
+            batch.exec()
+        for k in FIELDS:
+            assert np.array_equal(alone.fluid.read(k), batched.fluid.read(k)), k
+    finally:
+        batch.close()
+        alone.close()
+        batched.close()
