@@ -367,7 +367,9 @@ typedef struct sphx_batch_options {
                                0: the same launches issued directly every step          */
     int autotune;           /* 1 (default): time the shape candidates over the first
                                steps and keep the fastest; 0: use the fields below     */
-    int tile_waves;         /* waves per workgroup of the tiled neighbour build: 1, 2, 4 */
+    int tile_waves;         /* 64-particle chunks per workgroup of the tiled neighbour build:
+                               2 or 4 with one wave each, 1 with one wave or, in a batch of
+                               few chunks, with four                                    */
     uint32_t stage_min;     /* scenes with at least this many fluid particles run the
                                acoustic passes from LDS-staged neighbour records       */
     uint32_t substep_margin;/* captured sub-steps beyond the last step's largest count */

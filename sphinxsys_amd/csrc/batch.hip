@@ -362,8 +362,6 @@ BatchConfig config_launch(sphx_batch *b)
     const int w = wave_slot(b->shape.tile_waves);
     c.map_chunks = b->map_chunks[w];
     c.blocks_chunks = b->blocks_chunks[w];
-    c.split_chunks = b->map_chunks[0];
-    c.blocks_single = b->blocks_chunks[0];
     c.rel_scene = b->rel_scene;
     c.needed = b->readback + b->scenes.size() * STEP_SLOTS;
     c.tile_waves = b->shape.tile_waves;

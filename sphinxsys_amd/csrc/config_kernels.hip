@@ -2207,10 +2207,10 @@ sphx_status batch_cell_linked_list(const BatchConfig &b)
     return SPHX_OK;
 }
 
-template <int D, int W>
+template <int D, int W, int V = 1>
 static void launch_batch_tile(const BatchConfig &b)
 {
-    hipLaunchKernelGGL((kb_relation_tile<D, W>), dim3(b.blocks_chunks), dim3(W * 64), 0, b.stream,
+    hipLaunchKernelGGL((kb_relation_tile<D, W, V>), dim3(b.blocks_chunks), dim3(W * V * 64), 0, b.stream,
                        (const BuildArgs *)b.build, b.map_chunks, b.rel_scene, b.gate);
 }
 
@@ -2223,16 +2223,8 @@ sphx_status batch_relations(const BatchConfig &b)
         set_error("tiled relation build: 1, 2 or 4 waves per workgroup");
         return SPHX_E_ARG;
     }
-    if (b.split_chunks && tile_split(b.blocks_single))
-    {
-        const dim3 g(b.blocks_single), blk(kTileSplit * 64);
-        if (b.D == 2)
-            hipLaunchKernelGGL((kb_relation_tile<2, 1, kTileSplit>), g, blk, 0, b.stream, (const BuildArgs *)b.build,
-                               b.split_chunks, b.rel_scene, b.gate);
-        else
-            hipLaunchKernelGGL((kb_relation_tile<3, 1, kTileSplit>), g, blk, 0, b.stream, (const BuildArgs *)b.build,
-                               b.split_chunks, b.rel_scene, b.gate);
-    }
+    if (w == 1 && tile_split(b.blocks_chunks))
+        b.D == 2 ? launch_batch_tile<2, 1, kTileSplit>(b) : launch_batch_tile<3, 1, kTileSplit>(b);
     else if (b.D == 2)
         w == 1 ? launch_batch_tile<2, 1>(b) : w == 2 ? launch_batch_tile<2, 2>(b) : launch_batch_tile<2, 4>(b);
     else

@@ -367,11 +367,9 @@ struct BatchConfig
     uint32_t n_rel = 0;
     const uint32_t *map_chunks = nullptr;
     uint32_t blocks_chunks = 0;
-    const uint32_t *split_chunks = nullptr; // the map of one chunk per workgroup and its length
-    uint32_t blocks_single = 0;
     const uint32_t *rel_scene = nullptr;
     unsigned long long *needed = nullptr; // per relation, zeroed here before the build
-    int tile_waves = 1;                   // waves per workgroup of the tiled build (1, 2 or 4)
+    int tile_waves = 1;                   // chunks per workgroup of the tiled build (1, 2 or 4)
     // staging: table per scene (n_src 0: not staged), 256-particle map
     const void *stage = nullptr;
 };

@@ -250,13 +250,36 @@ void regrown_lists()
     REQUIRE(g_uploads == 5); // and the three tables
     REQUIRE(API(sphx_batch_destroy)(batch) == SPHX_OK);
 }
+
+// Each value of tile_waves is a build of its own: for the few chunks of this
+// batch four waves on one chunk, or two or four chunks with one wave each
+void tile_waves()
+{
+    const char *kernel[] = {"kb_relation_tileILi2ELi1ELi4E", "kb_relation_tileILi2ELi2ELi1E",
+                            "kb_relation_tileILi2ELi4ELi1E"};
+    for (int k = 0; k < 3; ++k)
+    {
+        Scene s(0, 2, SPHX_MIXED, 5000);
+        sphx_batch *batch = nullptr;
+        sphx_advection_config cfg{1.0, 0.25, 0.6, SPHX_RIEMANN_ACOUSTIC, SPHX_FLOW_FREE_SURFACE, 0, 0, 0.0, 0};
+        sphx_batch_options o{0, 0, 1 << k, 0, 1};
+        REQUIRE(API(sphx_batch_create)(0, &batch) == SPHX_OK);
+        REQUIRE(API(sphx_batch_set_options)(batch, &o) == SPHX_OK);
+        REQUIRE(API(sphx_batch_add_scene)(batch, s.inner, nullptr, 0, s.cll, &cfg) == SPHX_OK);
+        double t = 0.0;
+        g_launches.clear();
+        REQUIRE(API(sphx_batch_advection_step)(batch, &t, nullptr, nullptr, nullptr) == SPHX_OK);
+        REQUIRE(launches("kb_relation_tile") == 1 && launches(kernel[k]) == 1);
+        REQUIRE(API(sphx_batch_destroy)(batch) == SPHX_OK);
+    }
+}
 } // namespace
 
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
         {"large_write", large_write}, {"options_error", options_error}, {"options_device", options_device},
-        {"regrown_lists", regrown_lists}};
+        {"regrown_lists", regrown_lists}, {"tile_waves", tile_waves}};
     if (argc != 3 || !cases.count(argv[2]) || !(g_lib = dlopen(argv[1], RTLD_NOW)))
     {
         std::printf("usage: %s LIBRARY CASE\n", argv[0]);
