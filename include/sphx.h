@@ -349,7 +349,8 @@ sphx_status sphx_advection_step(sphx_relation *inner, sphx_relation *const *wall
  * more, whose neighbour lists outgrow their width, or that sorts this step is
  * finished by the host through the single-scene path.  An autotuner times
  * launch-shape candidates over the first steps (results do not depend on the
- * shape) and keeps the fastest; sphx_batch_tuning reports what it measured.
+ * shape) and keeps the fastest; candidates with the same launches are timed
+ * once and share the cost; sphx_batch_tuning reports what it measured.
  *
  * Every scene is a fluid body with its inner relation, 0..4 wall contact
  * relations and its cell linked list, built and initialised as for
@@ -370,8 +371,11 @@ typedef struct sphx_batch_options {
     int tile_waves;         /* 64-particle chunks per workgroup of the tiled neighbour build:
                                2 or 4 with one wave each, 1 with one wave or, in a batch of
                                few chunks, with four                                    */
-    uint32_t stage_min;     /* scenes with at least this many fluid particles run the
-                               acoustic passes from LDS-staged neighbour records       */
+    uint32_t stage_min;     /* of the scenes whose bodies run one lane per particle, those
+                               with at least this many fluid particles run the neighbour
+                               sums from LDS-staged records.  FP32-mixed 3D bodies and
+                               large ones do; smaller ones share a particle among lanes
+                               and are not staged, whatever this says                  */
     uint32_t substep_margin;/* captured sub-steps beyond the last step's largest count */
 } sphx_batch_options;
 

@@ -133,6 +133,13 @@ sphx_status alloc_dev(sphx_batch *b, T **p, size_t count)
     return SPHX_OK;
 }
 
+// whether a scene runs its passes from staged records under a shape (a relation
+// has staging sets only where its body runs one lane per particle)
+bool staged_under(const sphx_batch::Scene &sc, const Shape &shape)
+{
+    return sc.inner->staged && sc.inner->source->n >= shape.stage_min;
+}
+
 // scenes staged under the current shape whose staging sets are stale (their
 // lists were rebuilt since) get them made on their own stream
 sphx_status refresh_staging(sphx_batch *b)
@@ -156,7 +163,7 @@ sphx_status fill_records(sphx_batch *b)
     const size_t sa = batch_scene_args_bytes(b->P), ba = batch_build_args_bytes(), st = batch_stage_args_bytes();
     unsigned long long *needed = b->readback + (size_t)b->scenes.size() * STEP_SLOTS;
     for (auto &sc : b->scenes)
-        sc.staged = sc.inner->staged && sc.inner->source->n >= b->shape.stage_min;
+        sc.staged = staged_under(sc, b->shape);
     sphx_status status = refresh_staging(b); // the records hold the sets' addresses
     if (status)
     {
@@ -533,11 +540,51 @@ void tuning_candidates(sphx_batch *b)
     b->tuned = !b->opt.autotune;
     if (!b->opt.autotune)
         return;
-    // which scenes are staged (all, from 4096, 16384 or 65536 fluid particles;
-    // larger scenes always are, as in the single-scene path, whose 3D passes
-    // depend on it), then the tiled build's waves per workgroup for the best
+    // which of the scenes that have staging sets use them (all, from 4096, 16384 or
+    // 65536 fluid particles; larger scenes always do, as in the single-scene path,
+    // whose 3D passes depend on it), then the tiled build's chunks per workgroup
+    // for the best
     for (uint32_t smin : {0u, 4096u, 16384u, 65536u})
         b->candidates.push_back(Shape{1, smin});
+}
+
+// The cost of the next candidate.  After the four staging rules come the best
+// one's builds, after those the fastest shape of all is the batch's.
+sphx_status record_cost(sphx_batch *b, double cost)
+{
+    b->cost.push_back(cost);
+    b->next_candidate++;
+    const size_t best = (size_t)(std::min_element(b->cost.begin(), b->cost.end()) - b->cost.begin());
+    const Shape shape = b->candidates[best];
+    if (b->next_candidate == 4 && b->candidates.size() == 4)
+    {
+        b->candidates.push_back(Shape{2, shape.stage_min});
+        b->candidates.push_back(Shape{4, shape.stage_min});
+    }
+    if (b->next_candidate < b->candidates.size())
+        return SPHX_OK;
+    b->tuned = true;
+    if (b->shape == shape)
+        return SPHX_OK;
+    b->shape = shape;
+    return fill_records(b);
+}
+
+// A timed candidate that issues the launches of the next one for the present
+// scenes (-1: none): a step under the next one would capture and time them again.
+int same_launches(const sphx_batch *b)
+{
+    const Shape &next = b->candidates[b->next_candidate];
+    for (size_t k = 0; k < b->next_candidate; ++k)
+    {
+        const Shape &timed = b->candidates[k];
+        bool same = timed.tile_waves == next.tile_waves;
+        for (size_t s = 0; s < b->scenes.size() && same; ++s)
+            same = staged_under(b->scenes[s], timed) == staged_under(b->scenes[s], next);
+        if (same)
+            return (int)k;
+    }
+    return -1;
 }
 
 std::string shape_json(const Shape &s)
@@ -837,27 +884,11 @@ sphx_status sphx_batch_advection_step(sphx_batch *b, double *time, uint32_t *ste
     }
     if (timing)
     {
-        b->cost.push_back(particle_substeps > 0.0 ? 1e6 * ms / particle_substeps : 1e30);
-        b->next_candidate++;
-        if (b->next_candidate == 4 && b->candidates.size() == 4)
-        {
-            // best staging rule, then the build's waves per workgroup
-            const size_t best = (size_t)(std::min_element(b->cost.begin(), b->cost.end()) - b->cost.begin());
-            const uint32_t smin = b->candidates[best].stage_min;
-            b->candidates.push_back(Shape{2, smin});
-            b->candidates.push_back(Shape{4, smin});
-        }
-        if (b->next_candidate >= b->candidates.size())
-        {
-            const size_t best = (size_t)(std::min_element(b->cost.begin(), b->cost.end()) - b->cost.begin());
-            b->tuned = true;
-            if (!(b->shape == b->candidates[best]))
-            {
-                b->shape = b->candidates[best];
-                if ((s = fill_records(b)))
-                    return s;
-            }
-        }
+        s = record_cost(b, particle_substeps > 0.0 ? 1e6 * ms / particle_substeps : 1e30);
+        for (int k; !s && !b->tuned && (k = same_launches(b)) >= 0;)
+            s = record_cost(b, b->cost[k]);
+        if (s)
+            return s;
     }
     if (s = upload_records(b); s)
         return s;

@@ -251,3 +251,29 @@ def test_lists_regrown_by_the_caller_between_batch_steps(hip, precision):
         batch.close()
         alone.close()
         batched.close()
+
+
+def test_tuner_times_the_same_launches_once(hip):
+    """No small 2D scene is staged, so the four staging rules are one launch
+    shape with one measured cost; every 3D FP32-mixed scene may be, so rules that
+    part scenes of 3,400 to 90,000 particles differently are measured apart."""
+    specs = specs_small(count=6, seed=17)
+    _, st, tuning = run_batched(hip, specs, capi.MIXED, 5)
+    costs = [c["ms_per_million_particle_substeps"] for c in tuning["candidates"]]
+    print(f"2D: {tuning}", flush=True)
+    assert (st == 0).all() and tuning["tuned"] and len(set(costs[:4])) == 1 and len(set(costs)) == 3
+    scenes = [cases.DamBreak(hip, cases.dambreak_3d(dp=dp), capi.MIXED) for dp in (0.06, 0.04, 0.025, 0.02)]
+    for sc in scenes:
+        sc.initialize()
+    batch = ck.BatchAdvection(hip, [sc.advection for sc in scenes])
+    try:
+        for _ in range(8):
+            batch.exec()
+        tuning = batch.tuning()
+        print(f"3D, {[sc.fluid.n for sc in scenes]} particles: {tuning}", flush=True)
+        # (six measurements, of which two may agree to the printed digits)
+        assert tuning["tuned"] and len(set(c["ms_per_million_particle_substeps"] for c in tuning["candidates"])) >= 5
+    finally:
+        batch.close()
+        for sc in scenes:
+            sc.close()
