@@ -2545,19 +2545,44 @@ __global__ void k_fill_u64(unsigned long long *p, size_t n, unsigned long long v
         p[i] = v;
 }
 
-// Interpolation<Contact<Real>>::interact (interpolation_dynamics.hpp:46-60).
-// One wave per observer, its neighbours over the lanes: a program has a few
-// probes, so the time is the latency of one observer's list.  The lanes' kernels
-// and values go through LDS and every lane adds them in list order, so the sums
-// are those of one thread walking the list, which took 44 us for the two probes
-// of a 90k-particle 3D tank: five advection steps and their probes take 6.33 ms
-// instead of 6.55.
-template <int D, class T>
-__global__ void __launch_bounds__(64) k_interpolate(const Rec4<T> *obs, const Rec4<T> *tar, const T *data,
-                                                    uint32_t stride, const uint32_t *chunk, const uint32_t *count,
-                                                    const uint32_t *slice, const KernelPoly<T> *poly, T *out)
+// Interpolation<Contact<Real>>::interact (interpolation_dynamics.hpp:46-60):
+// the kernel, volume and value of observer pi's neighbour j
+template <class T>
+struct InterpTerm
 {
-    __shared__ T s_W[64], s_vol[64], s_value[64];
+    T W, vol, value;
+};
+template <int D, class T>
+__device__ __forceinline__ InterpTerm<T> interp_term(const PV<T, D> &pi, const Rec4<T> *tar, const T *data,
+                                                     uint32_t stride, uint32_t j, const KernelPoly<T> *poly)
+{
+    const PV<T, D> pj = load_pv<T, D>(tar, j);
+    const T value = data[(size_t)j * stride];
+    const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
+    const T r2 = D == 3 ? dot3(dx, dx, dy, dy, dz, dz) : mad2(dx, dx, dy, dy);
+    const T x = sqrt(r2) * poly->x_per_r;
+    const int loc = min((int)x, kPolyIntervals - 1);
+    const T f = frac_part(x);
+    const T *c = poly->w[loc];
+    return {((c[3] * f + c[2]) * f + c[1]) * f + c[0], pj.vol, value};
+}
+// the sums, in list order in both kernels
+template <class T>
+__device__ __forceinline__ void interp_add(const InterpTerm<T> &t, T &q, T &w)
+{
+    q = fma(t.W * t.vol, t.value, q);
+    w = fma(t.W, t.vol, w);
+}
+
+// A few observers (a case's probes): one wave each, its neighbours over the
+// lanes, as the time is the latency of one observer's list.  The lanes' terms go
+// through LDS and every lane adds them.
+template <int D, class T>
+__global__ void __launch_bounds__(64) k_interpolate_wave(const Rec4<T> *obs, const Rec4<T> *tar, const T *data,
+                                                         uint32_t stride, const uint32_t *chunk, const uint32_t *count,
+                                                         const uint32_t *slice, const KernelPoly<T> *poly, T *out)
+{
+    __shared__ InterpTerm<T> term[64];
     const uint32_t i = blockIdx.x, lane = threadIdx.x;
     const PV<T, D> pi = load_pv<T, D>(obs, i);
     T q = 0, w = 0;
@@ -2566,31 +2591,32 @@ __global__ void __launch_bounds__(64) k_interpolate(const Rec4<T> *obs, const Re
     {
         const uint32_t m = min(64u, nc - k0);
         if (lane < m)
-        {
-            const uint32_t j = slice[nb + ((k0 + lane) << 6)];
-            const PV<T, D> pj = load_pv<T, D>(tar, j);
-            const T value = data[(size_t)j * stride];
-            const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = D == 3 ? pi.z - pj.z : T(0);
-            const T r2 = D == 3 ? dot3(dx, dx, dy, dy, dz, dz) : mad2(dx, dx, dy, dy);
-            const T x = sqrt(r2) * poly->x_per_r;
-            const int loc = min((int)x, kPolyIntervals - 1);
-            const T f = frac_part(x);
-            const T *c = poly->w[loc];
-            const T W = ((c[3] * f + c[2]) * f + c[1]) * f + c[0];
-            s_W[lane] = W;
-            s_vol[lane] = pj.vol;
-            s_value[lane] = value;
-        }
+            term[lane] = interp_term<D>(pi, tar, data, stride, slice[nb + ((k0 + lane) << 6)], poly);
         __syncthreads();
         for (uint32_t k = 0; k < m; ++k)
-        {
-            q = fma(s_W[k] * s_vol[k], s_value[k], q);
-            w = fma(s_W[k], s_vol[k], w);
-        }
+            interp_add(term[k], q, w);
         __syncthreads();
     }
     if (lane == 0)
         out[i] = q / (w + T(2.71051e-20));
+}
+
+// Many observers: one thread each; the lists' rows are read whole
+template <int D, class T>
+__global__ void __launch_bounds__(64) k_interpolate(const Rec4<T> *obs, uint32_t n_obs, const Rec4<T> *tar,
+                                                    const T *data, uint32_t stride, const uint32_t *chunk,
+                                                    const uint32_t *count, const uint32_t *slice,
+                                                    const KernelPoly<T> *poly, T *out)
+{
+    const uint32_t i = blockIdx.x * 64u + threadIdx.x;
+    if (i >= n_obs)
+        return;
+    const PV<T, D> pi = load_pv<T, D>(obs, i);
+    T q = 0, w = 0;
+    const uint32_t nb = chunk[i >> 6] + (i & 63u), nc = count[i];
+    for (uint32_t k = 0; k < nc; ++k)
+        interp_add(interp_term<D>(pi, tar, data, stride, slice[nb + (k << 6)], poly), q, w);
+    out[i] = q / (w + T(2.71051e-20));
 }
 
 //---------------------------------------------------------------------------
@@ -3426,6 +3452,12 @@ struct EnergyL
 };
 sphx_status mechanical_energy(sphx_body *b, const double *g, double *out) { return dispatch<EnergyL>(b, g, out); }
 
+// Observers up to which each takes a wave, with one thread each beyond.  The
+// call, wave / thread: 2 observers in 3D FP64 18 / 40 us, 4,096 26 / 57, 16,384
+// 48 / 80, 32,768 74 / 74, 65,536 127 / 113, 262,144 481 / 231, 1,000,000 1,570 /
+// 777 (the waves' lanes read a slice a line per entry, the threads whole rows).
+// In 2D they cross at 20,000 to 30,000, in 3D FP32-mixed at 100,000.
+constexpr uint32_t kWaveObservers = 32768;
 template <int D, int P>
 struct InterpL
 {
@@ -3441,10 +3473,15 @@ struct InterpL
                         : field == SPHX_FIELD_VELOCITY ? (const T *)t->vel + component
                                                        : (const T *)t->C;
         const uint32_t stride = field == SPHX_FIELD_VELOCITY ? 4u : 1u;
-        hipLaunchKernelGGL((k_interpolate<D, T>), dim3(o->n), dim3(64), 0, o->ctx->stream,
-                           (const Rec4<T> *)o->posvol, (const Rec4<T> *)t->posvol, data, stride,
-                           rel->chunk_offset, rel->neighbor_size, rel->slice, (const KernelPoly<T> *)rel->poly,
-                           (T *)o->interp);
+        if (o->n <= kWaveObservers)
+            hipLaunchKernelGGL((k_interpolate_wave<D, T>), dim3(o->n), dim3(64), 0, o->ctx->stream,
+                               (const Rec4<T> *)o->posvol, (const Rec4<T> *)t->posvol, data, stride, rel->chunk_offset,
+                               rel->neighbor_size, rel->slice, (const KernelPoly<T> *)rel->poly, (T *)o->interp);
+        else
+            hipLaunchKernelGGL((k_interpolate<D, T>), dim3(grid_for(o->n, 64)), dim3(64), 0, o->ctx->stream,
+                               (const Rec4<T> *)o->posvol, o->n, (const Rec4<T> *)t->posvol, data, stride,
+                               rel->chunk_offset, rel->neighbor_size, rel->slice, (const KernelPoly<T> *)rel->poly,
+                               (T *)o->interp);
         LAUNCH_CHECK();
         return SPHX_OK;
     }

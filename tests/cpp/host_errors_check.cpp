@@ -35,6 +35,8 @@ int g_captures = 0;          // stream captures begun
 unsigned long long g_needed = 0; // what the next read of a single device word returns
 std::map<const void *, std::string> g_names;
 std::map<std::string, int> g_launches; // kernel -> launches
+std::string g_record;                  // of this kernel's last launch:
+unsigned g_workgroups = 0;
 dim3 g_grid, g_block;
 size_t g_lds;
 hipStream_t g_stream;
@@ -72,6 +74,8 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3, void **, size_t, hipStre
     if (g.x == 0)
         return hipErrorInvalidConfiguration;
     ++g_launches[g_names[f]];
+    if (g_names[f].find(g_record) != std::string::npos)
+        g_workgroups = g.x;
     if (((Stream *)s)->device != g_device)
         ++g_other_device;
     return hipSuccess;
@@ -143,21 +147,27 @@ struct Scene
     Scene(int device, int dim, int precision, uint32_t n)
     {
         REQUIRE(API(sphx_context_create)(device, &ctx) == SPHX_OK);
-        sphx_body_desc d{};
-        d.dim = dim;
-        d.precision = precision;
-        d.kind = SPHX_BODY_FLUID;
-        d.n_particles = n;
-        d.spacing_ref = 0.01;
-        d.h_spacing_ratio = 1.3;
-        d.rho0 = 1.0;
-        d.c0 = 10.0;
-        REQUIRE(API(sphx_body_create)(ctx, &d, &body) == SPHX_OK);
+        body = make_body(dim, precision, SPHX_BODY_FLUID, n);
         const double lo[3] = {0, 0, 0}, up[3] = {1, 1, 1};
         REQUIRE(API(sphx_cell_linked_list_create)(body, lo, up, 0.026, 2, &cll) == SPHX_OK);
         REQUIRE(API(sphx_relation_create_inner)(body, cll, &inner) == SPHX_OK);
         REQUIRE(API(sphx_update_cell_linked_list)(cll) == SPHX_OK);
         REQUIRE(API(sphx_update_relation)(inner) == SPHX_OK);
+    }
+    sphx_body *make_body(int dim, int precision, int kind, uint32_t n)
+    {
+        sphx_body_desc d{};
+        d.dim = dim;
+        d.precision = precision;
+        d.kind = kind;
+        d.n_particles = n;
+        d.spacing_ref = 0.01;
+        d.h_spacing_ratio = 1.3;
+        d.rho0 = 1.0;
+        d.c0 = 10.0;
+        sphx_body *b = nullptr;
+        REQUIRE(API(sphx_body_create)(ctx, &d, &b) == SPHX_OK);
+        return b;
     }
 };
 
@@ -273,13 +283,31 @@ void tile_waves()
         REQUIRE(API(sphx_batch_destroy)(batch) == SPHX_OK);
     }
 }
+
+// a few observers take a workgroup each, many share one (their lists are laid
+// out for a thread each)
+void observers()
+{
+    Scene s(0, 3, SPHX_FP64, 1000);
+    for (uint32_t n : {1u, 100u, 32768u, 32769u, 1000000u})
+    {
+        sphx_body *o = s.make_body(3, SPHX_FP64, SPHX_BODY_OBSERVER, n);
+        sphx_relation *r = nullptr;
+        REQUIRE(API(sphx_relation_create_contact)(o, s.body, s.cll, &r) == SPHX_OK);
+        REQUIRE(API(sphx_update_relation)(r) == SPHX_OK);
+        std::vector<double> v(n);
+        g_record = "k_interpolate";
+        REQUIRE(API(sphx_interpolate_contact)(r, SPHX_FIELD_PRESSURE, v.data(), n) == SPHX_OK);
+        REQUIRE(g_workgroups == (n <= 32768 ? n : (n + 63) / 64));
+    }
+}
 } // namespace
 
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
         {"large_write", large_write}, {"options_error", options_error}, {"options_device", options_device},
-        {"regrown_lists", regrown_lists}, {"tile_waves", tile_waves}};
+        {"regrown_lists", regrown_lists}, {"tile_waves", tile_waves}, {"observers", observers}};
     if (argc != 3 || !cases.count(argv[2]) || !(g_lib = dlopen(argv[1], RTLD_NOW)))
     {
         std::printf("usage: %s LIBRARY CASE\n", argv[0]);

@@ -54,3 +54,23 @@ def test_interpolation_around_a_wave_of_neighbours(hip, oracle, dim, precision, 
     for g, w in zip(got, want):
         assert np.all(g[0] == 0.0) and np.all(w[0] == 0.0)
         assert np.all(np.abs(g[1] - w[1]) <= tol * np.abs(w[1])), (g, w)
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("precision", [capi.FP64, capi.MIXED])
+@pytest.mark.parametrize("n_obs", [32768, 32769])
+def test_interpolation_of_many_observers(hip, oracle, dim, precision, n_obs):
+    """Both sides of the observer count from which one thread instead of a wave
+    takes an observer, the last workgroup with one observer; the same tolerances."""
+    rng = np.random.default_rng(n_obs + dim)
+    m = 40 if dim == 2 else 12  # spacing 0.025 and 0.083, h = 0.13: at most 350 neighbours
+    axis = (np.arange(m) + 0.5) / m
+    points = np.stack([g.ravel() for g in np.meshgrid(*[axis] * dim, indexing="ij")], axis=1)
+    pressure, velocity = 1.0 + rng.random(len(points)), 1.0 + rng.random((len(points), dim))
+    observers = rng.random((n_obs, dim))
+    sizes, got = observed(hip, dim, precision, points, pressure, velocity, observers)
+    sizes_ref, want = observed(oracle, dim, capi.FP64, points, pressure, velocity, observers)
+    assert np.array_equal(sizes, sizes_ref) and sizes.min() > 0 and sizes.max() <= 350
+    tol = (1e-12 if precision == capi.FP64 else 3e-5) * 350 / 200
+    for g, w in zip(got, want):
+        assert np.all(np.abs(g - w) <= tol * np.abs(w)), np.max(np.abs(g - w) / np.abs(w))
