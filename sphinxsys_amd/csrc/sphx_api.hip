@@ -230,10 +230,11 @@ sphx_status alloc(sphx_body *b, void **p, size_t bytes)
 
 
 //---------------------------------------------------------------------------
-// Host <-> device transfer of one field.  The layout and precision conversion
-// runs on the device: a kernel writes the host's layout (rows of K doubles, or
-// 32-bit integers) straight into pinned host memory, or reads it from there,
-// and the host only copies between that memory and the caller's.  Converting on
+// Host <-> device transfer of one field through pinned host memory.  The layout
+// and precision conversion runs on the device: a kernel writes the host's layout
+// (rows of K doubles, or 32-bit integers) straight into that memory, or reads it
+// from there, and the host only copies between it and the caller's (a field of
+// one array is copied and converted on the host up to a size, below).  Converting on
 // the host, one component at a time through pageable copies, took 44 ms for the
 // Position of 8.0M particles and 52 us for that of 800; now 7.3 ms (26 GB/s, of
 // 37 that four copying threads reach into fresh pages) and 15 us.
@@ -245,15 +246,15 @@ struct FieldComponents
     uint32_t stride;
     double offset;   // host value = device value + offset (Compression is kept as C - 1 in FP32-mixed)
 };
-__device__ __forceinline__ uint32_t to_host(uint32_t v, double) { return v; }
+__host__ __device__ __forceinline__ uint32_t to_host(uint32_t v, double) { return v; }
 template <class E>
-__device__ __forceinline__ double to_host(E v, double offset)
+__host__ __device__ __forceinline__ double to_host(E v, double offset)
 {
     return offset != 0.0 ? (double)v + offset : (double)v;
 }
-__device__ __forceinline__ void from_host(uint32_t &d, uint32_t v, double) { d = v; }
+__host__ __device__ __forceinline__ void from_host(uint32_t &d, uint32_t v, double) { d = v; }
 template <class E>
-__device__ __forceinline__ void from_host(E &d, double v, double offset)
+__host__ __device__ __forceinline__ void from_host(E &d, double v, double offset)
 {
     d = E(offset != 0.0 ? v - offset : v);
 }
@@ -356,6 +357,54 @@ void copy_host(void *dst, const void *src, size_t bytes)
             h.join();
 }
 
+// Bytes up to which a field of one array (a scalar, or the velocity's records of
+// four) is copied as it lies and converted on the host: one copy starts sooner
+// than a kernel, and up to here the conversion costs less than the kernel's slower
+// way over the bus.  Read and write, copy / kernel, us: 3,000 doubles 11 + 11 / 16
+// + 16, 80,000 36 + 31 / 40 + 37, 300,000 125 + 91 / 121 + 111; 8,000 floats 12 + 11
+// / 17 + 17, 200,000 52 + 43 / 95 + 83, 1,000,000 241 + 181 / 288 + 238; 100,000
+// identifiers 27 + 23 / 30 + 27; 3,000 velocities in double 15 + 13 / 17 + 17, 12,000
+// 27 + 24 / 27 + 24, in float 3,000 14 + 13 / 17 + 17, 200,000 171 + 171 / 181 + 180.
+// (Pageable copies into the caller's array: as fast, but not the first 16 MB of a
+// stream, which take 1.2 us more per 4 KB.)
+template <int K, class E>
+constexpr size_t array_most()
+{
+    return sizeof(E) == 4 ? 4u << 20 : K == 1 ? 2u << 20 : 256u << 10;
+}
+static_assert(array_most<1, float>() <= 2 * kStagingHalf, "one staging buffer");
+
+template <int K, int STRIDE, class E, class H>
+sphx_status transfer_array(sphx_body *b, const FieldComponents<E> &f, H *host, bool write)
+{
+    hipStream_t s = b->ctx->stream;
+    const size_t n = b->n, bytes = n * STRIDE * sizeof(E);
+    const double offset = f.offset;
+    StagingBuffer stage;
+    sphx_status st;
+    if (bytes > kSmallTransfer && (st = stage.take()))
+        return st;
+    E *v = (E *)(bytes > kSmallTransfer ? stage.p : b->ctx->transfer_h);
+    if (write)
+    {
+        for (size_t i = 0; i < n; ++i)
+        {
+            for (int k = 0; k < K; ++k)
+                from_host(v[i * STRIDE + k], host[i * K + k], offset);
+            for (int k = K; k < STRIDE; ++k)
+                v[i * STRIDE + k] = E(0); // the rest of a record stays zero
+        }
+        SPHX_HIP(hipMemcpyAsync(f.c[0], v, bytes, hipMemcpyHostToDevice, s));
+    }
+    else
+        SPHX_HIP(hipMemcpyAsync(v, f.c[0], bytes, hipMemcpyDeviceToHost, s));
+    SPHX_HIP(hipStreamSynchronize(s));
+    for (size_t i = 0; !write && i < n; ++i)
+        for (int k = 0; k < K; ++k)
+            host[i * K + k] = to_host(v[i * STRIDE + k], offset);
+    return SPHX_OK;
+}
+
 template <int K, class E, class H>
 sphx_status transfer_rows(sphx_body *b, const FieldComponents<E> &f, H *host, bool write)
 {
@@ -363,6 +412,14 @@ sphx_status transfer_rows(sphx_body *b, const FieldComponents<E> &f, H *host, bo
     hipStream_t s = ctx->stream;
     constexpr size_t row = K * sizeof(H);
     const size_t n = b->n;
+    if (n * f.stride * sizeof(E) <= array_most<K, E>())
+    {
+        if constexpr (K == 1)
+            return transfer_array<1, 1>(b, f, host, write);
+        if constexpr (K == 2 || K == 3)
+            if (f.stride == 4u)
+                return transfer_array<K, 4>(b, f, host, write);
+    }
     auto launch = [&](unsigned char *stage, size_t first, size_t rows) -> sphx_status {
         const uint32_t values = (uint32_t)(rows * K);
         const dim3 g((values + 255u) / 256u), blk(256);

@@ -174,8 +174,8 @@ struct Scene
 // a large write whose kernels fail says so
 void large_write()
 {
-    Scene s(0, 2, SPHX_FP64, 100000);
-    std::vector<double> v(100000, 1.0);
+    Scene s(0, 2, SPHX_FP64, 1000000);
+    std::vector<double> v(1000000, 1.0);
     REQUIRE(API(sphx_body_write)(s.body, SPHX_FIELD_PRESSURE, v.data(), v.size()) == SPHX_OK);
     g_sync_error = 1;
     REQUIRE(API(sphx_body_write)(s.body, SPHX_FIELD_PRESSURE, v.data(), v.size()) == SPHX_E_HIP);
@@ -301,13 +301,40 @@ void observers()
         REQUIRE(g_workgroups == (n <= 32768 ? n : (n + 63) / 64));
     }
 }
+
+// a scalar or velocity field up to a size is copied as it lies, without a kernel
+void array_copies()
+{
+    for (int precision : {SPHX_FP64, SPHX_MIXED})
+        for (uint32_t n : {100u, 10000u, 100000u, 500000u, 2000000u})
+        {
+            Scene s(0, 3, precision, n);
+            std::vector<double> v(3 * (size_t)n, 1.0);
+            std::vector<uint32_t> id(n, 7u);
+            const bool fp64 = precision == SPHX_FP64;
+            for (bool write : {true, false})
+            {
+                auto copied = [&](int field, void *host) {
+                    g_launches.clear();
+                    REQUIRE((write ? API(sphx_body_write)(s.body, field, host, n)
+                                   : API(sphx_body_read)(s.body, field, host, n)) == SPHX_OK);
+                    return launches("k_field_") == 0;
+                };
+                REQUIRE(copied(SPHX_FIELD_PRESSURE, v.data()) == (n <= (fp64 ? 262144u : 1048576u)));
+                REQUIRE(copied(SPHX_FIELD_ORIGINAL_ID, id.data()) == (n <= 1048576u));
+                REQUIRE(copied(SPHX_FIELD_VELOCITY, v.data()) == (n <= (fp64 ? 8192u : 262144u)));
+                REQUIRE(!copied(SPHX_FIELD_POSITION, v.data()));
+            }
+        }
+}
 } // namespace
 
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
         {"large_write", large_write}, {"options_error", options_error}, {"options_device", options_device},
-        {"regrown_lists", regrown_lists}, {"tile_waves", tile_waves}, {"observers", observers}};
+        {"regrown_lists", regrown_lists}, {"tile_waves", tile_waves}, {"observers", observers},
+        {"array_copies", array_copies}};
     if (argc != 3 || !cases.count(argv[2]) || !(g_lib = dlopen(argv[1], RTLD_NOW)))
     {
         std::printf("usage: %s LIBRARY CASE\n", argv[0]);

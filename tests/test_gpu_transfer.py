@@ -2,7 +2,9 @@
 precision, exactly, for each device layout (three arrays, 4-wide records, one
 array, matrix components, 32-bit integers), with sizes on both sides of the
 context's own pinned buffer (262,144 bytes), of one half of a staging buffer
-(8 MiB) and over more than two halves."""
+(8 MiB) and over more than two halves, and of the sizes up to which a field of one
+array is copied as it lies: 262,144 doubles, 1,048,576 32-bit values, 8,192
+velocities in double and 262,144 in float."""
 import numpy as np
 import pytest
 
@@ -19,7 +21,8 @@ FIELDS = [("Position", lambda d: d, True), ("Velocity", lambda d: d, False), ("P
 
 @pytest.mark.parametrize("dim", [2, 3])
 @pytest.mark.parametrize("precision", [capi.FP64, capi.MIXED])
-@pytest.mark.parametrize("n", [1, 257, 3641, 10923, 32769, 349526, 800001])
+@pytest.mark.parametrize("n", [1, 257, 3641, 8192, 8193, 10923, 32769, 65536, 65537, 262144, 262145, 349526, 800001,
+                               1048576, 1048577])
 def test_write_read_round_trip(hip, dim, precision, n):
     rng = np.random.default_rng(n)
     ctx = ck.Context(hip)

@@ -20,7 +20,7 @@ def harness(tmp_path_factory):
 
 
 @pytest.mark.parametrize("case", ["large_write", "options_error", "options_device", "regrown_lists", "tile_waves",
-                                  "observers"])
+                                  "observers", "array_copies"])
 def test_host_paths_on_the_stand_in(harness, case):
     r = subprocess.run([harness, sphinxsys_amd.LIBRARY_PATH, case], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
