@@ -46,6 +46,11 @@ def test_fp64_sums_staged_and_not(hip, oracle, dim, m, window):
         for name in names + ["Pressure", "Force", "CompressionRate", "Compression", "Velocity", "Displacement"]:
             g, c = pr.read(name)
             assert rel_l2(g, c) < FP64_GATE, (correction, name)
+        pr.both(lambda s: ck.ViscousForceCK(s["inner"], *s["walls"], mu=0.1, correction=correction).exec())
+        pr.both(lambda s: ck.KernelGradientIntegral(s["inner"], *s["walls"], correction=correction).exec())
+        for name in ("ViscousForce", "KernelGradientIntegral"):
+            g, c = pr.read(name)
+            assert rel_l2(g, c) < FP64_GATE, (correction, name)
     pr.close()
 
 
