@@ -1291,8 +1291,12 @@ __global__ void __launch_bounds__(kThreads) k_cll_order(CllScene a) { cll_order_
 // The whole cell-list update of a small body in one workgroup: counts, scan,
 // slots and the order within a cell in LDS (a counter per cell and a 16-bit
 // index per particle), instead of five to seven launches of a few blocks each.
-// 800 particles in 2D (2,116 cells) 27 -> 10 us, 3,200 (8,281 cells) 28 -> 20; at
-// 8,000 in 3D (15,600 cells) one CU's divisions take longer, 77 instead of 40.
+// A particle's place in its cell is the number of smaller indices there, so a
+// full cell is no serial chain (a lane ordering a cell alone made 1,000 particles
+// in 3D, seventeen to a cell, take 24 us).  Launches / workgroup: 900 particles in
+// 2D 18 / 7 us, 3,600 20 / 9, 1,000 in 3D 19 / 7, 4,096 25 / 14, 4,096 in 15,625
+// cells 27 / 20; at 8,000 in 3D (15,600 cells) one CU's divisions took longer, 77
+// instead of 40.
 //---------------------------------------------------------------------------
 constexpr uint32_t kSmallThreads = 1024, kSmallRounds = 4;
 constexpr uint32_t kSmallParticles = kSmallThreads * kSmallRounds, kSmallCells = 16384;
@@ -1360,25 +1364,21 @@ __device__ __forceinline__ void cll_small_body(const CllScene &a, uint32_t *lds)
             idx[atomicAdd(&cnt[key[r]], 1u)] = (uint16_t)i;
     }
     __syncthreads();
-    // cnt[c] is now the end of cell c; its indices into ascending order
-    for (uint32_t c = t; c < a.ncells; c += kSmallThreads)
+    // cnt[c] is now the end of cell c: each particle's place among the ascending
+    // indices of its cell
+#pragma unroll
+    for (uint32_t r = 0; r < kSmallRounds; ++r)
     {
-        const uint32_t lo = c ? cnt[c - 1u] : 0u, hi = cnt[c];
-        for (uint32_t q = lo + 1u; q < hi; ++q)
+        const uint32_t i = r * kSmallThreads + t;
+        if (i < a.n)
         {
-            const uint16_t v = idx[q];
-            uint32_t r = q;
-            while (r > lo && idx[r - 1u] > v)
-            {
-                idx[r] = idx[r - 1u];
-                --r;
-            }
-            idx[r] = v;
+            const uint32_t lo = key[r] ? cnt[key[r] - 1u] : 0u, hi = cnt[key[r]];
+            uint32_t place = lo;
+            for (uint32_t q = lo; q < hi; ++q)
+                place += idx[q] < i ? 1u : 0u;
+            a.particle_index[place] = i;
         }
     }
-    __syncthreads();
-    for (uint32_t k = t; k < a.n; k += kSmallThreads)
-        a.particle_index[k] = idx[k];
 }
 template <int D>
 __global__ void __launch_bounds__(kSmallThreads) k_cll_small(CllScene a)
