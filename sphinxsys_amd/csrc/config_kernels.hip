@@ -966,14 +966,19 @@ __global__ void __launch_bounds__(kTileWaves * V * 64) k_relation_tile(BuildArgs
 {
     relation_tile_body<D, kTileWaves, V>(b, xcd_block_index());
 }
-// Waves per chunk of a build of nchunks chunks.  Inner build and wall contact,
-// one wave / four: 800 particles in 2D 41 + 24 / 18 + 14 us, 8,000 in 3D 88 + 54 /
-// 47 + 26, 90,000 133 + 68 / 92 + 39, 195,000 149 + 76 / 144 + 59, 415,000 226 +
-// 85 / 280 + 91 (each wave loads the candidates of its cells itself; eight waves
-// are slower from 90,000 on)
+// Whether a build of nchunks chunks has four waves per chunk.  One wave / four,
+// us, particles sorted: inner 2D 22,500 56 / 32, 126,000 62 / 52, 250,000 80 / 78;
+// inner 3D 27,000 78 / 44, 104,000 88 / 77, 149,000 101 / 97, 176,000 101 / 105,
+// 250,000 115 / 137, and disordered within 1,024 places 125,000 232 / 235, 149,000
+// 267 / 296 (each wave loads the candidates of its cells itself); tank walls 3D
+// 90,000 77 / 44, 195,000 83 / 58, 263,000 88 / 65.  Eight waves are slower from
+// 90,000 on.  A batch builds inner and wall lists in one launch: its step in 3D
+// 1,650 chunks 609 / 600, 2,480 715 / 715, 4,130 840 / 872, in 2D 4,000 360 / 342.
 constexpr int kTileSplit = 4;
-constexpr uint32_t kTileSplitBelow = 4096;
-inline bool tile_split(uint32_t nchunks) { return nchunks < kTileSplitBelow; }
+inline bool tile_split(int D, bool inner, uint32_t nchunks)
+{
+    return nchunks < (D == 3 && inner ? 2400u : 4096u);
+}
 
 //---------------------------------------------------------------------------
 // staging sets of the inner fluid relation, from its finished slices: for each
@@ -1948,7 +1953,7 @@ sphx_status relation_to_csr(sphx_relation *rel)
 template <int D>
 static sphx_status launch_tile(sphx_context *ctx, const BuildArgs &b, uint32_t nchunks)
 {
-    if (tile_split(nchunks))
+    if (tile_split(D, b.r.inner, nchunks))
         hipLaunchKernelGGL((k_relation_tile<D, kTileSplit>), dim3(nchunks), dim3(kTileSplit * 64), 0, ctx->stream, b);
     else
         hipLaunchKernelGGL((k_relation_tile<D, 1>), dim3(grid_for(nchunks, kTileWaves)), dim3(kTileWaves * 64), 0,
@@ -2223,7 +2228,7 @@ sphx_status batch_relations(const BatchConfig &b)
         set_error("tiled relation build: 1, 2 or 4 waves per workgroup");
         return SPHX_E_ARG;
     }
-    if (w == 1 && tile_split(b.blocks_chunks))
+    if (w == 1 && tile_split(b.D, true, b.blocks_chunks))
         b.D == 2 ? launch_batch_tile<2, 1, kTileSplit>(b) : launch_batch_tile<3, 1, kTileSplit>(b);
     else if (b.D == 2)
         w == 1 ? launch_batch_tile<2, 1>(b) : w == 2 ? launch_batch_tile<2, 2>(b) : launch_batch_tile<2, 4>(b);

@@ -1,5 +1,6 @@
 """Neighbour lists bit-exact with the oracle on both sides of the size from which
-one wave instead of four builds a chunk of 64 particles (262,144 particles),
+one wave instead of four builds a chunk of 64 particles (262,144 particles; inner
+relations in 3D 153,600),
 with a last chunk of a few particles, a window-shuffled order (sources of many
 cells in a chunk), and a cluster whose search boxes hold more candidates than
 the build keeps in registers (512)."""
@@ -12,7 +13,8 @@ from tests.test_gpu_parity import Pair, jittered_lattice, shuffled
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("dim,m,cluster", [(2, 511, 0), (2, 513, 700), (3, 63, 600), (3, 64, 0), (3, 65, 600), (3, 4, 0)])
+@pytest.mark.parametrize("dim,m,cluster", [(2, 511, 0), (2, 513, 700), (3, 63, 600), (3, 64, 0), (3, 65, 600), (3, 4, 0),
+                                           (3, 53, 600), (3, 54, 600)])
 def test_lists_built_by_one_and_four_waves(hip, oracle, dim, m, cluster):
     dp = 0.02
     fluid = shuffled(jittered_lattice(dim, m, dp, 8), 200, 9)
