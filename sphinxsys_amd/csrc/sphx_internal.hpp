@@ -55,13 +55,13 @@ constexpr uint32_t kStageCap = 1536;           // distinct neighbours staged per
 // 65 with eight, 45 + 58 with four, 58 + 67 staged with one.  The upper lines lie
 // where the whole step is as fast with one lane and staging (FP64: 134,000
 // particles in 3D 1,011 us with four, 1,058 with one; 214,000 1,400 and 1,361;
-// 125,000 in 2D 431 and 423).  One lane in FP32-mixed 3D, whose second half step
-// equals its cell traversal bit for bit.
-constexpr uint32_t kSplitFew3D = 16384, kSplit3D = 163840, kSplit2D = 131072;
+// 125,000 in 2D 431 and 423.  FP32-mixed in 2D: 80,000 246 and 262, 100,000 278 and
+// 278).  FP32-mixed 3D has one lane: its passes with four were not measured.
+constexpr uint32_t kSplitFew3D = 16384, kSplit3D = 163840, kSplit2D = 131072, kSplit2DMixed = 98304;
 constexpr int split_lanes(int D, int P, uint32_t n)
 {
     if (D == 2)
-        return n < kSplit2D ? 4 : 1;
+        return n < (P == P_FP64 ? kSplit2D : kSplit2DMixed) ? 4 : 1;
     return P != P_FP64 ? 1 : n < kSplitFew3D ? 8 : n < kSplit3D ? 4 : 1;
 }
 // reported through the relation build's `needed` slot when a search box holds
