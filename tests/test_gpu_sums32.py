@@ -12,6 +12,7 @@ import pytest
 from sphinxsys_amd import _capi as capi
 from sphinxsys_amd import ck
 from tests.test_gpu_parity import Pair, jittered_lattice, rel_l2, shuffled
+from tests.test_gpu_sums64 import distinct_neighbours
 
 pytestmark = pytest.mark.gpu
 
@@ -25,14 +26,19 @@ def slab(m):
     return wall, np.tile([0.0, 1.0], (len(wall), 1))
 
 
-@pytest.mark.parametrize("m,window", [(313, None), (313, 0), (314, None), (314, 1024), (314, 0)])
-def test_mixed_sums_against_the_oracle(hip, oracle, m, window):
-    """Ordered, shuffled in windows (some blocks have more distinct neighbours than
-    are staged) and shuffled throughout (all have)."""
+@pytest.mark.parametrize("m,ordered", [(313, 1.0), (313, 0.0), (314, 1.0), (314, 0.5), (314, 0.0)])
+def test_mixed_sums_against_the_oracle(hip, oracle, m, ordered):
+    """A part of the particles in a lattice's rows, whose blocks of 256 have few
+    enough distinct neighbours to be staged, the rest shuffled, whose blocks have
+    too many."""
     fluid = jittered_lattice(2, m, DP, 3)
-    if window is not None:
-        fluid = shuffled(fluid, window, 4)
+    cut = int(ordered * len(fluid))
+    fluid[cut:] = np.random.default_rng(4).permutation(fluid[cut:])
     pr = Pair(hip, oracle, fluid, DP, *slab(m), capi.MIXED, rho0=1000.0, c0=20.0)
+    for cap in (1400, 1536):  # of the passes, of the other sums
+        part = np.mean(distinct_neighbours(pr.gpu["inner"]) <= cap)
+        print(f"{m} a side, {ordered} in rows: blocks staged {part}", flush=True)
+        assert abs(part - ordered) < 0.05, part
     rng = np.random.default_rng(6)
     n = len(fluid)
     pr.write("Compression", 1.0 + rng.uniform(-0.01, 0.01, n))

@@ -1,9 +1,9 @@
 """The FP64 neighbour sums against the oracle at the sizes where their form
 changes (eight, four and one lanes per particle, the last from LDS-staged
-records), bodies of less than a wave, last blocks of a few particles, and
-shuffled orders, whose blocks have more distinct neighbours than the kernels
-stage (some of them in a window of 1024, all of them in a full shuffle) and
-read from global memory.
+records), bodies of less than a wave, last blocks of a few particles, and orders
+in which the blocks of 256 particles have few enough distinct neighbours to be
+staged (particles sorted), too many (a lattice's rows, a full shuffle) or some of
+each (a sorted body shuffled in windows), the others read from global memory.
 
 Gate: 1e-10 relative L2, the FP64 gate of the same comparison on smaller bodies.
 Several lanes add every 4th or 8th term and then each other's sums, so the terms
@@ -21,18 +21,40 @@ from tests.test_gpu_parity import FP64_GATE, Pair, jittered_lattice, rel_l2, shu
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("dim,m,window", [(2, 7, None), (2, 362, None), (2, 363, None), (2, 363, 0),
-                                          (3, 5, None), (3, 25, None), (3, 26, None), (3, 54, None),
-                                          (3, 55, None), (3, 55, 1024), (3, 55, 0)])
-def test_fp64_sums_staged_and_not(hip, oracle, dim, m, window):
+# distinct neighbours of a block that the summation, the first and the second pass stage
+CAPS = {2: (768, 768, 768), 3: (1536, 1344, 1440)}
+
+
+def distinct_neighbours(relation):
+    """Per block of 256 particles, from its lists."""
+    size, offset, index = relation.read()
+    return np.array([len(np.unique(index[offset[i]:offset[min(i + 256, len(size))]])) for i in range(0, len(size), 256)])
+
+
+@pytest.mark.parametrize("dim,m,order", [(2, 7, "rows"), (2, 362, "sorted"), (2, 363, "sorted"), (2, 363, "windows"),
+                                         (2, 363, "rows"), (2, 363, "shuffled"),
+                                         (3, 5, "rows"), (3, 25, "sorted"), (3, 26, "rows"), (3, 54, "sorted"),
+                                         (3, 55, "sorted"), (3, 55, "windows"), (3, 55, "rows"), (3, 55, "shuffled")])
+def test_fp64_sums_staged_and_not(hip, oracle, dim, m, order):
     dp = 0.02
     fluid = jittered_lattice(dim, m, dp, 3)
-    if window is not None:
-        fluid = shuffled(fluid, window, 4)
     wall = jittered_lattice(dim, m, dp, 5, jitter=0.0)
     wall = wall[wall[:, -1] < 3 * dp].copy()
     wall[:, -1] -= 3 * dp
+    if order == "shuffled":
+        fluid = shuffled(fluid, 0, 4)
     pr = Pair(hip, oracle, fluid, dp, wall, np.tile(np.eye(dim)[-1], (len(wall), 1)), capi.FP64, rho0=1000.0, c0=20.0)
+    if order in ("sorted", "windows"):
+        pr.both(lambda s: ck.ParticleSortCK(s["f"], s["fc"]).exec())
+        if order == "windows":
+            pr.write("Position", shuffled(pr.read("Position")[0], 300, 4))
+        pr.both(lambda s: ck.UpdateCellLinkedList(s["fc"]).exec())
+        pr.both(lambda s: ck.UpdateRelation(s["inner"], *s["walls"]).exec())
+    if m in (363, 55):
+        staged = [np.mean(distinct_neighbours(pr.gpu["inner"]) <= cap) for cap in CAPS[dim]]
+        print(f"{dim}D {order}: staged blocks {staged}", flush=True)
+        for part in staged:
+            assert {"sorted": part > 0.5, "windows": 0.05 < part < 0.95}.get(order, part < 0.05), staged
     rng = np.random.default_rng(6)
     n = len(fluid)
     pr.write("Compression", 1.0 + rng.uniform(-0.01, 0.01, n))
