@@ -231,13 +231,12 @@ sphx_status build_tables(sphx_batch *b)
         const uint32_t n = sc.inner->source->n;
         const uint64_t nc = sc.cll->ncells;
         const uint64_t b256 = (n + 255u) / 256u, bcells = (nc + 1 + 255u) / 256u;
+        const uint64_t bsums = ((uint64_t)n * split_lanes(b->D, b->P, n) + 255u) / 256u;
         const uint32_t tiles = batch_cll_tiles(sc.cll);
-        if (b256 > kMapLimit || bcells > kMapLimit || tiles > kMapLimit)
+        if (b256 > kMapLimit || bsums > kMapLimit || bcells > kMapLimit || tiles > kMapLimit)
             return batch_error(SPHX_E_CAPACITY, "a batched scene exceeds 65536 blocks of particles or cells");
         for (uint32_t k = 0; k < b256; ++k)
             m256.push_back((uint32_t)(s << 16) | k);
-        // (at most 512 blocks where a scene has several lanes per particle)
-        const uint64_t bsums = ((uint64_t)n * split_lanes(b->D, b->P, n) + 255u) / 256u;
         for (uint32_t k = 0; k < bsums; ++k)
             msums.push_back((uint32_t)(s << 16) | k);
         for (uint32_t k = 0; k < bcells; ++k)

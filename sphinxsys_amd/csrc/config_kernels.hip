@@ -1400,13 +1400,6 @@ __global__ void __launch_bounds__(kSmallThreads) kb_cll_small(const CllScene *__
     if (gate[blockIdx.x])
         cll_small_body<D>(tab[blockIdx.x], cll_lds);
 }
-template <class K>
-void allow_lds(K kernel, size_t bytes)
-{
-    if (bytes > 65536)
-        (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-}
-
 __global__ void __launch_bounds__(kThreads) kb_cll_clear(const CllScene *__restrict__ tab,
                                                          const uint32_t *__restrict__ map,
                                                          const uint32_t *__restrict__ gate)

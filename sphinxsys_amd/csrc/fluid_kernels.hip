@@ -207,8 +207,8 @@ __device__ __forceinline__ T eval_poly(const PolyLDS<T> &lds, T r, T x_per_r)
 // through the nodes loc - 1 .. loc + 2 is the quartic less the product of the
 // distances to them, (f + 1) f (f - 1)(f - 2) = u (u - 2) with f = x - loc and
 // u = f^2 - f.  The FP64 passes use it: a table interval is a 32-byte LDS read
-// at random among the lanes and 8 registers for each pair in flight (pass 1 takes
-// 140 registers instead of 220, pass 2 174 instead of 256).  FP32-mixed keeps
+// at random among the lanes and 8 registers for each pair in flight (in 3D pass 1
+// takes 134 registers instead of 220, pass 2 168 instead of 256).  FP32-mixed keeps
 // the table: there the closed form made pass 1 slower (8M particles: 826 -> 873
 // us) and pass 2 faster (1125 -> 1070 us) by as much.
 __device__ __forceinline__ double kernel_gradient(double r, double x_per_r)
@@ -470,23 +470,21 @@ __device__ __forceinline__ PairGeo<T> pair_geometry_of(const PV<T, D> &pi, const
 }
 
 // The neighbour walk of for_each_neighbor with the latencies overlapped: the
-// entries are taken in batches of 8; the list entries of the next batch are
+// entries are taken in batches of KB; the list entries of the next batch are
 // loaded while the current one is evaluated, and for each batch the records
-// are fetched, the distances computed and the 8 kernel intervals requested
-// from LDS before any pair is finished.  fetch(entry) returns a record with
+// are fetched, the distances computed and the KB kernel intervals requested
+// from LDS before any pair is finished.  fetch(entry) returns a whole record with
 // the neighbour's position and volume in .pv (entries past the count fetch
-// entry 0, which every non-empty list has, and are not finished); late(entry,
-// record) loads the rest of the record, issued with the kernel intervals once
-// the positions are no longer needed (so the batch's records and geometry do
-// not hold registers at the same time); pair(record, geo) finishes a pair.
-// Pairs are finished in list order with the arithmetic of eval_poly, so the
-// sums are those of the plain walk.  With S lanes a particle, base and count are
-// those of the lane's own entries (split_count), S apart.  In double the kernel gradient is the closed
-// form over grad_scale, which the caller's sums are multiplied by at the end.
-template <int D, uint32_t KB, int S = 1, class T, class I, class Fetch, class Late, class Pair>
+// entry 0, which every non-empty list has, and are not finished); pair(record,
+// geo) finishes a pair.  Pairs are finished in list order with the arithmetic of
+// eval_poly, so the sums are those of the plain walk.  With S lanes a particle,
+// base and count are those of the lane's own entries (split_count), S apart.  In
+// double the kernel gradient is the closed form over grad_scale, which the
+// caller's sums are multiplied by at the end.
+template <int D, uint32_t KB, int S = 1, class T, class I, class Fetch, class Pair>
 __device__ __forceinline__ void walk_pipelined(const I *entries, uint32_t base, uint32_t count,
                                                const PV<T, D> &pi, const PolyLDS<T> &lds, T x_per_r,
-                                               Fetch &&fetch, Late &&late, Pair &&pair)
+                                               Fetch &&fetch, Pair &&pair)
 {
     // pairs per batch: 8 in double, 4 where several lanes share a particle (short
     // lists, more waves: 90,000 particles in 3D 45 + 58 -> 43 + 54 us); 6 is faster
@@ -535,9 +533,6 @@ __device__ __forceinline__ void walk_pipelined(const I *entries, uint32_t base, 
 #pragma unroll
         for (uint32_t q = 0; q < kBatch; ++q)
             c[q] = *reinterpret_cast<const Coef4<T> *>(lds.c[loc[q]]);
-#pragma unroll
-        for (uint32_t q = 0; q < kBatch; ++q)
-            late(idx[q], rec[q]);
         // keep the batch's reads issued together (the scheduler would otherwise
         // sink each next to its use and wait on it alone)
         __builtin_amdgcn_sched_barrier(0);
@@ -932,7 +927,6 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
     };
     auto pair = [&](const Rec &rj, const PairGeo<T> &g) { add(term(rj, g)); };
     const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
-    auto no_late = [](uint32_t, Rec &) {};
     constexpr uint32_t kWalkBatch = P == P_MIXED ? 6u : S > 1 ? 4u : 8u;
     auto global_rec = [&](uint32_t j) { return Rec{load_pv<T, D>(a.posvol, j), a.p[j]}; };
     if constexpr (kOrdered<T, S>)
@@ -945,11 +939,10 @@ __device__ __forceinline__ void pass1_body(const FluidArgs<typename Prec<P>::T> 
             add);
     else if (staged)
         walk_pipelined<D, kWalkBatch>(
-            a.local_slice, nb, nc, pi, poly_in, x_per_r, [&](uint32_t r) { return Rec{s_pv.get(r), s_p[r]}; }, no_late,
-            pair);
+            a.local_slice, nb, nc, pi, poly_in, x_per_r, [&](uint32_t r) { return Rec{s_pv.get(r), s_p[r]}; }, pair);
     else
         walk_pipelined<D, kWalkBatch, S>(a.slice, nb + (lane.sub << 6), split_count<S>(nc, lane.sub), pi, poly_in,
-                                         x_per_r, global_rec, no_late, pair);
+                                         x_per_r, global_rec, pair);
     if constexpr (S > 1 && !kOrdered<T, S>)
     {
         fx = lane_sum<S>(fx);
@@ -1391,9 +1384,6 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
         };
         auto pair = [&](const Rec &rj, const PairGeo<T> &g) { add(term(rj, g)); };
         const uint32_t nb = a.chunk[i >> 6] + (i & 63u), nc = a.count[i];
-        // whole records up front: loading the velocities late (as pass 1 loads
-        // its pressures) makes this pass spill under its register cap
-        auto no_late = [](uint32_t, Rec &) {};
         constexpr uint32_t kWalkBatch = P == P_MIXED ? 6u : S > 1 ? 4u : 8u;
         auto global_rec = [&](uint32_t j) { return Rec{load_pv<T, D>(a.posvol, j), a.vel[j]}; };
         if constexpr (TRAV)
@@ -1410,10 +1400,10 @@ __device__ __forceinline__ void pass2_body(const FluidArgs<typename Prec<P>::T> 
         else if (staged)
             walk_pipelined<D, kWalkBatch>(
                 a.local_slice, nb, nc, pi, poly_in, x_per_r,
-                [&](uint32_t r) { return Rec{s_pv.get(r), s_v.get(r)}; }, no_late, pair);
+                [&](uint32_t r) { return Rec{s_pv.get(r), s_v.get(r)}; }, pair);
         else
             walk_pipelined<D, kWalkBatch, S>(a.slice, nb + (lane.sub << 6), split_count<S>(nc, lane.sub), pi, poly_in,
-                                             x_per_r, global_rec, no_late, pair);
+                                             x_per_r, global_rec, pair);
         if constexpr (S > 1 && !kOrdered<T, S>)
         {
             div = lane_sum<S>(div);
@@ -2764,9 +2754,7 @@ __global__ void kb_gate(const SceneArgs<T> *__restrict__ tab, uint32_t n_scenes,
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n_scenes)
         return;
-    unsigned long long *st = tab[s].scalars + step_slot(substeps & 1u);
-    if (tab[s].f.n == 0u)
-        st[STEP_ERROR] = 1; // no particle, no time step
+    const unsigned long long *st = tab[s].scalars + step_slot(substeps & 1u);
     for (int k = 0; k < STEP_SLOTS; ++k)
         state[(size_t)s * STEP_SLOTS + k] = st[k];
     const bool done = st[STEP_ERROR] == 0 && !(get_double(st + STEP_RELAXATION) < get_double(st + STEP_ADV_DT));
@@ -2904,14 +2892,6 @@ static sphx_status dispatch(sphx_body *b, A &&...args)
     if (b->D == 2 && b->P == P_MIXED)
         return L<2, P_MIXED>::run(b, args...);
     return L<3, P_MIXED>::run(b, args...);
-}
-
-// kernels that take more than 64 KiB of dynamic LDS must say so first
-template <class K>
-static void allow_lds(K kernel, size_t bytes)
-{
-    if (bytes > 65536)
-        (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
 #define LAUNCH_CHECK()                     \

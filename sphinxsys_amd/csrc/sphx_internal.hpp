@@ -21,6 +21,14 @@ sphx_status hip_fail(hipError_t e, const char *what);
             return ::sphx::hip_fail(e_, #call);       \
     } while (0)
 
+// kernels that take more than 64 KiB of dynamic LDS must say so first
+template <class K>
+void allow_lds(K kernel, size_t bytes)
+{
+    if (bytes > 65536)
+        (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+
 // Device memory of the objects of a context (s is the context's stream).
 // dev_free waits for that stream only and keeps the block for a later
 // dev_alloc of the process (up to the block's size and at least half of it)
