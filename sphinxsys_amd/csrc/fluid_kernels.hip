@@ -3497,6 +3497,7 @@ struct InterpL
                         : field == SPHX_FIELD_VELOCITY ? (const T *)t->vel + component
                                                        : (const T *)t->C;
         const uint32_t stride = field == SPHX_FIELD_VELOCITY ? 4u : 1u;
+        o->ctx->work_queued = true;
         if (o->n <= kWaveObservers)
             hipLaunchKernelGGL((k_interpolate_wave<D, T>), dim3(o->n), dim3(64), 0, o->ctx->stream,
                                (const Rec4<T> *)o->posvol, (const Rec4<T> *)t->posvol, data, stride, rel->chunk_offset,

@@ -138,12 +138,18 @@ void Scratch::release()
     bytes = 0;
 }
 
+static sphx_status wait_for_stream(sphx_context *ctx)
+{
+    SPHX_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->work_queued = false;
+    return SPHX_OK;
+}
+
 sphx_status read_scalars(sphx_context *ctx, int first, int count)
 {
     SPHX_HIP(hipMemcpyAsync(ctx->scalars_h + first, ctx->scalars_d + first, count * sizeof(unsigned long long),
                             hipMemcpyDeviceToHost, ctx->stream));
-    SPHX_HIP(hipStreamSynchronize(ctx->stream));
-    return SPHX_OK;
+    return wait_for_stream(ctx);
 }
 
 // events come from a per-context pool (creating two events per launch costs
@@ -162,6 +168,7 @@ static hipEvent_t pooled_event(sphx_context *ctx)
 
 ProfileScope::ProfileScope(sphx_context *c, const char *s) : ctx(c), stage(s)
 {
+    ctx->work_queued = true;
     // a null stage records nothing
     const bool timed = s && ctx->profiling && (!ctx->profile_passes_only || std::strncmp(s, "acoustic_pass", 13) == 0);
     start = timed ? pooled_event(ctx) : nullptr;
@@ -357,22 +364,26 @@ void copy_host(void *dst, const void *src, size_t bytes)
             h.join();
 }
 
-// Bytes up to which a field of one array (a scalar, or the velocity's records of
-// four) is copied as it lies and converted on the host: one copy starts sooner
-// than a kernel, and up to here the conversion costs less than the kernel's slower
-// way over the bus.  Read and write, copy / kernel, us: 3,000 doubles 11 + 11 / 16
-// + 16, 80,000 36 + 31 / 40 + 37, 300,000 125 + 91 / 121 + 111; 8,000 floats 12 + 11
-// / 17 + 17, 200,000 52 + 43 / 95 + 83, 1,000,000 241 + 181 / 288 + 238; 100,000
-// identifiers 27 + 23 / 30 + 27; 3,000 velocities in double 15 + 13 / 17 + 17, 12,000
-// 27 + 24 / 27 + 24, in float 3,000 14 + 13 / 17 + 17, 200,000 171 + 171 / 181 + 180.
-// (Pageable copies into the caller's array: as fast, but not the first 16 MB of a
-// stream, which take 1.2 us more per 4 KB.)
+// Whether a field of one array (a scalar, or the velocity's records of four) is
+// copied as it lies and converted on the host: up to a size, and where no work
+// is queued before it.  One copy then starts sooner than a kernel, and up to the
+// size the conversion costs less than the kernel's slower way over the bus; behind
+// other kernels the copy engine waits longer than the next kernel does (a search of
+// 8,000 particles and two reads 208 us with copies, 203 with kernels).  Read and
+// write, copy / kernel, us: 3,000 doubles 11 + 11 / 16 + 16, 80,000 36 + 31 / 40 +
+// 37, 216,000 108 + 70 / 96 + 85; 8,000 floats 12 + 11 / 17 + 17, 200,000 52 + 43 / 95
+// + 83, 1,000,000 323 + 181 / 287 + 238; 100,000 identifiers 27 + 23 / 30 + 27,
+// 1,000,000 238 + 148 / 174 + 158; 3,000 velocities in double 15 + 13 / 17 + 17,
+// 12,000 27 + 24 / 27 + 24, in float 3,000 14 + 13 / 17 + 17, 80,000 81 + 74 / 106 +
+// 92.  (Pageable copies into the caller's array: as fast, but not the first 16 MB
+// of a stream, which take 1.2 us more per 4 KB.)
 template <int K, class E>
-constexpr size_t array_most()
+bool copies_as_it_lies(size_t bytes, bool write, bool queued)
 {
-    return sizeof(E) == 4 ? 4u << 20 : K == 1 ? 2u << 20 : 256u << 10;
+    constexpr bool floats = std::is_same<E, float>::value;
+    const size_t most = K > 1 ? (floats ? 2u << 20 : 256u << 10) : write ? 4u << 20 : floats ? 2u << 20 : 1u << 20;
+    return bytes <= most && (!queued || (floats && bytes > (64u << 10))); // (floats take half of the bus)
 }
-static_assert(array_most<1, float>() <= 2 * kStagingHalf, "one staging buffer");
 
 template <int K, int STRIDE, class E, class H>
 sphx_status transfer_array(sphx_body *b, const FieldComponents<E> &f, H *host, bool write)
@@ -381,7 +392,7 @@ sphx_status transfer_array(sphx_body *b, const FieldComponents<E> &f, H *host, b
     const size_t n = b->n, bytes = n * STRIDE * sizeof(E);
     const double offset = f.offset;
     StagingBuffer stage;
-    sphx_status st;
+    sphx_status st = SPHX_OK;
     if (bytes > kSmallTransfer && (st = stage.take()))
         return st;
     E *v = (E *)(bytes > kSmallTransfer ? stage.p : b->ctx->transfer_h);
@@ -398,7 +409,8 @@ sphx_status transfer_array(sphx_body *b, const FieldComponents<E> &f, H *host, b
     }
     else
         SPHX_HIP(hipMemcpyAsync(v, f.c[0], bytes, hipMemcpyDeviceToHost, s));
-    SPHX_HIP(hipStreamSynchronize(s));
+    if ((st = wait_for_stream(b->ctx)))
+        return st;
     for (size_t i = 0; !write && i < n; ++i)
         for (int k = 0; k < K; ++k)
             host[i * K + k] = to_host(v[i * STRIDE + k], offset);
@@ -412,14 +424,9 @@ sphx_status transfer_rows(sphx_body *b, const FieldComponents<E> &f, H *host, bo
     hipStream_t s = ctx->stream;
     constexpr size_t row = K * sizeof(H);
     const size_t n = b->n;
-    if (n * f.stride * sizeof(E) <= array_most<K, E>())
-    {
-        if constexpr (K == 1)
-            return transfer_array<1, 1>(b, f, host, write);
-        if constexpr (K == 2 || K == 3)
-            if (f.stride == 4u)
-                return transfer_array<K, 4>(b, f, host, write);
-    }
+    if constexpr (K <= 3)
+        if ((K == 1 || f.stride == 4u) && copies_as_it_lies<K, E>(n * f.stride * sizeof(E), write, ctx->work_queued))
+            return transfer_array<K, K == 1 ? 1 : 4>(b, f, host, write);
     auto launch = [&](unsigned char *stage, size_t first, size_t rows) -> sphx_status {
         const uint32_t values = (uint32_t)(rows * K);
         const dim3 g((values + 255u) / 256u), blk(256);
@@ -437,7 +444,8 @@ sphx_status transfer_rows(sphx_body *b, const FieldComponents<E> &f, H *host, bo
             std::memcpy(ctx->transfer_h, host, n * row);
         if ((st = launch(ctx->transfer_h, 0, n)))
             return st;
-        SPHX_HIP(hipStreamSynchronize(s));
+        if ((st = wait_for_stream(ctx)))
+            return st;
         if (!write)
             std::memcpy(host, ctx->transfer_h, n * row);
         return SPHX_OK;
@@ -487,8 +495,7 @@ sphx_status transfer_rows(sphx_body *b, const FieldComponents<E> &f, H *host, bo
             copy_host(host + (k - 1) * per * K, half[(k - 1) & 1], rows_of(k - 1) * row);
         }
     }
-    SPHX_HIP(hipStreamSynchronize(s)); // a failed kernel of a write is reported here
-    return SPHX_OK;
+    return wait_for_stream(ctx); // a failed kernel of a write is reported here
 }
 
 template <class T>
@@ -911,8 +918,7 @@ sphx_status sphx_context_synchronize(sphx_context *ctx)
 {
     if (!ctx)
         return arg_error("null context");
-    SPHX_HIP(hipStreamSynchronize(ctx->stream));
-    return SPHX_OK;
+    return wait_for_stream(ctx);
 }
 
 sphx_status sphx_profile_enable(sphx_context *ctx, int enable)

@@ -138,6 +138,9 @@ struct sphx_context
     // while its scalars are set, the acoustic kernels take dt and their run flag from the device-side loop
     sphx::StepBegin step;
     uint32_t last_substeps = 0; // sub-steps of the previous sphx_advection_step
+    // work was launched since the host last waited for the stream; only how a
+    // field is transferred depends on it
+    bool work_queued = false;
 };
 
 struct sphx_body

@@ -302,29 +302,39 @@ void observers()
     }
 }
 
-// a scalar or velocity field up to a size is copied as it lies, without a kernel
+// a scalar or velocity field up to a size is copied as it lies, without a kernel,
+// if no dynamics was launched since the last wait or it is of floats (over 64 KB)
 void array_copies()
 {
     for (int precision : {SPHX_FP64, SPHX_MIXED})
         for (uint32_t n : {100u, 10000u, 100000u, 500000u, 2000000u})
         {
             Scene s(0, 3, precision, n);
+            REQUIRE(API(sphx_context_synchronize)(s.ctx) == SPHX_OK);
             std::vector<double> v(3 * (size_t)n, 1.0);
             std::vector<uint32_t> id(n, 7u);
-            const bool fp64 = precision == SPHX_FP64;
-            for (bool write : {true, false})
-            {
-                auto copied = [&](int field, void *host) {
-                    g_launches.clear();
-                    REQUIRE((write ? API(sphx_body_write)(s.body, field, host, n)
-                                   : API(sphx_body_read)(s.body, field, host, n)) == SPHX_OK);
-                    return launches("k_field_") == 0;
-                };
-                REQUIRE(copied(SPHX_FIELD_PRESSURE, v.data()) == (n <= (fp64 ? 262144u : 1048576u)));
-                REQUIRE(copied(SPHX_FIELD_ORIGINAL_ID, id.data()) == (n <= 1048576u));
-                REQUIRE(copied(SPHX_FIELD_VELOCITY, v.data()) == (n <= (fp64 ? 8192u : 262144u)));
-                REQUIRE(!copied(SPHX_FIELD_POSITION, v.data()));
-            }
+            const bool floats = precision == SPHX_MIXED;
+            const size_t real = floats ? 4 : 8;
+            for (bool busy : {false, true})
+                for (bool write : {true, false})
+                {
+                    auto copied = [&](int field, void *host) {
+                        if (busy)
+                            REQUIRE(API(sphx_advection_step_setup)(s.body) == SPHX_OK);
+                        g_launches.clear();
+                        REQUIRE((write ? API(sphx_body_write)(s.body, field, host, n)
+                                       : API(sphx_body_read)(s.body, field, host, n)) == SPHX_OK);
+                        return launches("k_field_") == 0;
+                    };
+                    auto expected = [&](size_t bytes, size_t most, bool is_float) {
+                        return bytes * n <= most << 10 && (!busy || (is_float && bytes * n > 65536));
+                    };
+                    REQUIRE(copied(SPHX_FIELD_PRESSURE, v.data()) ==
+                            expected(real, write ? 4096 : floats ? 2048 : 1024, floats));
+                    REQUIRE(copied(SPHX_FIELD_ORIGINAL_ID, id.data()) == expected(4, write ? 4096 : 1024, false));
+                    REQUIRE(copied(SPHX_FIELD_VELOCITY, v.data()) == expected(4 * real, floats ? 2048 : 256, floats));
+                    REQUIRE(!copied(SPHX_FIELD_POSITION, v.data()));
+                }
         }
 }
 } // namespace
