@@ -5,8 +5,8 @@ the step captured in a HIP graph and replayed -- must end bit-identical to
 the same scene advanced alone with sphx_advection_step: positions,
 velocities, compression, forces, particle order, physical time and sub-step
 counts.  Covered: FP64 and FP32-mixed, graph and direct launches, the
-autotuner's shape changes (LDS staging switched per scene, tiled-build waves
-per workgroup), fewer captured sub-steps than a scene needs (the host
+autotuner's shape changes (LDS staging switched per 3D scene, chunks per
+workgroup of the tiled build), fewer captured sub-steps than a scene needs (the host
 finishes it), a particle sort inside the batch, a diverged scene, and the
 256-tank batched workload (1k-64k particles per tank) over 40 advection
 steps.  FP64 batched scenes are also checked against the oracle."""
@@ -276,4 +276,31 @@ def test_tuner_times_the_same_launches_once(hip):
     finally:
         batch.close()
         for sc in scenes:
+            sc.close()
+
+
+@pytest.mark.parametrize("use_graph,tile_waves", [(0, 2), (1, 4), (1, 1)])
+def test_batch_of_staged_and_unstaged_3d_scenes(hip, use_graph, tile_waves):
+    """3D FP32-mixed scenes of 3,400 to 26,400 particles, two on each side of
+    stage_min, and each number of chunks per workgroup of the list build."""
+    geoms = [cases.dambreak_3d(dp=dp) for dp in (0.03, 0.06, 0.04, 0.05)]
+    alone, batched = ([cases.DamBreak(hip, g, capi.MIXED) for g in geoms] for _ in range(2))
+    for sc in alone + batched:
+        sc.initialize()
+        sc.ctx.synchronize()
+    batch = ck.BatchAdvection(hip, [sc.advection for sc in batched],
+                              options=dict(use_graph=use_graph, autotune=0, tile_waves=tile_waves, stage_min=8000,
+                                           substep_margin=0))
+    try:
+        for _ in range(5):
+            for sc in alone:
+                sc.advection_step()
+            batch.exec()
+        assert batch.tuning()["shape"] == {"tile_waves": tile_waves, "stage_min": 8000}
+        for a, b in zip(alone, batched):
+            for k in FIELDS:
+                assert np.array_equal(a.fluid.read(k), b.fluid.read(k)), (a.fluid.n, k)
+    finally:
+        batch.close()
+        for sc in alone + batched:
             sc.close()
