@@ -410,8 +410,9 @@ sphx_status sphx_batch_tuning(const sphx_batch *batch, char *json, size_t capaci
  * (tiled list build of contact relations), "relation_scan" (per-lane scan build,
  * used when a list outgrows the LDS tile), "relation_stage" (LDS staging sets
  * of an inner relation), "cell_linked_list", "particle_sort",
- * "time_step_reduce", "state_update", "linear_correction" (correction matrix and
- * its neighbour sum), "surface_indication".  Reading synchronises the stream and
+ * "time_step_reduce" (the time-step calls; within an advection step their maxima
+ * are part of "state_update"), "state_update", "linear_correction" (correction
+ * matrix and its neighbour sum), "surface_indication".  Reading synchronises the stream and
  * returns the accumulated milliseconds and launch count since enabling.
  * enable: 0 off, 1 every stage, 2 only "acoustic_pass1" and "acoustic_pass2"
  * (each event pair delays the next launch by a few microseconds, so timing

@@ -863,7 +863,7 @@ static_assert(pass1_cap<3, P_MIXED>() <= kStageCap && pass2_cap<3, P_FP64>() <= 
 // The FP32-mixed pass walks six pairs per batch (94 VGPRs: five waves per SIMD,
 // no spills).  The FP64 passes are bound by their neighbour reads: 989k particles
 // in 3D took 425 us (pass 1) and 572 us (pass 2) a launch with 32-byte records
-// gathered through the vector cache at two waves per SIMD, 248 and 325 us with
+// gathered through the vector cache at two waves per SIMD, 241 and 311 us with
 // the block's records staged in LDS.
 //---------------------------------------------------------------------------
 
