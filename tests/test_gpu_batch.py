@@ -279,12 +279,16 @@ def test_tuner_times_the_same_launches_once(hip):
             sc.close()
 
 
-@pytest.mark.parametrize("use_graph,tile_waves", [(0, 2), (1, 4), (1, 1)])
-def test_batch_of_staged_and_unstaged_3d_scenes(hip, use_graph, tile_waves):
-    """3D FP32-mixed scenes of 3,400 to 26,400 particles, two on each side of
-    stage_min, and each number of chunks per workgroup of the list build."""
-    geoms = [cases.dambreak_3d(dp=dp) for dp in (0.03, 0.06, 0.04, 0.05)]
-    alone, batched = ([cases.DamBreak(hip, g, capi.MIXED) for g in geoms] for _ in range(2))
+@pytest.mark.parametrize("precision,use_graph,tile_waves", [(capi.MIXED, 0, 2), (capi.MIXED, 1, 4), (capi.MIXED, 1, 1),
+                                                            (capi.FP64, 1, 1)])
+def test_batch_of_3d_scenes_of_each_form(hip, precision, use_graph, tile_waves):
+    """FP32-mixed scenes of 3,400 to 26,400 particles, two on each side of
+    stage_min, with each number of chunks per workgroup of the list build; FP64
+    scenes of 3,400, 26,400 and 195,000 particles: eight, four and one (staged)
+    lanes per particle."""
+    sizes = (0.03, 0.06, 0.04, 0.05) if precision == capi.MIXED else (0.03, 0.06, 0.0155)
+    geoms = [cases.dambreak_3d(dp=dp) for dp in sizes]
+    alone, batched = ([cases.DamBreak(hip, g, precision) for g in geoms] for _ in range(2))
     for sc in alone + batched:
         sc.initialize()
         sc.ctx.synchronize()
